@@ -123,6 +123,13 @@ __global__ __launch_bounds__(1024) void k_group_assignments(const int* __restric
   if (tid == 0) { counters[0] = n_routed; counters[1] = n_shared; }
 }
 
+// groups of at most rgmax assignments of one expert, into p.groups / p.counters (rows * top_k <= FFMOE_DECODE_MAX_ASSIGN)
+int decode_group_assignments(const DecodeParams& p, int rgmax, hipStream_t st) {
+  hipLaunchKernelGGL(k_group_assignments, dim3(1), dim3(1024), size_t(p.rows) * p.top_k * sizeof(int), st, p.ids, p.active, p.valid, p.generation,
+                     p.assignment_gen, p.groups, p.counters, p.rows, p.top_k, p.experts, p.has_shared, rgmax);
+  return ff_launch_status();
+}
+
 }  // namespace ffmoe
 
 using namespace ffmoe;

@@ -1,12 +1,17 @@
 // Entry points of the E8M0 block-32 expert path (W4A8 routed experts, W8A8 shared expert, exact arithmetic); the
 // kernels are in e8m0_kernel.cuh.
 #include "e8m0_kernel.cuh"
+#include <algorithm>
+
+namespace ffmoe {
+int decode_group_assignments(const DecodeParams& p, int rgmax, hipStream_t st);
+}
 
 using namespace ffmoe;
 
 namespace {
 struct E8m0Layout {
-  uint64_t xq, xs, h, hq, hs, live, total;
+  uint64_t xq, xs, h, hq, hs, live, groups, counters, total;
 };
 E8m0Layout e8m0_layout(int rows, int top_k, int hidden, int inter, int shared_inter) {
   const uint64_t R = rows, A = uint64_t(rows) * top_k, S = A + R;
@@ -20,6 +25,8 @@ E8m0Layout e8m0_layout(int rows, int top_k, int hidden, int inter, int shared_in
   l.hq = at; at = up(at + S * imax);
   l.hs = at; at = up(at + S * (imax / 32));
   l.live = at; at = up(at + S * 4);
+  l.groups = at; at = up(at + (S + 2) * sizeof(GroupDesc));
+  l.counters = at; at = up(at + 8);
   l.total = at;
   return l;
 }
@@ -88,6 +95,37 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_decode_contribute_e8
   uint32_t* live = (uint32_t*)(sc + l.live);
   hipStream_t st = (hipStream_t)stream;
   const int S = R * K + R;
+  // Exact arithmetic on the matrix cores wherever the contractions are whole instructions (multiples of 128 columns) and a
+  // token's exponent planes fit LDS. Several rows: the assignments of an expert share a pass over its weights in pairs.
+  auto tiles_lds = [&](int tokens) { return std::max(e8m0_tiles_lds(0, H, tokens), e8m0_tiles_lds(1, imax, tokens)); };
+  constexpr size_t TWO_BLOCKS = 80 * 1024, ONE_BLOCK = 160 * 1024;  // LDS per CU: 160 KB
+  if (exact && H % 128 == 0 && I % 128 == 0 && SI % 128 == 0 && tiles_lds(1) <= ONE_BLOCK) {
+    const bool pairs = R > 1 && K > 0 && (long long)R * K <= FFMOE_DECODE_MAX_ASSIGN && tiles_lds(FFMOE_E8M0_TOK) <= TWO_BLOCKS;
+    const int tokens = pairs ? FFMOE_E8M0_TOK : 1;
+    long long groups = S;
+    if (pairs) {
+      p.groups = (GroupDesc*)(sc + l.groups);
+      p.counters = (int*)(sc + l.counters);
+      FF_TRY(decode_group_assignments(p, tokens, st));
+      const long long routed = (long long)R * K, most = E + routed / tokens;  // an expert leaves at most one group unfilled
+      groups = (routed < most ? routed : most) + (shared ? (R + tokens - 1) / tokens : 0);
+    } else if (!shared) {
+      groups = (long long)R * K;
+    }
+    const long long gs = shared ? (R + tokens - 1) / tokens : 0, gr = groups - gs;
+    const long long b0 = gs * (SI / 16) + gr * (I / 32), b1 = gs * (H / 32) + gr * ((H + 127) / 128);
+    FF_REQUIRE(b0 < (1ll << 31) && b1 < (1ll << 31), FFMOE_ERR_SHAPE, "rows=%d top_k=%d exceed the launch grid", R, K);
+    const size_t l0 = e8m0_tiles_lds(0, H, tokens), l1 = e8m0_tiles_lds(1, imax, tokens);
+    if (R > 1) {
+      hipLaunchKernelGGL(k_act_quant_e8m0, dim3((H / 32 + 63) / 64, R), dim3(256), 0, st, p.x, H, sc + l.xq, H, sc + l.xs, H / 32, H, (const uint32_t*)nullptr);
+      hipLaunchKernelGGL((k_e8m0_tiles<0, true>), dim3((unsigned)b0), dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
+    } else {
+      hipLaunchKernelGGL((k_e8m0_tiles<0, false>), dim3((unsigned)b0), dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
+    }
+    FF_TRY(ff_launch_status());
+    hipLaunchKernelGGL((k_e8m0_tiles<1, false>), dim3((unsigned)b1), dim3(FFMOE_E8M0_NT), l1, st, q, tokens);
+    return ff_launch_status();
+  }
   hipLaunchKernelGGL(k_act_quant_e8m0, dim3((H / 32 + 63) / 64, R), dim3(256), 0, st, p.x, H, sc + l.xq, H, sc + l.xs, H / 32, H, (const uint32_t*)nullptr);
   hipLaunchKernelGGL(k_e8m0_live, dim3((S + 255) / 256), dim3(256), 0, st, p, live);
   if (exact) hipLaunchKernelGGL((k_e8m0_stage<0>), dim3((imax + 7) / 8, R, K + 1), dim3(256), size_t(H / 32) * 33 * 4, st, q);

@@ -305,6 +305,532 @@ __global__ __launch_bounds__(256) void k_e8m0_stage(const E8m0Params q) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// The same contract on the matrix cores, still exact (contractions that are multiples of 128; k_e8m0_stage keeps the others).
+//
+// v_mfma_scale_f32_16x16x128_f8f6f4 takes the E2M1 codes and their E8M0 scales as they are. Left to itself it is not exact:
+// it keeps the bits of 8 consecutive products down to 2^-13 of the largest one, and FP32 across them. Both limits go away
+// when an instruction's column holds ONE 32-element group of the token (the other columns' elements are zeros) and only
+// the elements of one half of E4M3's exponents (codes with bit 6 clear: 7 binades, bit 6 set: 8 binades): every product is
+// then an integer below 2^14.5 times the column's unit and a group sum below 2^20 units, so the FP32 result is the exact
+// group sum (times the group's two scales, an exponent). Four groups x two halves are eight of the sixteen columns: two
+// tokens per instruction. The FP32 sums are added in FP64 in any order, which equals the contract's ascending chain as
+// long as nothing rounds: certain when the groups' exponents of a row span few enough binades (checked per row and
+// token from the scale codes of the groups that are not all zero); a row that fails is redone in the contract's order.
+// The shared expert's E4M3 x E4M3 products need 8 + 11 bits: v_mfma_f32_16x16x32_bf16 on codes widened to BF16, the token
+// in three exponent classes (at most 6 binades) by columns and the weights in two (bit 6) by instructions, group sums below
+// 2^24 units.
+//
+// Bound by HBM and, with several tokens, by the vector ALUs: an instruction's 2048 weights cost them about 45 instructions
+// (mostly the FP64 conversions and additions of its four result registers), where packed-byte dot products need 3.9 a
+// weight. One token, 8 of 256 experts + shared at hidden 7168 / intermediate 2048 (231 MB): gate/up 111 -> 36 us, down
+// 38 -> 20.5 us, four launches for quantizers and flags fewer; the call by rows (64 experts), per (row, choice) before and
+// in pairs now: 1 row 158 -> 55 us, 2 rows 287 -> 103, 4 rows 500 -> 173, 12 rows 1283 -> 348. Weights requested in operand order
+// instead of row by row cost 8 us of the one-token call (the vector L1 then looks up 16 bytes at a time), blocks of four
+// waves, which quantize the token twice as often, 9 us. With several rows the tokens are quantized by a launch of their own:
+// in the blocks it would be a quarter of their instructions.
+typedef float e8_f32x4 __attribute__((ext_vector_type(4)));
+typedef int e8_i32x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 e8_bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int FFMOE_E8M0_TOK = 2;  // tokens of one expert per pass over its weights
+constexpr int FFMOE_E8M0_NT = 512;
+// bytes between the exponent planes of a token: 128 past a multiple of 256, so that two planes fall on different banks
+__host__ __device__ __forceinline__ int e8m0_plane(int k) { return k + (k % 256 == 0 ? 128 : 0); }
+struct E8m0Red {  // cross-lane and cross-wave hand-over of a tile, per wave
+  double total[2][FFMOE_E8M0_TOK][16], mass[2][FFMOE_E8M0_TOK][16];
+  int smin[2][16], smax[2][16];  // routed: scale codes of the row's groups that are not all zero; shared: smin[m][token] = exponent
+};
+static_assert(sizeof(E8m0Red) <= 2048, "a wave's hand-over lies in its weight buffer");
+// LDS of a block: per wave a weight buffer (2 KB per matrix, the hand-over behind it), the tokens' planes, their scales, the
+// tiles' weight scales
+__host__ __device__ __forceinline__ int e8m0_wbuf(int stage) { return 8 * (stage == 0 ? 4096 : 2048); }
+__host__ __device__ __forceinline__ size_t e8m0_tiles_lds(int stage, int k, int tokens) {
+  const size_t routed = size_t(tokens) * 2 * e8m0_plane(k) + size_t(stage == 0 ? 64 : 128) * (k / 32);
+  const size_t shared = size_t(tokens) * 3 * e8m0_plane(k) + size_t(4) * (k / 32);
+  return e8m0_wbuf(stage) + size_t(tokens) * (k / 32) + (routed > shared ? routed : shared) + 16;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_add_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const int lo = dpp_or<CTRL, 0xf>(0, int(uint32_t(b))), hi = dpp_or<CTRL, 0xf>(0, int(uint32_t(b >> 32)));
+  return v + __builtin_bit_cast(double, (uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
+}
+// sum over the eight lanes of a half row, in every one of them
+__device__ __forceinline__ double sum8_f64(double v) {
+  v = dpp_add_f64<DPP_QUAD_SWAP1>(v);
+  v = dpp_add_f64<DPP_QUAD_SWAP2>(v);
+  return dpp_add_f64<DPP_ROW_HALF_MIRROR>(v);
+}
+
+// Eight values of a 32-element group (four neighbouring lanes of a quad hold the group) to E4M3 codes and the group's scale
+// code: the quantizer of k_act_quant_e8m0 (the scale is a power of two, so its division is an exponent step)
+__device__ __forceinline__ int e8m0_scale_exponent(float amax) {
+  amax = fmaxf(amax, 1e-4f);
+  const uint32_t qb = __float_as_uint(__fmul_rn(amax, 1.0f / 448.0f));
+  const int exponent = int((qb >> 23) & 0xffu) - 127 + ((qb & 0x7fffffu) != 0u ? 1 : 0);
+  return exponent < -127 ? -127 : (exponent > 127 ? 127 : exponent);
+}
+__device__ __forceinline__ float e8m0_scaled(float v, int exponent) { return fminf(448.0f, fmaxf(-448.0f, __builtin_amdgcn_ldexpf(v, -exponent))); }
+
+// The tokens of a group into LDS: E4M3 codes by exponent class (THREE: exponents 0..5, 6..10, 11..15; else bit 6 of the code)
+// and one E8M0 scale per 32. CODES: the source is quantized already, else BF16. range[2 t], [2 t + 1]: smallest and largest
+// scale code of token t over its groups that are not all zero. K is a multiple of 128: quads of lanes stay whole.
+template <bool THREE, bool CODES>
+__device__ __forceinline__ void e8m0_stage_tokens(const uint64_t (&src)[FFMOE_E8M0_TOK], const uint64_t (&ssrc)[FFMOE_E8M0_TOK], int n, int K, uint8_t* planes,
+                                                  int ps, uint8_t* scales, int* range, int tid) {
+  constexpr int NP = THREE ? 3 : 2;
+  const int per = K >> 3;
+#pragma unroll
+  for (int t = 0; t < FFMOE_E8M0_TOK; ++t) {
+    if (t >= n) break;
+    int lo = 255, hi = 0;
+    uint8_t* pl = planes + size_t(t) * NP * ps;
+    for (int v = tid; v < per; v += FFMOE_E8M0_NT) {  // eight elements a lane, a quad of lanes a group
+      uint32_t o[2];
+      int code;
+      if (CODES) {
+        const u32x2 d = load_global<u32x2>(reinterpret_cast<const uint8_t*>(src[t]) + size_t(v) * 8);
+        o[0] = d.x; o[1] = d.y;
+        code = load_global<uint8_t>(reinterpret_cast<const uint8_t*>(ssrc[t]) + (v >> 2));
+      } else {
+        const u32x4 w = load16(reinterpret_cast<const uint8_t*>(src[t]) + size_t(v) * 16);
+        float f[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { f[2 * q] = bf16lo(w[q]); f[2 * q + 1] = bf16hi(w[q]); }
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(f[i]));
+        amax = fmaxf(amax, dpp_or<DPP_QUAD_SWAP1, 0xf>(0.0f, amax));
+        amax = fmaxf(amax, dpp_or<DPP_QUAD_SWAP2, 0xf>(0.0f, amax));
+        const int exponent = e8m0_scale_exponent(amax);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = e8m0_scaled(f[i], exponent);
+        o[0] = e4m3x4_encode_finite(f[0], f[1], f[2], f[3]);
+        o[1] = e4m3x4_encode_finite(f[4], f[5], f[6], f[7]);
+        code = exponent + 127;
+      }
+      uint32_t cls[3][2];
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        if (THREE) {  // the code without its sign against 6 << 3 and 11 << 3, byte by byte
+          const uint32_t m = o[d] & 0x7f7f7f7fu;
+          const uint32_t b6 = ((m + 0x50505050u) >> 7) & 0x01010101u, b11 = ((m + 0x28282828u) >> 7) & 0x01010101u;
+          const uint32_t m6 = (b6 << 8) - b6, m11 = (b11 << 8) - b11;
+          cls[0][d] = o[d] & ~m6; cls[1][d] = o[d] & m6 & ~m11; cls[2][d] = o[d] & m11;
+        } else {
+          const uint32_t b = (o[d] >> 6) & 0x01010101u, m = (b << 8) - b;
+          cls[0][d] = o[d] & ~m; cls[1][d] = o[d] & m; cls[2][d] = 0u;
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < NP; ++c) *reinterpret_cast<u32x2*>(pl + size_t(c) * ps + size_t(v) * 8) = u32x2{cls[c][0], cls[c][1]};
+      uint32_t any = (o[0] | o[1]) & 0x7f7f7f7fu;
+      any |= uint32_t(dpp_or<DPP_QUAD_SWAP1, 0xf>(0, int(any)));
+      any |= uint32_t(dpp_or<DPP_QUAD_SWAP2, 0xf>(0, int(any)));
+      if ((v & 3) == 0) scales[size_t(t) * (K >> 5) + (v >> 2)] = uint8_t(code);
+      if (any) { lo = code < lo ? code : lo; hi = code > hi ? code : hi; }
+    }
+    // one LDS atomic per wave and bound
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      int u = __shfl_xor(lo, off, 64); lo = u < lo ? u : lo;
+      u = __shfl_xor(hi, off, 64); hi = u > hi ? u : hi;
+    }
+    if ((tid & 63) == 0) { atomicMin(range + 2 * t, lo); atomicMax(range + 2 * t + 1, hi); }
+  }
+}
+
+// `bytes` (a multiple of 4) of weight scales into LDS by `nt` threads
+__device__ __forceinline__ void e8m0_copy_scales(uint8_t* dst, uint64_t src, int bytes, int tid, int nt) {
+  if (((src | uint64_t(bytes)) & 15) == 0) {
+    for (int v = tid; v < (bytes >> 4); v += nt) reinterpret_cast<u32x4*>(dst)[v] = load16(reinterpret_cast<const uint8_t*>(src) + size_t(v) * 16);
+  } else {
+    for (int v = tid; v < bytes; v += nt) dst[v] = load_global<uint8_t>(reinterpret_cast<const uint8_t*>(src) + v);
+  }
+}
+
+// The contract's own order for one row: ascending groups, one FP64 fma each. planes: the token's exponent planes (a code
+// sits in one of them, the others hold zero).
+__device__ __forceinline__ double e8m0_row_ordered(bool packed, const uint8_t* wrow, const uint8_t* srow, const uint8_t* planes, int ps, int nplanes,
+                                                   const uint8_t* xscales, int G) {
+  double t = 0.0;
+  for (int g = 0; g < G; ++g) {
+    long long sum = 0;
+    for (int i = 0; i < 32; ++i) {
+      const int k = g * 32 + i;
+      uint32_t code = 0;
+      for (int c = 0; c < nplanes; ++c) code |= planes[size_t(c) * ps + k];
+      const int bv = packed ? e2m1_int((wrow[k >> 1] >> (4 * (k & 1))) & 15u) : e4m3_int(wrow[k]);
+      sum += (long long)e4m3_int(code) * bv;
+    }
+    t = fma(double(sum), pow2_f64(int(xscales[g]) + int(srow[g]) - (packed ? 264 : 272)), t);
+  }
+  return t;
+}
+
+// grid: (group, tile) pairs, blocks of eight waves.
+// STAGE 0, routed expert: 32 output columns per block, so that a block holds whole quantization groups of its activations and
+//   stores them quantized: waves 0-3 the first 16 columns, 4-7 the others, a quarter of the contraction each, gate and up
+//   rows side by side (one read of the token serves both). Shared expert: 16 columns, the contraction over all eight waves,
+//   BF16 activations.
+// STAGE 1, routed: a tile of 16 output columns per wave over the whole (shorter) contraction. Shared: two tiles, four waves each.
+// CODES: the tokens come quantized (xq / xs); else every block quantizes the BF16 rows it needs.
+template <int STAGE, bool CODES>
+__global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Params q, int lds_tokens) {
+  const DecodeParams& p = q.d;
+  constexpr int NMAT = STAGE == 0 ? 2 : 1;
+  constexpr int T = FFMOE_E8M0_TOK;
+  constexpr int WB = STAGE == 0 ? 4096 : 2048;  // weight buffer per wave
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int A = p.rows * p.top_k;
+  // blocks of the shared expert first (longer tiles), then the routed groups'; output columns per block: see above
+  const int cols_s = STAGE == 0 ? 16 : 32, cols_r = STAGE == 0 ? 32 : 128;
+  const int tiles_s = (STAGE == 0 ? p.shared_inter : p.hidden) / cols_s, tiles_r = ((STAGE == 0 ? p.inter : p.hidden) + cols_r - 1) / cols_r;
+  const int n_routed = p.groups ? load_uniform<int>(p.counters) : A;
+  const int n_shared = p.groups ? load_uniform<int>(p.counters + 1) : (p.has_shared ? p.rows : 0);
+  int group, tile;
+  {
+    const uint32_t b = blockIdx.x, bs = uint32_t(n_shared) * uint32_t(tiles_s);
+    if (b < bs) {
+      group = int(b / uint32_t(tiles_s));
+      tile = int(b) - group * tiles_s;
+      group += n_routed;
+    } else {
+      group = int((b - bs) / uint32_t(tiles_r));
+      if (group >= n_routed) return;
+      tile = int(b - bs) - group * tiles_r;
+    }
+  }
+  int expert, gn, grow[T], gslot[T];
+  load_group<T>(p, group, expert, gn, grow, gslot);
+  if (gn == 0) return;
+  const bool is_shared = expert < 0;
+  const int K = STAGE == 0 ? p.hidden : (is_shared ? p.shared_inter : p.inter);
+  const int out = STAGE == 0 ? (is_shared ? p.shared_inter : p.inter) : p.hidden;
+  // first output column of this wave's tile; columns per block
+  const int cols = is_shared ? cols_s : cols_r;
+  const int first = tile * cols;
+  const int sub = STAGE == 0 ? (is_shared ? 0 : wave >> 2) : (is_shared ? wave >> 2 : wave);
+  const bool tile_ok = first + sub * 16 < out;
+  const int j0 = tile_ok ? first + sub * 16 : out - 16;  // a wave past the end repeats the last tile and stores nothing
+  const int G = K >> 5, KB = K >> 7, ps = e8m0_plane(K);
+  uint8_t* wbuf = lds + size_t(wave) * WB;
+  E8m0Red& red = *reinterpret_cast<E8m0Red*>(wbuf);
+  uint8_t* xsc = lds + 8 * WB;                    // [token][G]
+  uint8_t* wsc = xsc + ((size_t(lds_tokens) * G + 15) & ~size_t(15));
+  uint8_t* planes = wsc + size_t(is_shared ? 4 : (STAGE == 0 ? 64 : 128)) * G;
+  __shared__ int range[2 * T];
+  if (tid < 2 * T) range[tid] = (tid & 1) ? 0 : 255;
+
+  uint64_t sl[2 * NMAT];
+#pragma unroll
+  for (int m = 0; m < NMAT; ++m) {
+    const int base = STAGE == 0 ? 2 * m : 4;
+    if (is_shared) {
+      sl[2 * m] = p.shared_slot[base];
+      sl[2 * m + 1] = p.shared_slot[base + 1];
+    } else {
+      sl[2 * m] = load_uniform<uint64_t>(p.slots + size_t(expert) * 6 + base);
+      sl[2 * m + 1] = load_uniform<uint64_t>(p.slots + size_t(expert) * 6 + base + 1);
+    }
+  }
+  uint64_t src[T], ssrc[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int r = grow[t < gn ? t : 0], s = gslot[t < gn ? t : 0];
+    if (STAGE == 0) src[t] = CODES ? uint64_t(q.xq + size_t(r) * p.hidden) : uint64_t(p.x + size_t(r) * p.hidden);
+    else src[t] = is_shared ? uint64_t(p.h + size_t(s) * p.h_stride) : uint64_t(q.hq + size_t(s) * p.h_stride);
+    ssrc[t] = STAGE == 0 ? uint64_t(q.xs + size_t(r) * (p.hidden >> 5)) : uint64_t(q.hs + size_t(s) * (p.h_stride >> 5));
+  }
+  const int i = lane & 15, c = lane >> 4;
+  const int tok = i >> 3 < gn ? i >> 3 : 0;
+
+  if (!is_shared) {
+    // Weights travel row-contiguously, eight lanes per 128-byte line (two K blocks), and are turned into operand order
+    // through the wave's own buffer (LDS operations of a wave execute in order): requested in operand order the vector L1
+    // looks up 16 bytes at a time. D pairs of K blocks are on their way.
+    constexpr int D = 2;
+    const int NP = (KB + 1) >> 1;
+    const int wq = wave & 3;
+    const int k0 = STAGE == 0 ? NP * wq / 4 : 0, k1 = STAGE == 0 ? NP * (wq + 1) / 4 : NP;
+    const uint32_t rowb = uint32_t(K) >> 1;
+    const uint32_t lrow = uint32_t(lane >> 3) * rowb, lcol = uint32_t(lane & 7) * 16u;
+    uint64_t wb[NMAT];
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) wb[m] = sl[2 * m] + uint64_t(j0) * rowb;
+    u32x4 w[D][NMAT][2];
+    auto request = [&](int s, int kp) {  // past the end: one line with every lane, nothing reads it
+      const uint32_t col = uint32_t(kp) * 128u + lcol;
+      const uint32_t off = kp < k1 ? lrow + (col + 16u <= rowb ? col : rowb - 16u) : 0u;  // an odd last K block has half a line
+#pragma unroll
+      for (int m = 0; m < NMAT; ++m)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) w[s][m][h] = load16(reinterpret_cast<const uint8_t*>(wb[m]) + off + (kp < k1 ? uint32_t(h) * 8u * rowb : 0u));
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) request(s, k0 + s);
+    __syncthreads();  // range[] is initialised
+    e8m0_stage_tokens<false, STAGE == 1 || CODES>(src, ssrc, gn, K, planes, ps, xsc, range, tid);
+    // weight scales: the 16 rows of a tile are one run of memory per matrix
+    if (STAGE == 0) {
+      const int cnt = min(32, out - first);
+#pragma unroll
+      for (int m = 0; m < NMAT; ++m) e8m0_copy_scales(wsc + size_t(m) * 32 * G, sl[2 * m + 1] + uint64_t(first) * G, cnt * G, tid, FFMOE_E8M0_NT);
+    } else {
+      e8m0_copy_scales(wsc, sl[1] + uint64_t(first) * G, min(128, out - first) * G, tid, FFMOE_E8M0_NT);
+    }
+    __syncthreads();
+    const int piece = (i >> 2) & 1, g = i & 3;
+    const bool mine = (g & 1) == (c >> 1);
+    const uint32_t mlo = mine && g < 2 ? ~0u : 0u, mhi = mine && g >= 2 ? ~0u : 0u;
+    const uint8_t* bp = planes + size_t(tok * 2 + piece) * ps + (g >> 1) * 64 + c * 16;
+    const uint8_t* bs = xsc + size_t(tok) * G + c;
+    const uint8_t* ap = wsc + size_t(j0 - first + i) * G + c;
+    const int wr = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+    const int rd0 = i * 128 + ((c ^ (i & 7)) << 4), rd1 = i * 128 + (((4 + c) ^ (i & 7)) << 4);
+    double acc[NMAT][4];
+    int smin[NMAT], smax[NMAT];
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      smin[m] = 255; smax[m] = 0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[m][r] = 0.0;
+    }
+    for (int kpo = k0; kpo < k1; kpo += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        const int kp = kpo + s;
+        u32x4 a[NMAT][2];
+#pragma unroll
+        for (int m = 0; m < NMAT; ++m) {
+          *reinterpret_cast<u32x4*>(wbuf + m * 2048 + wr) = w[s][m][0];
+          *reinterpret_cast<u32x4*>(wbuf + m * 2048 + 1024 + wr) = w[s][m][1];
+        }
+        request(s, kp + D);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int m = 0; m < NMAT; ++m) {
+          a[m][0] = *reinterpret_cast<const u32x4*>(wbuf + m * 2048 + rd0);
+          a[m][1] = *reinterpret_cast<const u32x4*>(wbuf + m * 2048 + rd1);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int kb = 2 * kp + h;
+          const bool ok = kp < k1 && kb < KB;
+          const int kc = ok ? kb : 0;
+          const uint32_t in = ok ? ~0u : 0u;  // blocks past the end meet a zero token
+          const u32x4 b = *reinterpret_cast<const u32x4*>(bp + size_t(kc) * 128);
+          const int sx = bs[4 * kc];
+          const e8_i32x8 tk = {int(b[0] & mlo & in), int(b[1] & mlo & in), int(b[2] & mlo & in), int(b[3] & mlo & in),
+                               int(b[0] & mhi & in), int(b[1] & mhi & in), int(b[2] & mhi & in), int(b[3] & mhi & in)};
+#pragma unroll
+          for (int m = 0; m < NMAT; ++m) {
+            const int sw = ap[size_t(m) * 32 * G + 4 * kc];
+            const u32x4 v = a[m][h];
+            const bool nz = ((v[0] | v[1] | v[2] | v[3]) & 0x77777777u & in) != 0u;
+            smin[m] = nz && sw < smin[m] ? sw : smin[m];
+            smax[m] = nz && sw > smax[m] ? sw : smax[m];
+            const e8_i32x8 wf = {int(v[0]), int(v[1]), int(v[2]), int(v[3]), 0, 0, 0, 0};
+            const e8_f32x4 r = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, tk, e8_f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 4, 0, 0, sw, 0, sx);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[m][e] += double(r[e]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      int o = __shfl_xor(smin[m], 16, 64); smin[m] = o < smin[m] ? o : smin[m];
+      o = __shfl_xor(smin[m], 32, 64); smin[m] = o < smin[m] ? o : smin[m];
+      o = __shfl_xor(smax[m], 16, 64); smax[m] = o > smax[m] ? o : smax[m];
+      o = __shfl_xor(smax[m], 32, 64); smax[m] = o > smax[m] ? o : smax[m];
+      if (lane < 16) { red.smin[m][lane] = smin[m]; red.smax[m][lane] = smax[m]; }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double t = sum8_f64(acc[m][r]);
+        if ((lane & 7) == r) red.total[m][(lane >> 3) & 1][4 * c + r] = t;
+      }
+    }
+  } else {
+    // E4M3 x E4M3: a lane's 16 bytes lie inside one group (lanes c = 0, 1 the first of a pair of groups, 2, 3 the second); a
+    // column takes one group and one exponent class of the token, two instructions (low and high eight bytes) per weight class
+    constexpr int D = 4;
+    const int QB = K >> 6;
+    const int wq = STAGE == 0 ? wave : wave & 3, nq = STAGE == 0 ? 8 : 4;
+    const int k0 = QB * wq / nq, k1 = QB * (wq + 1) / nq;
+    const uint32_t loff = uint32_t(i) * uint32_t(K) + uint32_t(c) * 16u;
+    uint64_t wb[NMAT], sb[NMAT];
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      wb[m] = sl[2 * m] + uint64_t(j0) * uint64_t(K);
+      sb[m] = sl[2 * m + 1] + uint64_t(first >> 5) * uint64_t(G);  // the block's columns lie in one row of 32 x 32 blocks
+    }
+    u32x4 w[D][NMAT];
+    auto request = [&](int s, int kb) {
+      const uint32_t off = kb < k1 ? loff + uint32_t(kb) * 64u : 0u;
+#pragma unroll
+      for (int m = 0; m < NMAT; ++m) w[s][m] = load16(reinterpret_cast<const uint8_t*>(wb[m]) + off);
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) request(s, k0 + s);
+    __syncthreads();
+    e8m0_stage_tokens<true, STAGE == 0 && CODES>(src, ssrc, gn, K, planes, ps, xsc, range, tid);
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) e8m0_copy_scales(wsc + m * G, sb[m], G, tid, FFMOE_E8M0_NT);
+    __syncthreads();
+    const int piece = (i >> 1) & 3, gsel = i & 1;
+    const uint32_t mask = piece < 3 && gsel == (c >> 1) ? ~0u : 0u;
+    const uint8_t* bp = planes + size_t(tok * 3 + (piece < 3 ? piece : 0)) * ps + c * 16;
+    const uint8_t* bs = xsc + size_t(tok) * G + gsel;
+    const uint8_t* ap = wsc + gsel;
+    double acc[NMAT][4], mass[NMAT][4];
+    int emin[NMAT];
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      emin[m] = 4096;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) { acc[m][r] = 0.0; mass[m][r] = 0.0; }
+    }
+    auto widen = [](uint32_t d0, uint32_t d1) {  // eight codes to BF16
+      const bf16x2 a0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(int(d0), 1.0f, false), a1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(int(d0), 1.0f, true);
+      const bf16x2 a2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(int(d1), 1.0f, false), a3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(int(d1), 1.0f, true);
+      return e8_bf16x8{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+    };
+    for (int kbo = k0; kbo < k1; kbo += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        const int kb = kbo + s;
+        const int kc = kb < k1 ? kb : k1 - 1;
+        const uint32_t in = kb < k1 ? mask : 0u;
+        const u32x4 b = *reinterpret_cast<const u32x4*>(bp + size_t(kc) * 64);
+        const e8_bf16x8 blo = widen(b[0] & in, b[1] & in), bhi = widen(b[2] & in, b[3] & in);
+        const int sx = bs[2 * kc];
+#pragma unroll
+        for (int m = 0; m < NMAT; ++m) {
+          const int e = sx + int(ap[size_t(m) * G + 2 * kc]) - 254;
+          const double scale = pow2_f64(e);
+          uint32_t wh[4], wl[4];
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const uint32_t bit = (w[s][m][d] >> 6) & 0x01010101u, hm = (bit << 8) - bit;
+            wh[d] = w[s][m][d] & hm;
+            wl[d] = w[s][m][d] & ~hm;
+          }
+          const e8_f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+          e8_f32x4 rl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen(wl[0], wl[1]), blo, z, 0, 0, 0);
+          e8_f32x4 rh = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen(wh[0], wh[1]), blo, z, 0, 0, 0);
+          rl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen(wl[2], wl[3]), bhi, rl, 0, 0, 0);
+          rh = __builtin_amdgcn_mfma_f32_16x16x32_bf16(widen(wh[2], wh[3]), bhi, rh, 0, 0, 0);
+          bool nz = false;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double sum = double(rl[r]) + double(rh[r]);
+            acc[m][r] = fma(sum, scale, acc[m][r]);
+            mass[m][r] = fma(fabs(sum), scale, mass[m][r]);
+            nz = nz || sum != 0.0;
+          }
+          emin[m] = nz && e < emin[m] ? e : emin[m];
+        }
+        request(s, kb + D);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < NMAT; ++m) {
+      // smallest exponent of a token's columns, over all rows of the tile
+      for (int off = 1; off < 64; off <<= 1) {
+        if (off == 8) continue;
+        const int o = __shfl_xor(emin[m], off, 64);
+        emin[m] = o < emin[m] ? o : emin[m];
+      }
+      if ((lane & ~8) == 0) red.smin[m][lane >> 3] = emin[m];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double t = sum8_f64(acc[m][r]), ms = sum8_f64(mass[m][r]);
+        if ((lane & 7) == r) {
+          red.total[m][(lane >> 3) & 1][4 * c + r] = t;
+          red.mass[m][(lane >> 3) & 1][4 * c + r] = ms;
+        }
+      }
+    }
+  }
+  // one lane per (output column, token): the waves' parts, the check, the epilogue
+  const bool per_wave = STAGE == 1 && !is_shared;
+  if (per_wave) wave_lds_fence();
+  else __syncthreads();
+  const int width = per_wave ? 16 : cols;  // 16 or 32: the columns of a token are one run of lanes
+  const int item = per_wave ? lane : tid;
+  const int jc = item & (width - 1), t = item / width;
+  const int j = (per_wave ? j0 : first) + jc;
+  if (t >= gn || j >= out || (per_wave && !tile_ok)) return;
+  const int row = jc & 15;
+  const int w_lo = per_wave ? wave : (STAGE == 0 && is_shared) ? 0 : 4 * (jc >> 4);
+  const int w_hi = per_wave ? wave + 1 : (STAGE == 0 && is_shared) ? 8 : w_lo + 4;
+  double total[NMAT];
+#pragma unroll
+  for (int m = 0; m < NMAT; ++m) {
+    double v = 0.0, ms = 0.0;
+    int lo = is_shared ? 4096 : 255, hi = 0;
+    for (int u = w_lo; u < w_hi; ++u) {
+      const E8m0Red& ru = *reinterpret_cast<const E8m0Red*>(lds + size_t(u) * WB);
+      v += ru.total[m][t][row];
+      if (is_shared) {
+        ms += ru.mass[m][t][row];
+        lo = ru.smin[m][t] < lo ? ru.smin[m][t] : lo;
+      } else {
+        lo = ru.smin[m][row] < lo ? ru.smin[m][row] : lo;
+        hi = ru.smax[m][row] > hi ? ru.smax[m][row] : hi;
+      }
+    }
+    bool exact;
+    if (is_shared) {
+      exact = lo == 4096 || ms < pow2_f64(53 + lo - 18);  // units of 2^-18 below the smallest group's exponent
+    } else {
+      // |group sum| < 2^27 units, G of them; the FP32 results stay away from both ends of the exponent range
+      const int xlo = range[2 * t], xhi = range[2 * t + 1];
+      const int span = (xhi + hi) - (xlo + lo);
+      exact = lo > hi || xlo > xhi || (span + 27 + (32 - __builtin_clz(G)) <= 53 && xlo + lo >= 140 && xhi + hi <= 370 && hi <= 254);
+    }
+    if (!exact) {
+      const uint8_t* wrow = reinterpret_cast<const uint8_t*>(sl[2 * m]) + size_t(j) * (is_shared ? K : K >> 1);
+      const uint8_t* srow = reinterpret_cast<const uint8_t*>(sl[2 * m + 1]) + size_t(is_shared ? j >> 5 : j) * G;
+      const int np = is_shared ? 3 : 2;
+      v = e8m0_row_ordered(!is_shared, wrow, srow, planes + size_t(t) * np * ps, ps, np, xsc + size_t(t) * G, G);
+    }
+    total[m] = v;
+  }
+  const int slot = t == 0 ? gslot[0] : gslot[1], trow = t == 0 ? grow[0] : grow[1];
+  if (STAGE == 0) {
+    const float g = fminf(bf16_to_f32(bf16_round_f64(total[0])), p.swiglu_limit);
+    const float u = fmaxf(fminf(bf16_to_f32(bf16_round_f64(total[NMAT - 1])), p.swiglu_limit), -p.swiglu_limit);
+    const float wk = is_shared ? 1.0f : reinterpret_cast<const float*>(p.weights)[slot];
+    const float silu = __fdiv_rn(g, __fadd_rn(1.0f, det_expf(-g)));
+    const uint16_t hb = f32_to_bf16(__fmul_rn(__fmul_rn(silu, u), wk));
+    if (is_shared) {
+      p.h[size_t(slot) * p.h_stride + j] = hb;
+    } else {  // the 32 columns of the block are one quantization group per token, one run of 32 lanes
+      const float hv = bf16_to_f32(hb);
+      float amax = fabsf(hv);
+#pragma unroll
+      for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 32));
+      const int exponent = e8m0_scale_exponent(amax);
+      q.hq[size_t(slot) * p.h_stride + j] = uint8_t(e4m3x4_encode_finite(e8m0_scaled(hv, exponent), 0.0f, 0.0f, 0.0f));
+      if (jc == 0) q.hs[size_t(slot) * (p.h_stride >> 5) + (j >> 5)] = uint8_t(exponent + 127);
+    }
+  } else {
+    const uint16_t o = bf16_round_f64(total[0]);
+    if (is_shared) p.shared_out[size_t(trow) * p.hidden + j] = o;
+    else {
+      p.contributions[size_t(slot) * p.hidden + j] = o;
+      if (j == 0 && p.done) p.done[slot] = 1u;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // The FP32-chain variant (kernels/moe_ffn.cu:469-576 W4A8, :764-865 W8A8 shared expert): the reference gives a 32-lane
 // warp to an output row; here a half wave plays the warp, lane for lane, so chunk ownership, the fma chains and the
 // xor-butterfly sum are the reference's and the result is bit-equal to it (up to its expf).

@@ -228,3 +228,50 @@ def test_e8m0_fp32_chain_variant_bit_exact(hidden, inter, shared_inter, rows, to
             assert np.array_equal(got[r, c], want), (r, c)
         assert np.array_equal(got_sh[r], orc.expert_ffn_e8m0_f32(0, xb[r], *sh_ref, limit, 1.0)), r
     assert np.all(op.done.cpu().numpy() == 1)
+
+
+@pytest.mark.parametrize("hidden,inter,shared_inter,rows,top_k", [
+    (128, 128, 128, 1, 1),    # one K block: waves without work, half a line of codes per row
+    (384, 128, 256, 2, 2),    # an odd number of K blocks, two tokens per instruction
+    (256, 640, 128, 5, 3),    # a ragged last block of output columns, an unpaired token
+    (1152, 384, 640, 1, 6),
+    (2304, 896, 384, 3, 2),
+])
+def test_e8m0_matrix_core_tiles_bit_exact_on_any_code(hidden, inter, shared_inter, rows, top_k):
+    """The matrix-core kernels of the exact arithmetic at the edges of their tiles, on weight codes drawn uniformly (every E2M1
+    nibble, both zeros; every finite E4M3 code, so products over the whole exponent range) and on activations whose groups
+    mix the largest with the smallest E4M3 magnitudes, some groups all zero. Exact: any rounded product or sum is a failure."""
+    rng = np.random.default_rng(9000 + hidden + rows)
+    experts, limit = max(6, top_k), 7.0
+    routed, ref, sh_table, sh_ref = _tables(experts, hidden, inter, shared_inter, 9100 + rows)
+    for e in range(experts):
+        v = routed.expert_views(e)
+        for i in range(3):
+            codes = rng.integers(0, 256, tuple(v[2 * i].shape), dtype=np.uint8)
+            scales = rng.integers(116, 122, tuple(v[2 * i + 1].shape), dtype=np.uint8)
+            codes[0, :16] = 0  # an all-zero group with a scale of its own
+            scales[0, 0] = 3
+            v[2 * i].copy_(torch.from_numpy(codes)); v[2 * i + 1].copy_(torch.from_numpy(scales))
+            ref[e][2 * i], ref[e][2 * i + 1] = codes, scales
+    v = sh_table.expert_views(0)
+    for i in range(3):
+        codes = rng.integers(0, 256, tuple(v[2 * i].shape), dtype=np.uint8)
+        codes[(codes & 127) == 127] = 0x7e
+        scales = rng.integers(108, 111, tuple(v[2 * i + 1].shape), dtype=np.uint8)
+        v[2 * i].copy_(torch.from_numpy(codes)); v[2 * i + 1].copy_(torch.from_numpy(scales))
+        sh_ref[2 * i], sh_ref[2 * i + 1] = codes, scales
+    mag = np.exp2(rng.uniform(-16, 0, (rows, hidden))) * rng.choice([-1.0, 1.0], (rows, hidden))
+    mag[:, ::32] = 1.0
+    mag[0, 32:64] = 0.0
+    x = torch.from_numpy(mag.astype(np.float32)).to(torch.bfloat16)
+    ids = torch.from_numpy(np.stack([rng.permutation(experts)[:top_k] for _ in range(rows)]).astype(np.int32))
+    wt = torch.from_numpy(rng.uniform(0.05, 0.5, (rows, top_k)).astype(np.float32))
+    op = E8m0DecodeOps(routed, sh_table.shared_struct(0), rows, top_k, limit)
+    contrib, shared_out = op.contribute(x.to(DEV), ids.to(DEV), wt.to(DEV))
+    torch.cuda.synchronize()
+    got, got_sh, xb = bits(contrib), bits(shared_out), bits(x)
+    for r in range(rows):
+        for c in range(top_k):
+            assert np.array_equal(got[r, c], orc.expert_ffn_e8m0(1, xb[r], *ref[int(ids[r, c])], limit, float(wt[r, c]))), (r, c)
+        assert np.array_equal(got_sh[r], orc.expert_ffn_e8m0(0, xb[r], *sh_ref, limit, 1.0)), r
+    assert np.all(op.done.cpu().numpy() == 1)
