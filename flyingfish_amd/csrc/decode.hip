@@ -25,6 +25,8 @@ int decode_token_layer_bf16(const FinishParams& q, hipStream_t st);
 int decode_token_layer_fp8c(const FinishParams& q, hipStream_t st);
 int decode_form_launch(int fmt, int form, const DecodeParams& p, int stage_mask, hipStream_t st);
 int decode_form_grouped_launch(int fmt, int form, int rg, const DecodeParams& p, unsigned max_groups, int stage_mask, hipStream_t st);
+bool decode_form_rows_fit(int fmt, const DecodeParams& p);
+int decode_form_rows_launch(int fmt, int form, int rg, const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st);
 int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int stages, void* stream);
 int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, int H, int swiglu, float limit, void* act, void* shared_out,
                       int stage_mask, void* stream_);
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(1024) void k_group_assignments(const int* __restric
                                                             GroupDesc* __restrict__ groups, int* __restrict__ counters,
                                                             int rows, int top_k, int experts, int has_shared, int rgmax) {
   extern __shared__ int s_ids[];  // [A] expert id or -1
-  __shared__ int s_scan[FFMOE_MAX_EXPERTS];
+  __shared__ int s_scan[16];
   const int tid = threadIdx.x;
   const int A = rows * top_k;
   for (int a = tid; a < A; a += blockDim.x) {
@@ -90,17 +92,24 @@ __global__ __launch_bounds__(1024) void k_group_assignments(const int* __restric
   if (tid < experts)
     for (int a = 0; a < A; ++a) cnt += s_ids[a] == tid;
   const int chunks = (cnt + rgmax - 1) / rgmax;
-  // inclusive scan over experts (blockDim == 1024 >= experts)
-  s_scan[tid] = tid < experts ? chunks : 0;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int v = tid >= off ? s_scan[tid - off] : 0;
-    __syncthreads();
-    s_scan[tid] += v;
-    __syncthreads();
+  // inclusive scan over experts (blockDim == 1024 >= experts): inside the waves, then over the sixteen wave totals
+  int incl = tid < experts ? chunks : 0;
+  const int lane = tid & 63, wv = tid >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __builtin_amdgcn_ds_bpermute(((lane - off) & 63) << 2, incl);
+    if (lane >= off) incl += v;
   }
-  const int base = s_scan[tid] - chunks;
-  const int n_routed = s_scan[1023];
+  if (lane == 63) s_scan[wv] = incl;
+  __syncthreads();
+  int before = 0, n_routed = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    const int v = s_scan[w];
+    before += w < wv ? v : 0;
+    n_routed += v;
+  }
+  const int base = before + incl - chunks;
   if (tid < experts && cnt > 0) {
     int filled = 0, gi = base;
     for (int a = 0; a < A; ++a) {
@@ -263,15 +272,30 @@ static int decode_impl(const ffmoe_expert_table* table, const ffmoe_shared_exper
     // the expert's weights (the same bits as one block per (row, choice), which one row, cohorts beyond the grouping
     // kernel's LDS and FFMOE_FORM_GROUPED=0 keep).
     int frg = FFMOE_DECODE_RG;
-    while (frg > 1 && size_t(frg) * kmax_lds * 2 > 64 * 1024) frg >>= 1;
+    const bool rows_fit = decode_form_rows_fit(fmt, p);
+    if (rows_fit)
+      while (frg > 1 && frg / 2 >= R) frg >>= 1;  // the streaming kernels: no more tokens per group than there are rows
+    else
+      while (frg > 1 && size_t(frg) * kmax_lds * 2 > 64 * 1024) frg >>= 1;
     const bool can_group = R > 1 && frg > 1 && size_t(A) * sizeof(int) <= 64 * 1024 && uint64_t(LA) + R + 2 <= 65535;
-    // it pays from about two rows per expert on (per-channel FP8, hidden 4096, 32 experts top-4: 64 rows 0.89 against
-    // 1.56 ms in the Lane16 order, 512 rows 3.6 against 13.0 ms; 8 rows 0.41 against 0.30 ms)
+    // one block per (row, group) kernels: it pays from about two rows per expert on (per-channel FP8, hidden 4096, 32 experts
+    // top-4: 64 rows 0.89 against 1.56 ms in the Lane16 order, 512 rows 3.6 against 13.0 ms; 8 rows 0.41 against 0.30 ms)
     bool grouped = can_group && A >= 2 * E;
+    if (rows_fit) {
+      // Streaming kernels: grouping costs its launch and 3 - 5 us of worse balance and saves the passes over weights that tokens
+      // share. Expected passes saved x bytes of an expert, per-channel FP8, Lane16, us grouped / not: 2 rows top-6 of 64 at
+      // 4096 / 1536 (25 MB) 79 / 68, 2 rows top-8 at 7168 / 2048 (83 MB) 152 / 151, 4 rows top-6 (92 MB) 119 / 107, 4 rows top-8
+      // (380 MB) 252 / 266, 8 rows top-6 (250 MB) 169 / 186, 32 rows (3.1 GB) 389 / 660.
+      double missed = 1.0;
+      for (int i = 0; i < R && missed > 1e-3; ++i) missed *= 1.0 - double(K) / E;
+      const double saved = double(A) - E * (1.0 - missed) + (shared ? R - 1 : 0);
+      grouped = can_group && saved * 3.0 * H * I * (fmt == FFMOE_FMT_BF16 ? 2 : 1) > 150e6;
+    }
     if (const char* f = getenv("FFMOE_FORM_GROUPED")) grouped = can_group && atoi(f) != 0;
     if (!grouped) {
       p.groups = nullptr;
       p.counters = nullptr;
+      if (rows_fit) return decode_form_rows_launch(fmt, form, 1, p, (long long)A, shared ? R : 0, stage_mask, st);
       return decode_form_launch(fmt, form, p, stage_mask, st);
     }
     p.groups = (GroupDesc*)(sc + hbytes);
@@ -280,6 +304,10 @@ static int decode_impl(const ffmoe_expert_table* table, const ffmoe_shared_exper
     if (stage_mask & 1) hipLaunchKernelGGL(k_group_assignments, dim3(1), dim3(1024), A * sizeof(int), st, args->ids, args->active, table->valid, p.generation,
                                            p.assignment_gen, p.groups, p.counters, R, K, E, p.has_shared, frg);
     FF_TRY(ff_launch_status());
+    if (rows_fit) {  // an expert leaves at most one group unfilled
+      const long long most = (long long)E + (long long)A / frg;
+      return decode_form_rows_launch(fmt, form, frg, p, (long long)A < most ? (long long)A : most, shared ? (R + frg - 1) / frg : 0, stage_mask, st);
+    }
     // at most one group per assignment and per shared row, so A + R bounds what the counters can hold
     return decode_form_grouped_launch(fmt, form, frg, p, unsigned(A + R), stage_mask, st);
   }

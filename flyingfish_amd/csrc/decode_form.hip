@@ -24,4 +24,24 @@ int decode_form_grouped_launch(int fmt, int form, int rg, const DecodeParams& p,
   if (fmt == FFMOE_FMT_BF16) return form_grouped_fmt<FmtBf16>(form, rg, p, max_groups, stage_mask, st);
   return form_grouped_fmt<FmtFp8Channel>(form, rg, p, max_groups, stage_mask, st);
 }
+
+template <class F>
+static int form_rows_fmt(int form, int rg, const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st) {
+  const bool l16 = form == FFMOE_FORM_LANE16;
+#define FF_FORM_ROWS(T) \
+  (l16 ? launch_form_rows<F, FFMOE_FORM_LANE16_, T>(p, routed, shared, stage_mask, st) : launch_form_rows<F, FFMOE_FORM_LANE8_, T>(p, routed, shared, stage_mask, st))
+  switch (rg) {
+    case 8: return FF_FORM_ROWS(8);
+    case 4: return FF_FORM_ROWS(4);
+    case 2: return FF_FORM_ROWS(2);
+    default: return FF_FORM_ROWS(1);
+  }
+#undef FF_FORM_ROWS
+}
+bool decode_form_rows_fit(int fmt, const DecodeParams& p) { return fmt == FFMOE_FMT_BF16 ? form_rows_fit<FmtBf16>(p) : form_rows_fit<FmtFp8Channel>(p); }
+// rg: assignments of one expert per group (1: every assignment its own, no descriptors); routed, shared: upper bounds of the groups
+int decode_form_rows_launch(int fmt, int form, int rg, const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st) {
+  if (fmt == FFMOE_FMT_BF16) return form_rows_fmt<FmtBf16>(form, rg, p, routed, shared, stage_mask, st);
+  return form_rows_fmt<FmtFp8Channel>(form, rg, p, routed, shared, stage_mask, st);
+}
 }  // namespace ffmoe

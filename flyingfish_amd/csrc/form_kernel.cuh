@@ -313,6 +313,292 @@ __global__ __launch_bounds__(256) void k_decode_form_grouped(const DecodeParams 
   }
 }
 
+// The same sums with the weights streamed through LDS (contractions that are whole 128-byte lines of every weight row; the two
+// kernels above keep the others). A wave owns 32 weight rows - 16 gate rows and the up rows beside them, or 32 down rows -
+// and moves them in chunks of 128 bytes a row: eight lanes request one line, the chunk goes into the wave's own LDS buffer
+// (16-byte pieces XOR-swizzled by the row; LDS operations of a wave execute in order, so nothing waits between its writes
+// and reads) and every lane picks out the elements of its accumulators. Requested in accumulator order instead, a row gives
+// 16 bytes per request and its line is looked up in the vector L1, and often fetched, eight times.
+//   Lane16: four lanes a row, four of the sixteen accumulators each, two rows per lane.
+//   Lane8:  eight lanes a row, every eighth vector of 8 elements each, four rows per lane.
+// A lane's rows share its reads of the activations, the tokens of a group (up to T) share the dequantization of its rows.
+// Bound by the vector ALUs next to HBM: dequantizing a per-channel FP8 weight to an FP32 operand takes 3 instructions
+// (conversion, scale, BF16 rounding, unpacking; pairs where the ISA has them), a token 1.5 more.
+// One token, 8 of 64 experts + shared at hidden 7168 / intermediate 2048, us before / now: per-channel FP8 Lane16 336 / 94,
+// Lane8 174 / 88 (397 MB: 4.5 TB/s), BF16 Lane16 420 / 148, Lane8 194 / 147 (5.4 TB/s); 4 rows at 4096 / 1536, top-6: Lane16
+// 282 / 96; 32 rows at 7168, in groups: Lane16 2305 / 920. One chunk ahead is enough for the groups of one FP8 token, two chunks
+// cost them waves; three or four change nothing for BF16.
+template <class F, int FORM>
+struct FormShape {
+  static constexpr int EB = std::is_same<F, FmtBf16>::value ? 2 : 1;  // bytes per weight
+  static constexpr int CH = 128 / EB;                                 // elements of a row per chunk
+  static constexpr int L = FORM == FFMOE_FORM_LANE16_ ? 4 : 8;        // lanes per row
+  static constexpr int NR = FORM == FFMOE_FORM_LANE16_ ? 2 : 4;       // rows per lane
+  static constexpr int EL = FORM == FFMOE_FORM_LANE16_ ? 4 : 8;  // elements of a lane per step: 4 | 8
+  static constexpr int STEP = FORM == FFMOE_FORM_LANE16_ ? 16 : 64;   // elements of a row per step
+  static constexpr int STEPS = CH / STEP;
+};
+constexpr int FFMOE_FORM_WAVE_LDS = 32 * 128;
+
+constexpr int FFMOE_FORM_SEG = 2048;  // elements of a token in LDS at a time: longer rows would leave one or two blocks per CU
+
+struct FormTile {
+  int K, out, j0;          // contraction, output columns, first column of the wave
+  bool live, is_shared;
+  uint64_t sl[4];          // STAGE 0: gate codes, scales, up codes, scales; STAGE 1: down codes, scales
+  int gn;
+};
+
+// N: tokens of the group as a constant (gn of them exist, the others repeat the last one and store nothing): as run-time tests inside
+// the loop the tokens' branches cost a group of one 40 %
+template <class F, int FORM, int STAGE, int N, int T>
+__device__ __forceinline__ void form_rows_run(const DecodeParams& p, const FormTile& f, const int (&grow)[T], const int (&gslot)[T], uint8_t* lds) {
+  using S = FormShape<F, FORM>;
+  constexpr int NR = S::NR, L = S::L, RPL = 64 / L;
+  constexpr bool L16 = FORM == FFMOE_FORM_LANE16_;
+  constexpr int NACC = L16 ? 4 : 1;
+  constexpr int D = N == 1 && S::EB == 1 ? 1 : 2;  // chunks on their way
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int K = f.K;
+  const int jb = f.live ? f.j0 : 0;
+  const uint32_t rowb = uint32_t(K) * S::EB;
+  const int NC = int(rowb >> 7);
+  // rows 8 h .. 8 h + 7 of the wave's buffer: their matrix and first weight row
+  uint64_t base[4];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int mat = STAGE == 1 ? 0 : (L16 ? h >> 1 : h & 1);
+    const int row = jb + (STAGE == 1 ? 8 * h : 8 * (L16 ? h & 1 : h >> 1));
+    base[h] = f.sl[2 * mat] + uint64_t(row) * rowb;
+  }
+  const uint32_t loff = uint32_t(lane >> 3) * rowb + uint32_t(lane & 7) * 16u;
+  u32x4 w[D][4];
+  auto request = [&](int s, int c) {  // past the end: one line with every lane, nothing reads it
+    const uint32_t off = c < NC ? loff + uint32_t(c) * 128u : 0u;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) w[s][h] = load16_stream(reinterpret_cast<const uint8_t*>(base[h]) + off);
+  };
+#pragma unroll
+  for (int s = 0; s < D; ++s) request(s, s);
+  // per-channel scales of this lane's rows
+  const int r = lane / L, sub = lane % L;
+  float scale[NR];
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    scale[n] = 1.0f;
+    if constexpr (S::EB == 1) {
+      const int mat = STAGE == 1 ? 0 : n & 1;
+      const int row = jb + (STAGE == 1 ? n * RPL : (n >> 1) * RPL) + r;
+      scale[n] = bf16_to_f32(load_global<uint16_t>(reinterpret_cast<const uint16_t*>(f.sl[2 * mat + 1]) + row));
+    }
+  }
+  uint8_t* wl = lds + size_t(wave) * FFMOE_FORM_WAVE_LDS;
+  uint8_t* xs = lds + 4 * FFMOE_FORM_WAVE_LDS;
+  auto key = [](int row) { return (row ^ (row >> 3)) & 7; };
+  float acc[NR][N][NACC];
+#pragma unroll
+  for (int n = 0; n < NR; ++n)
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+#pragma unroll
+      for (int a = 0; a < NACC; ++a) acc[n][t][a] = 0.0f;
+  for (int k0 = 0; k0 < K; k0 += FFMOE_FORM_SEG) {
+    const int len = K - k0 < FFMOE_FORM_SEG ? K - k0 : FFMOE_FORM_SEG;
+    if (k0 > 0) __syncthreads();  // the previous segment has been read
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      const int tt = t < f.gn ? t : f.gn - 1;
+      int row = grow[0], slot = gslot[0];
+#pragma unroll
+      for (int q = 1; q < (N < T ? N : T); ++q) { row = tt == q ? grow[q] : row; slot = tt == q ? gslot[q] : slot; }
+      const uint16_t* src = (STAGE == 0 ? p.x + size_t(row) * p.hidden : p.h + size_t(slot) * p.h_stride) + k0;
+      u32x4* d4 = reinterpret_cast<u32x4*>(xs + size_t(t) * FFMOE_FORM_SEG * 2);
+      if (tid < (len >> 3)) d4[tid] = load16(src + size_t(tid) * 8);
+    }
+    __syncthreads();
+    const int c_end = f.live ? (k0 + len) / S::CH : 0;
+    for (int c0 = k0 / S::CH; c0 < c_end; c0 += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        const int c = c0 + s;
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int row = 8 * h + (lane >> 3);
+          *reinterpret_cast<u32x4*>(wl + row * 128 + (((lane & 7) ^ key(row)) << 4)) = w[s][h];
+        }
+        request(s, c + D);
+        __builtin_amdgcn_wave_barrier();
+        if (c < c_end) {  // only the last segment can hold an odd number of chunks
+          const uint8_t* xc = xs + size_t(c * S::CH - k0) * 2 + sub * (S::EL * 2);
+#pragma unroll
+          for (int st = 0; st < S::STEPS; ++st) {
+            float wf[NR][S::EL];
+#pragma unroll
+            for (int n = 0; n < NR; ++n) {
+              const int row = n * RPL + r;
+              const int byte = (st * S::STEP + sub * S::EL) * S::EB;  // inside the row's chunk
+              const uint8_t* at = wl + row * 128 + (((byte >> 4) ^ key(row)) << 4) + (byte & 15);
+              if constexpr (S::EB == 1) {
+                uint32_t d[S::EL / 4];
+                if constexpr (S::EL == 4) d[0] = *reinterpret_cast<const uint32_t*>(at);
+                else { const u32x2 v = *reinterpret_cast<const u32x2*>(at); d[0] = v.x; d[1] = v.y; }
+#pragma unroll
+                for (int q = 0; q < S::EL / 4; ++q) {
+                  uint32_t w01, w23;
+                  dequant4_e4m3(d[q], scale[n], w01, w23);  // bf16(e4m3 * scale), src/fp8.rs:138-140
+                  wf[n][4 * q] = __uint_as_float(w01 << 16); wf[n][4 * q + 1] = __uint_as_float(w01 & 0xffff0000u);
+                  wf[n][4 * q + 2] = __uint_as_float(w23 << 16); wf[n][4 * q + 3] = __uint_as_float(w23 & 0xffff0000u);
+                }
+              } else {
+                uint32_t d[S::EL / 2];
+                if constexpr (S::EL == 4) { const u32x2 v = *reinterpret_cast<const u32x2*>(at); d[0] = v.x; d[1] = v.y; }
+                else { const u32x4 v = *reinterpret_cast<const u32x4*>(at); d[0] = v[0]; d[1] = v[1]; d[2] = v[2]; d[3] = v[3]; }
+#pragma unroll
+                for (int q = 0; q < S::EL / 2; ++q) { wf[n][2 * q] = __uint_as_float(d[q] << 16); wf[n][2 * q + 1] = __uint_as_float(d[q] & 0xffff0000u); }
+              }
+            }
+#pragma unroll
+            for (int t = 0; t < N; ++t) {
+              const uint8_t* xa = xc + t * (FFMOE_FORM_SEG * 2) + st * (S::STEP * 2);
+              float xf[S::EL];
+              uint32_t d[S::EL / 2];
+              if constexpr (S::EL == 4) { const u32x2 v = *reinterpret_cast<const u32x2*>(xa); d[0] = v.x; d[1] = v.y; }
+              else { const u32x4 v = *reinterpret_cast<const u32x4*>(xa); d[0] = v[0]; d[1] = v[1]; d[2] = v[2]; d[3] = v[3]; }
+#pragma unroll
+              for (int q = 0; q < S::EL / 2; ++q) { xf[2 * q] = __uint_as_float(d[q] << 16); xf[2 * q + 1] = __uint_as_float(d[q] & 0xffff0000u); }
+#pragma unroll
+              for (int n = 0; n < NR; ++n) {
+                if constexpr (L16) {
+#pragma unroll
+                  for (int a = 0; a < 4; ++a) acc[n][t][a] = __fmaf_rn(xf[a], wf[n][a], acc[n][t][a]);
+                } else {
+                  float inner = 0.0f;
+#pragma unroll
+                  for (int e = 0; e < S::EL; ++e) inner = __fmaf_rn(xf[e], wf[n][e], inner);
+                  acc[n][t][0] = __fadd_rn(acc[n][t][0], inner);
+                }
+              }
+            }
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+  }
+  if (!f.live) return;
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    if (t >= f.gn || t >= T) break;
+    const int row = grow[t < T ? t : 0], slot = gslot[t < T ? t : 0];
+    float total[NR];  // in every lane of the row: the trees of form_dot, whose additions commute
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+      if constexpr (L16) {
+        float v = __fadd_rn(__fadd_rn(acc[n][t][0], acc[n][t][1]), __fadd_rn(acc[n][t][2], acc[n][t][3]));
+        v = __fadd_rn(v, dpp_or<DPP_QUAD_SWAP1, 0xf>(0.0f, v));
+        total[n] = __fadd_rn(v, dpp_or<DPP_QUAD_SWAP2, 0xf>(0.0f, v));
+      } else {
+        float v = acc[n][t][0];
+        v = __fadd_rn(v, lane_xor(v, 4));
+        v = __fadd_rn(v, dpp_or<DPP_QUAD_SWAP2, 0xf>(0.0f, v));
+        total[n] = __fadd_rn(v, dpp_or<DPP_QUAD_SWAP1, 0xf>(0.0f, v));
+      }
+    }
+    if (sub != (t & (L - 1))) continue;  // the tokens' epilogues go to different lanes
+    if (STAGE == 0) {
+      const bool reciprocal = L16 && (p.swiglu == FFMOE_SWIGLU_TWICE || p.swiglu == FFMOE_SWIGLU_CLAMPED_TWICE);
+#pragma unroll
+      for (int n = 0; n < NR; n += 2)
+        p.h[size_t(slot) * p.h_stride + f.j0 + (n >> 1) * RPL + r] =
+            form_swiglu(bround(total[n]), bround(total[n + 1]), p.swiglu, p.swiglu_limit, reciprocal);
+    } else {
+      float wk = 1.0f;
+      if (!f.is_shared)
+        wk = p.weights_f32 ? reinterpret_cast<const float*>(p.weights)[slot] : bf16_to_f32(reinterpret_cast<const uint16_t*>(p.weights)[slot]);
+#pragma unroll
+      for (int n = 0; n < NR; ++n) {
+        const int j = f.j0 + n * RPL + r;
+        if (f.is_shared) {
+          p.shared_out[size_t(row) * p.hidden + j] = f32_to_bf16(total[n]);
+        } else {
+          const float v = __fmul_rn(p.routed_weight == FFMOE_WEIGHT_AFTER_DOWN_BF16 ? bround(total[n]) : total[n], wk);
+          p.contributions[size_t(slot) * p.hidden + j] = f32_to_bf16(v);
+          if (j == 0 && p.done) p.done[slot] = 1u;
+        }
+      }
+    }
+  }
+}
+
+// grid: (group, tile of output columns) pairs, the shared expert's first
+template <class F, int FORM, int STAGE, int T>
+__global__ __launch_bounds__(256) void k_decode_form_rows(const DecodeParams p) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  constexpr int COLS = STAGE == 0 ? 64 : 128;  // output columns per block
+  const int wave = uni(int(threadIdx.x) >> 6);
+  const int A = p.rows * p.top_k;
+  const int tiles_s = ((STAGE == 0 ? p.shared_inter : p.hidden) + COLS - 1) / COLS, tiles_r = ((STAGE == 0 ? p.inter : p.hidden) + COLS - 1) / COLS;
+  const int n_routed = p.groups ? load_uniform<int>(p.counters) : A;
+  const int n_shared = p.groups ? load_uniform<int>(p.counters + 1) : (p.has_shared ? p.rows : 0);
+  int group, tile;
+  {
+    const uint32_t b = blockIdx.x, bs = uint32_t(n_shared) * uint32_t(tiles_s);
+    if (b < bs) {
+      group = int(b / uint32_t(tiles_s));
+      tile = int(b) - group * tiles_s;
+      group += n_routed;
+    } else {
+      group = int((b - bs) / uint32_t(tiles_r));
+      if (group >= n_routed) return;
+      tile = int(b - bs) - group * tiles_r;
+    }
+  }
+  int expert, grow[T], gslot[T];
+  FormTile f;
+  load_group<T>(p, group, expert, f.gn, grow, gslot);
+  if (f.gn == 0) return;  // inactive, invalid or stale choice: nothing written, done stays 0
+  f.is_shared = expert < 0;
+  f.K = STAGE == 0 ? p.hidden : (f.is_shared ? p.shared_inter : p.inter);
+  f.out = STAGE == 0 ? (f.is_shared ? p.shared_inter : p.inter) : p.hidden;
+  f.j0 = tile * COLS + wave * (COLS / 4);
+  f.live = f.j0 < f.out;  // columns come in multiples of 64: a wave is inside or outside as a whole
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = STAGE == 0 ? i : 4 + (i & 1);
+    f.sl[i] = f.is_shared ? p.shared_slot[e] : load_uniform<uint64_t>(p.slots + size_t(expert) * 6 + e);
+  }
+  if (T == 1 || f.gn == 1) form_rows_run<F, FORM, STAGE, 1, T>(p, f, grow, gslot, lds);
+  else if (T == 2 || f.gn == 2) form_rows_run<F, FORM, STAGE, 2, T>(p, f, grow, gslot, lds);
+  else if (f.gn == 3) form_rows_run<F, FORM, STAGE, 3, T>(p, f, grow, gslot, lds);
+  else if (T == 4 || f.gn == 4) form_rows_run<F, FORM, STAGE, 4, T>(p, f, grow, gslot, lds);
+  else if (f.gn <= 6) form_rows_run<F, FORM, STAGE, 6, T>(p, f, grow, gslot, lds);
+  else form_rows_run<F, FORM, STAGE, 8, T>(p, f, grow, gslot, lds);
+}
+
+// whole lines of every row: the streaming form of the kernels applies
+template <class F>
+bool form_rows_fit(const DecodeParams& p) {
+  constexpr int CH = FormShape<F, FFMOE_FORM_LANE16_>::CH;
+  return p.hidden % CH == 0 && p.inter % CH == 0 && (!p.has_shared || p.shared_inter % CH == 0);
+}
+
+template <class F, int FORM, int T>
+int launch_form_rows(const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st) {
+  const long long b0 = routed * ((p.inter + 63) / 64) + shared * ((p.shared_inter + 63) / 64), b1 = (routed + shared) * ((p.hidden + 127) / 128);
+  if (b0 >= (1ll << 31) || b1 >= (1ll << 31)) return ff_fail(FFMOE_ERR_SHAPE, "%lld groups exceed the launch grid", routed + shared);
+  constexpr size_t lds = 4 * FFMOE_FORM_WAVE_LDS + size_t(T) * FFMOE_FORM_SEG * 2;
+  if (stage_mask & 1) {
+    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 0, T>), dim3((unsigned)b0), dim3(256), lds, st, p);
+    FF_TRY(ff_launch_status());
+  }
+  if (stage_mask & 2) {
+    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 1, T>), dim3((unsigned)b1), dim3(256), lds, st, p);
+    FF_TRY(ff_launch_status());
+  }
+  return 0;
+}
+
 template <class F, int FORM, int RG>
 int launch_form_grouped(const DecodeParams& p, unsigned max_groups, int stage_mask, hipStream_t st) {
   constexpr int ROWS = 256 / (FORM == FFMOE_FORM_LANE16_ ? 2 : 8);

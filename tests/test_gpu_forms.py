@@ -178,3 +178,32 @@ def test_form_entry_rejects_other_formats():
     w = torch.ones((1, 1), device=DEV)
     with pytest.raises(capi.FfmoeError):
         op.contribute(x, ids, w, form=capi.FORM_LANE8)
+
+
+@pytest.mark.parametrize("fmt", [capi.FMT_BF16, capi.FMT_FP8_CHANNEL])
+@pytest.mark.parametrize("form", [capi.FORM_LANE16, capi.FORM_LANE8])
+@pytest.mark.parametrize("hidden,inter,rows", [
+    (128, 128, 1),     # one line per row
+    (2176, 128, 2),    # a token longer than its LDS segment, an odd number of lines behind it
+    (384, 384, 3), (256, 128, 4), (256, 128, 5), (256, 128, 6), (256, 128, 7), (256, 128, 8), (256, 256, 9),  # every group size
+])
+def test_streamed_form_kernels_bit_exact(fmt, form, hidden, inter, rows, monkeypatch):
+    """The line-streaming kernels at the edges of their chunks, segments and group sizes, every row on one of two experts:
+    contributions and the shared row equal to the oracle's orders bit for bit, grouped and one assignment at a time."""
+    experts, top_k = 2, 1
+    table, ref, sh, x, _, wt = _case(fmt, experts, hidden, inter, rows, top_k, 6000 + rows, True)
+    ids = torch.zeros((rows, top_k), dtype=torch.int32)
+    ids[-1, 0] = 1
+    oform = orc.LANE16 if form == capi.FORM_LANE16 else orc.LANE8
+    kind = orc.SILU_RCP if form == capi.FORM_LANE16 else orc.SILU_DIV
+    xb = bits(x)
+    want = np.stack([orc.expert_ffn(xb[r], *ref[int(ids[r, 0])], float(wt[r, 0]), orc.TWICE, 0.0, orc.AFTER_DOWN_BF16, oform, kind) for r in range(rows)])
+    want_sh = np.stack([orc.expert_ffn(xb[r], *ref[experts], 1.0, orc.TWICE, 0.0, orc.AFTER_DOWN_BF16, oform, kind, apply_weight=False) for r in range(rows)])
+    for grouped in ("1", "0"):
+        monkeypatch.setenv("FFMOE_FORM_GROUPED", grouped)
+        op = DecodeOps(table, sh, rows, top_k, weights_f32=True)
+        contrib, shared_out = op.contribute(x.to(DEV), ids.to(DEV), wt.to(DEV), form=form)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(contrib)[:, 0], want), grouped
+        assert np.array_equal(bits(shared_out), want_sh), grouped
+        assert np.all(op.done.cpu().numpy() == 1)
