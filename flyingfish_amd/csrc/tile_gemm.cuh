@@ -1,0 +1,197 @@
+// Dense W8A8 GEMM over many rows: a 128 x 128 output tile per block of four waves, both operands through
+// LDS by direct loads (global_load_lds), two blocks per CU.
+//
+// Same arithmetic as k_w8a8_grouped (w8a8_gemm.cuh), instruction for instruction, so the same bits: one
+// v_mfma_f32_16x16x128_f8f6f4 per 16 x 16 tile and K block, total = fma(block sum, sw * sx, total).
+//
+// What bounds it: operand traffic on its way into the CU. k_w8a8_grouped gives every wave 64 weight rows x 64 tokens, moves
+// the weights through registers into a wave-private transposition buffer and so passes 24 KB through LDS per 16 matrix
+// instructions; its cache-resident rate stays near 1.2 PFLOP/s. Here two waves share each operand half, nothing goes through
+// registers on its way in, and a wave's 16 instructions read 16 KB; the 32 KB of a K block are requested one K block ahead
+// and land while the previous one is multiplied. Two independent blocks per CU (66 KB of LDS each) cover each other's
+// barriers, first loads and epilogues. Measured: 4096 x 7168 -> 4096 in 142 us = 1.69 PFLOP/s (matrix cores busy 40 % of
+// the cycles at the 2.0 GHz the chip holds here), 2048 x 2048 -> 7168 66 -> 47 us. The same loop without its loads takes
+// 105 us. Not faster: 256 x 128 tiles with three stages and one block per CU (145 us), 256 x 256 tiles (144), the next K block's
+// operands read into registers under the matrix work (155).
+#pragma once
+#include "w8a8_gemm.cuh"
+
+namespace ffmoe {
+
+// 16 (4) bytes per lane from base + offset into LDS at lds + 16 (4) x lane. No register holds the data, so the caller's
+// s_waitcnt before the barrier that publishes the tile is all the bookkeeping there is. (m0 is a reserved register: nothing the
+// compiler generates for these kernels reads it, and it accepts no clobber of it.)
+__device__ __forceinline__ void lds_load16(uint32_t lds, uint64_t base, uint32_t offset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
+__device__ __forceinline__ void lds_load16(uint32_t lds, const void* p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ void lds_load4(uint32_t lds, const void* p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return uint32_t(uni(int(uint32_t(uintptr_t((const __attribute__((address_space(3))) void*)p)))));
+}
+
+// Waves: wave / 2 is the weight half (64 rows), wave % 2 the token half (64 tokens). LDS rows are 128 bytes, 16-byte piece
+// c of row r at c ^ (r / 2 & 7), so that the 16 rows of an operand read cover all 64 banks (keyed by r & 7 half of the LDS cycles
+// were conflicts); the swizzle is applied to the source address, since a direct load writes its lanes in order.
+template <int MODE>
+__global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
+  struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; float sx[4][64]; };
+  __shared__ __attribute__((aligned(16))) Stage stage[2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int wr = wave >> 1, wt = wave & 1;
+  const int K = p.K, N = p.N, KB = K >> 7;
+  const uint32_t total = p.total_units;
+  const int ntiles = (N + (MODE == 0 ? 63 : 127)) / (MODE == 0 ? 64 : 128);
+  const int groups = (p.rows_total + 127) / 128;
+  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3, per_xcd = gridDim.x >> 3;
+  const uint32_t span = (total + 7u) >> 3;
+  const uint32_t span_end = min(total, (xcd + 1u) * span);
+  const uint32_t lds_w[2] = {lds_address(stage[0].w) + uint32_t(wave) * 4096u, lds_address(stage[1].w) + uint32_t(wave) * 4096u};
+  const uint32_t lds_t[2] = {lds_address(stage[0].t) + uint32_t(wave) * 4096u, lds_address(stage[1].t) + uint32_t(wave) * 4096u};
+  const uint32_t lds_s[2] = {lds_address(stage[0].sx[wave]), lds_address(stage[1].sx[wave])};
+  const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ (lane >> 4)) << 4);  // odd requests: piece ^ 4
+  // operand reads: row lane % 16, bytes 32 c .. 32 c + 31 of the K block for lane group c
+  const int r16 = lane & 15, c2 = (lane >> 4) * 2;
+  const int rd_lo = r16 * 128 + ((c2 ^ (r16 >> 1)) << 4), rd_hi = r16 * 128 + (((c2 + 1) ^ (r16 >> 1)) << 4);
+
+  for (uint32_t u = xcd * span + slot; u < span_end; u += per_xcd) {
+    // blocks of eight column tiles, row groups inside: the blocks of an XCD run an 8 x 8 window of tiles (4096 x 7168 -> 4096:
+    // 172 -> 158 us against row groups innermost, whose window is 2 x 32)
+    const int tb = int(u) / (groups * 8), v = int(u) - tb * groups * 8;
+    const int width = min(8, ntiles - tb * 8);
+    const int t = tb * 8 + v % width, start = (v / width) * 128, n = min(128, p.rows_total - start);
+    const uint64_t wc[2] = {p.w0_codes, MODE == 0 ? p.w1_codes : p.w0_codes}, ws[2] = {p.w0_scales, MODE == 0 ? p.w1_scales : p.w0_scales};
+    // Output column of this wave's fragment f; fragments past N are clamped onto the last 16 rows and dropped at the store.
+    // MODE 0: fragments 0, 1 are gate rows, 2, 3 the up rows of the same columns.
+    auto column = [&](int half, int f) { return MODE == 0 ? t * 64 + half * 32 + (f & 1) * 16 : t * 128 + half * 64 + f * 16; };
+    uint64_t wbase[4];  // request i of this wave: eight weight rows of fragment 2 (wave % 2) + i / 2 of weight half wave / 2
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int f = 2 * wt + (i >> 1);
+      wbase[i] = uni64((MODE == 0 ? wc[f >> 1] : wc[0]) + uint64_t(min(column(wr, f), N - 16) + (i & 1) * 8) * uint64_t(K));
+    }
+    const uint8_t* tsrc[4];  // request i: token rows 32 wave + 8 i + lane / 8
+    const float* ssrc;       // the scales of this wave's 64 tokens
+    auto token_row = [&](int m) { return start + min(m, n - 1); };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) tsrc[i] = p.a_codes + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * K + (((lane & 7) ^ (lane >> 4) ^ 4 * (i & 1)) << 4);
+    ssrc = p.a_scales + size_t(token_row(wt * 64 + lane)) * KB;
+    // one 128-row scale block per wave (its columns sit inside one), lane l keeps K block l (+ 64)
+    const int srow = min(column(wr, 0), N - 16) >> 7;
+    const float* sw0 = reinterpret_cast<const float*>(ws[0]) + size_t(srow) * KB;
+    const float* sw1 = reinterpret_cast<const float*>(ws[1]) + size_t(srow) * KB;
+
+    auto request = [&](int kb, int b) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lds_load16(lds_w[b] + i * 1024u, wbase[i] + uint64_t(uint32_t(kb) * 128u), woff ^ (64u * (i & 1)));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lds_load16(lds_t[b] + i * 1024u, tsrc[i] + uint32_t(kb) * 128u);
+      lds_load4(lds_s[b], ssrc + kb);
+    };
+    __syncthreads();  // the previous unit's last tile has been read
+    request(0, 0);
+
+    float acc[4][4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][f][r] = 0.0f;
+
+    auto block = [&](int kb, int b, float s0, float s1) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();  // K block kb is there for every wave, and nobody reads the other buffer any more
+      if (kb + 1 < KB) request(kb + 1, b ^ 1);
+      const uint8_t* wl = stage[b].w + wr * 8192;
+      const uint8_t* tl = stage[b].t + wt * 8192;
+      const float* sl = stage[b].sx[wave] + r16;
+      v8i wf[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(wl + f * 2048 + rd_lo), hi = *reinterpret_cast<const u32x4*>(wl + f * 2048 + rd_hi);
+        wf[f] = v8i{int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]), int(hi[0]), int(hi[1]), int(hi[2]), int(hi[3])};
+      }
+      u32x4 tlo[2], thi[2];
+      float sx[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) sx[m] = sl[16 * m];
+      tlo[0] = *reinterpret_cast<const u32x4*>(tl + rd_lo);
+      thi[0] = *reinterpret_cast<const u32x4*>(tl + rd_hi);
+      v4f pr[2][4];
+      // row fragment m's products are folded into the totals while fragment m + 1 is in the matrix core
+#pragma unroll
+      for (int m = 0; m <= 4; ++m) {
+        if (m < 4) {
+          if (m + 1 < 4) {
+            tlo[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_lo);
+            thi[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_hi);
+          }
+          const u32x4 lo = tlo[m & 1], hi = thi[m & 1];
+          const v8i tok = {int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]), int(hi[0]), int(hi[1]), int(hi[2]), int(hi[3])};
+#pragma unroll
+          for (int f = 0; f < 4; ++f) pr[m & 1][f] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[f], tok, v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0, 0, 0, 0);
+        }
+        if (m > 0) {
+          const float sc0 = __fmul_rn(s0, sx[m - 1]), sc1 = __fmul_rn(s1, sx[m - 1]);
+#pragma unroll
+          for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[m - 1][f][r] = __fmaf_rn(pr[(m - 1) & 1][f][r], (MODE == 0 && f >= 2) ? sc1 : sc0, acc[m - 1][f][r]);
+          // pins the fmas in front of the fence: without it they all end up behind the last one, after the matrix work
+#pragma unroll
+          for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) asm volatile("" ::"v"(acc[m - 1][f][r]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    for (int kb0 = 0; kb0 < KB; kb0 += 64) {
+      const int kl = min(kb0 + lane, KB - 1);
+      const float swl0 = landed(load_global<float>(sw0 + kl));
+      const float swl1 = MODE == 0 ? landed(load_global<float>(sw1 + kl)) : swl0;
+      const int kend = min(KB, kb0 + 64);
+      auto scale = [&](float v, int kb) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), kb - kb0)); };
+      for (int kb = kb0; kb < kend; kb += 2) {  // kb0 is even: buffer = parity of the K block
+        block(kb, 0, scale(swl0, kb), scale(swl1, kb));
+        if (kb + 1 < kend) block(kb + 1, 1, scale(swl0, kb + 1), scale(swl1, kb + 1));
+      }
+    }
+
+    const int sub = (lane >> 4) * 4;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int token = wt * 64 + 16 * m + r16;
+      if (token < n) {
+        const int pos = start + token;
+        if (MODE == 0) {
+#pragma unroll
+          for (int f = 0; f < 2; ++f) {
+            const int col = column(wr, f);
+            if (col + 16 <= N) {
+              uint32_t o[4];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[r] = swiglu_bf16_two_branch(bround(acc[m][f][r]), bround(acc[m][f + 2][r]), p.swiglu, p.limit);
+              *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col + sub) = u32x2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
+            }
+          }
+        } else {
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            const int col = column(wr, f);
+            if (col + 16 <= N)
+              *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col + sub) = u32x2{pack_bf16x2(acc[m][f][0], acc[m][f][1]), pack_bf16x2(acc[m][f][2], acc[m][f][3])};
+          }
+        }
+      }
+    }
+  }
+}
+
+}  // namespace ffmoe

@@ -1,0 +1,11 @@
+// Launch functions of tiles.hip
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace ffmoe {
+struct GemmParams;
+// W8A8 on 128 x 128 tiles (MODE of w8a8_gemm.cuh; a gate/up tile is 64 activation columns): units of a dense call
+inline uint32_t tile_units(int mode, int rows, int n) { return uint32_t((rows + 127) / 128) * uint32_t(mode == 0 ? (n + 63) / 64 : (n + 127) / 128); }
+int launch_w8a8_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream);
+}  // namespace ffmoe

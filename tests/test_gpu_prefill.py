@@ -11,7 +11,7 @@ import torch
 
 import oracle as orc
 from flyingfish_amd import capi, ops, synth
-from helpers import assert_close_with_rare_outliers, assert_swiglu_close, assert_close_bf16, assert_weighted_down_close, bf16_tensor, bits
+from helpers import assert_close_with_rare_outliers, assert_swiglu_close, assert_close_bf16, assert_weighted_down_close, bf16_tensor, bits, make_table
 
 pytestmark = pytest.mark.gpu
 # Values behind two composed stages (end to end) or behind a twice-rounded product (activations of the matrix-core paths):
@@ -39,6 +39,37 @@ def test_linear_w8a8_matches_oracle(m, n, k):
     torch.cuda.synchronize()
     assert_close_bf16(bits(y), want, "w8a8 linear vs 32-lane order", max_ulp=1)
     assert_close_bf16(bits(y), want64, "w8a8 linear vs FP64", max_ulp=1)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 128), (127, 144, 256), (129, 128, 384), (130, 272, 8320), (300, 1168, 1024), (1100, 400, 256)])
+def test_linear_w8a8_tile_kernel_equals_the_group_kernel_bitwise(m, n, k, monkeypatch):
+    """Ragged rows and columns, one to sixty-five K blocks, one and several windows of column tiles."""
+    wc, ws = _fp8_matrix(n, k, m * 7 + n)
+    x = synth.normal((m, k), 1.0, 5 + m, dtype=torch.bfloat16)
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_TILE", switch)
+        out.append(ops.Fp8Ops.linear(wc.cuda(), ws.cuda(), x.cuda(), capi.ACT_FP8_BLOCK128))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,inter", [(65, 128), (200, 384)])
+def test_prefill_shared_expert_tile_kernel_equals_the_group_kernel_bitwise(rows, inter, monkeypatch):
+    table, _ = make_table(capi.FMT_FP8_BLOCK128, 4, 256, inter, 77)
+    shared = table.shared_struct(3)
+    table.experts = 3
+    x = synth.normal((rows, 256), 1.0, 78).to(torch.bfloat16).cuda()
+    ids = torch.randint(0, 3, (rows, 1), generator=torch.Generator().manual_seed(5)).to(torch.int32).cuda()
+    w = torch.rand((rows, 1), generator=torch.Generator().manual_seed(6)).cuda()
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_TILE", switch)
+        op = ops.PrefillOps(table, rows, 1, shared=shared)
+        op.contribute(x, ids, w)
+        torch.cuda.synchronize()
+        out.append(op.shared_out.clone())
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
 def test_linear_w8a8_device_quantizer_chain():
