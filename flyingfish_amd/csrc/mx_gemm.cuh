@@ -43,6 +43,14 @@ struct MxParams {
   float limit;
 };
 
+// the contract's gate/up epilogue (kernels/moe_ffn.cu:601-700): BF16 dots, clamp, SiLU by division, x up x weight
+__device__ __forceinline__ uint32_t mx_swiglu(float gate, float up, float weight, float limit) {
+  const float g = fminf(bround(gate), limit);
+  const float u = fmaxf(fminf(bround(up), limit), -limit);
+  const float silu = __fdiv_rn(g, __fadd_rn(1.0f, det_expf(-g)));
+  return f32_to_bf16(__fmul_rn(__fmul_rn(silu, u), weight));
+}
+
 // PACKED 1: E2M1 codes [N, K / 2] (low nibble = even column), E8M0 scales [N, K / 32]
 // PACKED 0: E4M3 codes [N, K], E8M0 scales [N / 32, K / 32]
 // NW waves per block share one token tile (see k_w8a8_grouped): eight for 64-row groups of a cohort, one block per CU.
@@ -263,13 +271,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void k_mx_grouped(const M
             if (col0[f] + 16 <= N) {
               uint32_t o[4];
 #pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                // the contract's epilogue (kernels/moe_ffn.cu:601-700): BF16 dots, clamp, SiLU by division, x up x weight
-                const float g = fminf(bround(acc[m][f][r]), p.limit);
-                const float uu = fmaxf(fminf(bround(acc[m][f + 2][r]), p.limit), -p.limit);
-                const float silu = __fdiv_rn(g, __fadd_rn(1.0f, det_expf(-g)));
-                o[r] = f32_to_bf16(__fmul_rn(__fmul_rn(silu, uu), wk));
-              }
+              for (int r = 0; r < 4; ++r) o[r] = mx_swiglu(acc[m][f][r], acc[m][f + 2][r], wk, p.limit);
               const u32x2 v = {o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
               *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col) = v;
             }

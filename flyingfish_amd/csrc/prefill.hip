@@ -750,10 +750,12 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   uint8_t* s = (uint8_t*)args->scratch;
   PrefillBook b{(uint32_t*)(s + l.counts), (uint32_t*)(s + l.offsets), (uint32_t*)(s + l.gbase), (uint32_t*)(s + l.totals),
                 (int*)(s + l.perm), (GemmGroup*)(s + l.groups), (u32x2*)(s + l.units0), (u32x2*)(s + l.units1)};
-  const int mf = nv ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, !mx && !a16);
+  const char* mte = getenv("FFMOE_MX_TILE");
+  const bool mx_tile = mx && !(mte && atoi(mte) == 0);
+  const int mf = nv || mx_tile ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, !mx && !a16);
   const int tm = 16 * mf;
   // W8A8, W*A16 and MX cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
-  bool wide = mf == 4;
+  bool wide = mf == 4 && !mx_tile;
   if (const char* f = getenv("FFMOE_PREFILL_WIDE")) wide = (wide && atoi(f) != 0) || nv;
   const int tiles0 = wide ? (I + 255) / 256 : (I + 127) / 128, tiles1 = wide ? (H + 511) / 512 : (H + 255) / 256;
   // A shared expert of the routed experts' format and width rides in the routed launches as further row groups (W*A16
@@ -802,13 +804,15 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
     if (stages & 2) {
       p.a_codes = s + l.xq; p.a_scales = s + l.sx; p.units = b.units0; p.unit_total = b.totals + 0;
       p.weights = (const float*)args->weights; p.out = (uint16_t*)(s + l.act); p.K = H; p.N = I;
-      FF_TRY((launch_mx<0, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
+      if (mx_tile) FF_TRY(launch_mx_tile(0, p, blocks, stream));
+      else FF_TRY((launch_mx<0, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
     }
     if (stages & 4) FF_TRY(ffmoe_act_quant_e8m0(s + l.act, s + l.aq, s + l.sa, int(A), I, stream_));
     if (stages & 8) {
       p.a_codes = s + l.aq; p.a_scales = s + l.sa; p.units = b.units1; p.unit_total = b.totals + 1;
       p.weights = nullptr; p.out = (uint16_t*)args->contributions; p.done = args->done; p.K = I; p.N = H;
-      FF_TRY((launch_mx<1, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
+      if (mx_tile) FF_TRY(launch_mx_tile(1, p, blocks, stream));
+      else FF_TRY((launch_mx<1, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
     }
     if (shared) {
       const int smf = R > 32 ? 4 : R > 16 ? 2 : 1;

@@ -1,5 +1,6 @@
-// Launches of the 128 x 128 tile kernels (tile_gemm.cuh)
+// Launches of the kernels whose operand tiles go straight to LDS (tile_gemm.cuh, mx_tile.cuh)
 #include "tile_gemm.cuh"
+#include "mx_tile.cuh"
 #include "tiles.h"
 #include "api.h"
 
@@ -9,6 +10,17 @@ int launch_w8a8_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t
   if (mode == 0) hipLaunchKernelGGL(k_w8a8_tile<0>, dim3(blocks), dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(k_w8a8_tile<2>, dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
+}
+
+template <int MODE>
+static int launch_mx(const MxParams& p, unsigned blocks, hipStream_t stream) {
+  static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mx_tile<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, MX_TILE_LDS);
+  if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", MX_TILE_LDS, hipGetErrorString(ok));
+  hipLaunchKernelGGL(k_mx_tile<MODE>, dim3(blocks), dim3(256), MX_TILE_LDS, stream, p);
+  return ff_launch_status();
+}
+int launch_mx_tile(int mode, const MxParams& p, unsigned blocks, hipStream_t stream) {
+  return mode == 0 ? launch_mx<0>(p, blocks, stream) : launch_mx<1>(p, blocks, stream);
 }
 
 }  // namespace ffmoe
