@@ -1,14 +1,16 @@
 // Grouped GEMM of E2M1 / E8M0 experts against E4M3 / E8M0 activations: 128 weight rows x up to 64 tokens per block of four
 // waves, both operands through LDS by direct loads, two blocks per CU.
 //
-// Same instructions on the same operands in the same order as k_mx_grouped (mx_gemm.cuh), so the same bits; MODE as there.
+// MODE as in mx_gemm.cuh; one v_mfma_scale_f32_16x16x128_f8f6f4 per fragment pair and K block, K blocks in ascending order.
 //
 // What bounds it: a cohort is many experts of a few rows, which stream their weights, and a few popular ones, which run from
-// cache. k_mx_grouped asks for 64-byte pieces of the weight rows, holds them in registers on their way through a wave-private
-// transposition buffer, drains its queue at every K block and computes 64 tokens whatever the group holds. Here a stage is 256
-// columns, whole 128-byte lines of the weight rows; requests of up to 32 tokens run two stages ahead in a ring of three
-// (64 tokens: one stage, two buffers: 70 KB), a group moves and multiplies only its live 16-token fragments, and the second block of the
-// CU works while this one waits.
+// cache. A stage is 256 columns, whole 128-byte lines of the weight rows; requests for groups of up to 32 tokens run two stages
+// ahead in a ring of three (64 tokens: one stage, two buffers: 70 KB), a group moves and multiplies only its live 16-token
+// fragments, and the second block of the CU works while this one waits. Against 64-byte pieces of the weight rows moved through registers
+// and a transposition buffer, 64 tokens multiplied whatever the group holds (top-8 of 256 experts, hidden 7168, Zipf-like): 1500
+// tokens gate/up 1532 -> 1157 us, down 663 -> 600; a layer of 200 tokens, nearly all of it weight stream, 1464 -> 1052 us = 5.3 TB/s.
+// Not faster: the next unit's first stages requested behind this one's last (1180 / 605 us), the two blocks of a CU on
+// different halves of their XCD's units (1183 / 602).
 #pragma once
 #include "mx_gemm.cuh"
 #include "lds_load.cuh"
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(256, 2) void k_mx_tile(const MxParams p) {
 #pragma unroll
         for (int i = 0; i < MF; ++i)
           lds_load16(base + offsetof(MxStage<MF>, t) + uint32_t(i) * 4096u + uint32_t(wave) * 1024u, tsrc[i] + uint32_t(ks) * 256u - (half ? tback : 0));
-        const uint32_t soff = uint32_t(ks) * 8u - (half ? uint32_t(sdword) * 4u : 0u);
+        const int soff = ks * 8 - (half ? sdword * 4 : 0);  // signed: back to the row's first word where the only stage is a half
         lds_load4(base + offsetof(MxStage<MF>, ws) + uint32_t(wave) * 256u, wssrc + soff);
 #pragma unroll
         for (int i = 0; i < SW; ++i) lds_load4(base + offsetof(MxStage<MF>, ts) + uint32_t(wave) * (SW * 256u) + i * 256u, tssrc[i] + soff);

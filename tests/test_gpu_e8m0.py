@@ -170,6 +170,28 @@ def test_e8m0_prefill_on_the_mx_matrix_cores(rows, top_k, experts, hidden, inter
     assert_close_bf16(so, want_sd, "shared down projection of the device activations")
 
 
+@pytest.mark.parametrize("rows,hidden,inter", [(16, 128, 384), (33, 1280, 128), (65, 384, 640), (150, 768, 256)])
+def test_e8m0_prefill_rows_do_not_depend_on_their_group_bitwise(rows, hidden, inter):
+    """Groups of one to 64 rows, contractions of one to five stages with and without a last half, columns past the end of a
+    tile: every row equals itself in a cohort of its own."""
+    routed, _, _, _ = _tables(4, hidden, inter, 128, 800 + rows)
+    x = rand_bf16((rows, hidden), 1.0, 810 + rows).to(DEV)
+    g = synth.generator(820 + rows)
+    ids = torch.stack([torch.multinomial(torch.tensor([0.6, 0.3, 0.07, 0.03]), 2, generator=g) for _ in range(rows)]).to(torch.int32).to(DEV)
+    wt = (torch.rand((rows, 2), generator=g) * 0.5 + 0.05).to(DEV)
+
+    def op(n):
+        return PrefillOps(routed, n, 2, swiglu=capi.SWIGLU_CLAMPED_ONCE, swiglu_limit=7.0, routed_weight=capi.WEIGHT_BEFORE_DOWN_F32, weights_f32=True,
+                          act_mode=capi.ACT_E4M3_E8M0_32)
+    whole = op(rows)
+    got = whole.contribute(x, ids, wt)
+    one = op(1)
+    want = torch.stack([one.contribute(x[r:r + 1], ids[r:r + 1], wt[r:r + 1])[0].clone() for r in range(rows)])
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert int(whole.done.min()) == 1
+
+
 def test_e8m0_entry_checks_its_contract():
     routed, _, sh_table, _ = _tables(2, 64, 32, 32, 9)
     op = E8m0DecodeOps(routed, sh_table.shared_struct(0), 1, 1, 7.0)
