@@ -10,6 +10,10 @@ namespace ffmoe {
 __device__ __forceinline__ void lds_load16(uint32_t lds, uint64_t base, uint32_t offset) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
 }
+// with the streaming hint: the line is the first the L2 gives up again
+__device__ __forceinline__ void lds_load16_nt(uint32_t lds, uint64_t base, uint32_t offset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void* p) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
 }

@@ -396,6 +396,16 @@ bool nvfp4_lines_enabled() {
   return !(le && atoi(le) == 0);
 }
 
+// NVFP4 cohorts of a prompt chunk on the tile kernel (nvfp4_tile.cuh; FFMOE_NVFP4_TILE: 1 wherever it can run, 0 never; same
+// bits). It multiplies the live rows of 64-row groups, which pays where some experts are popular (256 experts, Zipf-like: 100
+// tokens 1168 -> 1058 us a layer, 200 tokens 1608 -> 1423, 1021 tokens 3136 -> 2414); on the one or two rows per expert of a
+// decode step the line kernel's wider blocks are ahead (32 tokens of top-8 of 256: 934 against 978 us; 64 tokens of 64
+// experts, even: 468 against 474).
+bool nvfp4_tiles(int rows, int top_k, int experts) {
+  if (const char* e = getenv("FFMOE_NVFP4_TILE")) return atoi(e) != 0;
+  return rows > 64 && (long long)rows * top_k > 3ll * experts;
+}
+
 // 16-row groups of the NVFP4 line kernel: one set of lines ahead and three blocks per CU (FFMOE_PREFILL_LINES_THREE_BLOCKS=0: two
 // sets ahead, two blocks; same bits); read at every call
 bool lines_three_blocks() {
@@ -483,16 +493,12 @@ int launch_tiles(int mode, GemmParams& p, hipStream_t stream) {
   return launch_w8a8_tile(mode, p, std::min<unsigned>((p.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
 }
 
-template <int MODE, int PACKED>
-int launch_mx(const MxParams& p, int mf, unsigned blocks, hipStream_t stream, bool wide = false) {
-  if (wide) {
-    hipLaunchKernelGGL((k_mx_grouped<4, MODE, PACKED, 2, 8>), dim3(blocks), dim3(512), 0, stream, p);
-    return ff_launch_status();
-  }
+template <int MODE>
+int launch_mx_dense(const MxParams& p, int mf, unsigned blocks, hipStream_t stream) {
   switch (mf) {
-    case 1: hipLaunchKernelGGL((k_mx_grouped<1, MODE, PACKED, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((k_mx_grouped<2, MODE, PACKED, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
-    default: hipLaunchKernelGGL((k_mx_grouped<4, MODE, PACKED, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
+    case 1: hipLaunchKernelGGL((k_mx_dense<1, MODE, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
+    case 2: hipLaunchKernelGGL((k_mx_dense<2, MODE, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
+    default: hipLaunchKernelGGL((k_mx_dense<4, MODE, 2>), dim3(blocks), dim3(256), 0, stream, p); break;
   }
   return ff_launch_status();
 }
@@ -750,12 +756,11 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   uint8_t* s = (uint8_t*)args->scratch;
   PrefillBook b{(uint32_t*)(s + l.counts), (uint32_t*)(s + l.offsets), (uint32_t*)(s + l.gbase), (uint32_t*)(s + l.totals),
                 (int*)(s + l.perm), (GemmGroup*)(s + l.groups), (u32x2*)(s + l.units0), (u32x2*)(s + l.units1)};
-  const char* mte = getenv("FFMOE_MX_TILE");
-  const bool mx_tile = mx && !(mte && atoi(mte) == 0);
-  const int mf = nv || mx_tile ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, !mx && !a16);
+  const bool nv_tile = a16 && table->format == FFMOE_FMT_NVFP4 && nvfp4_lines_enabled() && nvfp4_tiles(R, K, E) && H % 256 == 0 && I % 256 == 0;
+  const int mf = nv ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, (!mx && !a16) || mx || nv_tile);
   const int tm = 16 * mf;
-  // W8A8, W*A16 and MX cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
-  bool wide = mf == 4 && !mx_tile;
+  // W8A8 and W*A16 cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
+  bool wide = mf == 4 && !mx && !nv_tile;
   if (const char* f = getenv("FFMOE_PREFILL_WIDE")) wide = (wide && atoi(f) != 0) || nv;
   const int tiles0 = wide ? (I + 255) / 256 : (I + 127) / 128, tiles1 = wide ? (H + 511) / 512 : (H + 255) / 256;
   // A shared expert of the routed experts' format and width rides in the routed launches as further row groups (W*A16
@@ -804,15 +809,13 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
     if (stages & 2) {
       p.a_codes = s + l.xq; p.a_scales = s + l.sx; p.units = b.units0; p.unit_total = b.totals + 0;
       p.weights = (const float*)args->weights; p.out = (uint16_t*)(s + l.act); p.K = H; p.N = I;
-      if (mx_tile) FF_TRY(launch_mx_tile(0, p, blocks, stream));
-      else FF_TRY((launch_mx<0, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
+      FF_TRY(launch_mx_tile(0, p, blocks, stream));
     }
     if (stages & 4) FF_TRY(ffmoe_act_quant_e8m0(s + l.act, s + l.aq, s + l.sa, int(A), I, stream_));
     if (stages & 8) {
       p.a_codes = s + l.aq; p.a_scales = s + l.sa; p.units = b.units1; p.unit_total = b.totals + 1;
       p.weights = nullptr; p.out = (uint16_t*)args->contributions; p.done = args->done; p.K = I; p.N = H;
-      if (mx_tile) FF_TRY(launch_mx_tile(1, p, blocks, stream));
-      else FF_TRY((launch_mx<1, 1>(p, mf, wide ? blocks / 2 : blocks, stream, wide)));
+      FF_TRY(launch_mx_tile(1, p, blocks, stream));
     }
     if (shared) {
       const int smf = R > 32 ? 4 : R > 16 ? 2 : 1;
@@ -825,7 +828,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
         q.w0_codes = shared->slot[0]; q.w0_scales = shared->slot[1]; q.w1_codes = shared->slot[2]; q.w1_scales = shared->slot[3];
         q.total_units = sgroups * uint32_t((SI + 127) / 128);
         q.out = (uint16_t*)(s + l.sh_act); q.K = H; q.N = SI;
-        FF_TRY((launch_mx<0, 0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream)));
+        FF_TRY(launch_mx_dense<0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
       if (stages & 4) FF_TRY(ffmoe_act_quant_e8m0(s + l.sh_act, s + l.sh_aq, s + l.sh_sa, R, SI, stream_));
       if (stages & 8) {
@@ -833,7 +836,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
         q.w0_codes = shared->slot[4]; q.w0_scales = shared->slot[5]; q.w1_codes = 0; q.w1_scales = 0;
         q.total_units = sgroups * uint32_t((H + 255) / 256);
         q.out = (uint16_t*)args->shared_out; q.K = SI; q.N = H;
-        FF_TRY((launch_mx<2, 0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream)));
+        FF_TRY(launch_mx_dense<2>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
     }
     return 0;
@@ -853,13 +856,15 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
       p.a = (const uint16_t*)args->x; p.units = b.units0; p.unit_total = b.totals + 0;
       p.out = (uint16_t*)(s + l.act); p.K = H; p.N = I;
       p.a_sh = (const uint16_t*)args->x; p.out_sh = (uint16_t*)(s + l.sh_act);
-      FF_TRY(launch_w16_fmt<0>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
+      if (nv_tile) FF_TRY(launch_nvfp4_tile(0, p, blocks / 2 * 3, stream));
+      else FF_TRY(launch_w16_fmt<0>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
     }
     if (stages & 8) {
       p.a = (const uint16_t*)(s + l.act); p.units = b.units1; p.unit_total = b.totals + 1;
       p.out = (uint16_t*)args->contributions; p.done = args->done; p.weights = args->weights; p.K = I; p.N = H;
       p.a_sh = (const uint16_t*)(s + l.sh_act); p.out_sh = (uint16_t*)args->shared_out;
-      FF_TRY(launch_w16_fmt<1>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
+      if (nv_tile) FF_TRY(launch_nvfp4_tile(1, p, blocks / 2 * 3, stream));
+      else FF_TRY(launch_w16_fmt<1>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
     }
     if (shared && !ride)
       FF_TRY(shared_expert_w16(shared, args->x, R, H, args->swiglu, args->swiglu_limit, s + l.sh_act, args->shared_out,

@@ -1,6 +1,7 @@
-// Launches of the kernels whose operand tiles go straight to LDS (tile_gemm.cuh, mx_tile.cuh)
+// Launches of the kernels whose operand tiles go straight to LDS (tile_gemm.cuh, mx_tile.cuh, nvfp4_tile.cuh)
 #include "tile_gemm.cuh"
 #include "mx_tile.cuh"
+#include "nvfp4_tile.cuh"
 #include "tiles.h"
 #include "api.h"
 
@@ -21,6 +22,17 @@ static int launch_mx(const MxParams& p, unsigned blocks, hipStream_t stream) {
 }
 int launch_mx_tile(int mode, const MxParams& p, unsigned blocks, hipStream_t stream) {
   return mode == 0 ? launch_mx<0>(p, blocks, stream) : launch_mx<1>(p, blocks, stream);
+}
+
+template <int MODE>
+static int launch_nvfp4(const W16Params& p, unsigned blocks, hipStream_t stream) {
+  static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_nvfp4_tile<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, NV_TILE_LDS);
+  if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", NV_TILE_LDS, hipGetErrorString(ok));
+  hipLaunchKernelGGL(k_nvfp4_tile<MODE>, dim3(blocks), dim3(256), NV_TILE_LDS, stream, p);
+  return ff_launch_status();
+}
+int launch_nvfp4_tile(int mode, const W16Params& p, unsigned blocks, hipStream_t stream) {
+  return mode == 0 ? launch_nvfp4<0>(p, blocks, stream) : launch_nvfp4<1>(p, blocks, stream);
 }
 
 }  // namespace ffmoe

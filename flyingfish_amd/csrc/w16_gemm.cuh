@@ -229,8 +229,9 @@ __device__ __forceinline__ W16Unit w16_unit(const W16Params& p, uint32_t u, int 
 
 // Epilogue of the grouped W*A16 kernels: a lane holds token (lane % 16) of each row fragment and output columns
 // 4 (lane / 16) .. + 3 of each weight fragment.
-template <int MF, int MODE>
-__device__ __forceinline__ void w16_store(const v4f (&acc)[MF][4], const W16Params& p, bool ride, int start, int n, int t, const int (&col0)[4], int wave,
+// NF: weight fragments of the wave (MODE 0: NF / 2 of gate rows, then the up rows of the same columns).
+template <int MF, int MODE, int NF = 4>
+__device__ __forceinline__ void w16_store(const v4f (&acc)[MF][NF], const W16Params& p, bool ride, int start, int n, int t, const int (&col0)[NF], int wave,
                                           int lane) {
   const int N = p.N;
   const int tk = lane & 15, sub = (lane >> 4) * 4;
@@ -241,14 +242,14 @@ __device__ __forceinline__ void w16_store(const v4f (&acc)[MF][4], const W16Para
       const int pos = start + token;
       if (MODE == 0) {
 #pragma unroll
-        for (int f = 0; f < 2; ++f) {
+        for (int f = 0; f < NF / 2; ++f) {
           const int col = col0[f] + sub;
           if (col0[f] + 16 <= N) {
             uint32_t o[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              const uint32_t lo = swiglu_bf16(bround(acc[m][f][2 * h]), bround(acc[m][f + 2][2 * h]), p.swiglu, p.limit);
-              const uint32_t hi = swiglu_bf16(bround(acc[m][f][2 * h + 1]), bround(acc[m][f + 2][2 * h + 1]), p.swiglu, p.limit);
+              const uint32_t lo = swiglu_bf16(bround(acc[m][f][2 * h]), bround(acc[m][f + NF / 2][2 * h]), p.swiglu, p.limit);
+              const uint32_t hi = swiglu_bf16(bround(acc[m][f][2 * h + 1]), bround(acc[m][f + NF / 2][2 * h + 1]), p.swiglu, p.limit);
               o[h] = lo | (hi << 16);
             }
             const u32x2 v = {o[0], o[1]};
@@ -263,7 +264,7 @@ __device__ __forceinline__ void w16_store(const v4f (&acc)[MF][4], const W16Para
           rw = p.weights_f32 ? load_global<float>(reinterpret_cast<const float*>(p.weights) + a)
                              : bf16_to_f32(load_global<uint16_t>(reinterpret_cast<const uint16_t*>(p.weights) + a));
 #pragma unroll
-        for (int f = 0; f < 4; ++f) {
+        for (int f = 0; f < NF; ++f) {
           const int col = col0[f] + sub;
           if (col0[f] + 16 <= N) {
             float v[4];

@@ -619,6 +619,32 @@ def test_prefill_line_kernels_equal_the_k_block_kernel_bitwise(fmt, switch, rows
         assert np.array_equal(a, b), what
 
 
+@pytest.mark.parametrize("rows,mf,hidden,inter", [(3, None, 256, 256), (70, None, 512, 768), (70, "1", 256, 1280), (150, "2", 1024, 256), (400, None, 768, 512)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_prefill_nvfp4_tile_kernel_equals_the_line_kernel_bitwise(rows, mf, hidden, inter, shared, monkeypatch):
+    """One to twenty K stages, groups of one to 64 rows (skewed routing), a tile's columns past the end, the riding shared expert."""
+    table, _ = make_table(capi.FMT_NVFP4, 6, hidden, inter, 500 + rows)
+    sh = table.shared_struct(5) if shared else None
+    table.experts = 5
+    gen = torch.Generator().manual_seed(rows)
+    ids = torch.stack([torch.multinomial(torch.tensor([0.55, 0.3, 0.1, 0.04, 0.01]), 2, generator=gen) for _ in range(rows)]).to(torch.int32).cuda()
+    x = synth.normal((rows, hidden), 1.0, 501 + rows).to(torch.bfloat16).cuda()
+    w = torch.rand((rows, 2), generator=gen).cuda()
+    if mf:
+        monkeypatch.setenv("FFMOE_PREFILL_MF", mf)
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_NVFP4_TILE", switch)
+        op = ops.PrefillOps(table, rows, 2, shared=sh, act_mode=capi.ACT_BF16)
+        op.contribute(x, ids, w)
+        torch.cuda.synchronize()
+        out.append((op.contributions.clone(), op.done.clone(), op.shared_out.clone() if shared else None))
+    assert torch.equal(out[0][0].view(torch.int16), out[1][0].view(torch.int16))
+    assert torch.equal(out[0][1], out[1][1]) and int(out[1][1].min()) == 1
+    if shared:
+        assert torch.equal(out[0][2].view(torch.int16), out[1][2].view(torch.int16))
+
+
 @pytest.mark.parametrize("rows", [8, 16, 64, 65])
 @pytest.mark.parametrize("shared_inter", [256, 512])
 def test_decode_nvfp4_cohort_with_a_bf16_shared_expert(rows, shared_inter, monkeypatch):
