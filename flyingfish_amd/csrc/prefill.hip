@@ -488,9 +488,18 @@ bool use_tiles(int mode, int rows, int n) {
   if (const char* f = getenv("FFMOE_W8A8_TILE")) return atoi(f) != 0;
   return rows > 64 && 4ll * tile_units(mode, rows, n) >= 3ll * num_cus_p();
 }
-int launch_tiles(int mode, GemmParams& p, hipStream_t stream) {
+int launch_tiles(int mode, GemmParams& p, hipStream_t stream, bool mx = false) {
   p.total_units = tile_units(mode, p.rows_total, p.N);
-  return launch_w8a8_tile(mode, p, std::min<unsigned>((p.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
+  const unsigned blocks = std::min<unsigned>((p.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u);
+  return mx ? launch_mx_dense_tile(mode, p, blocks, stream) : launch_w8a8_tile(mode, p, blocks, stream);
+}
+// the E4M3 / E8M0 dense call as the tile kernel takes it
+int launch_tiles(int mode, const MxParams& q, hipStream_t stream) {
+  GemmParams p{};
+  p.a_codes = q.a_codes; p.a_scales = (const float*)q.a_scales;
+  p.w0_codes = q.w0_codes; p.w0_scales = q.w0_scales; p.w1_codes = q.w1_codes; p.w1_scales = q.w1_scales;
+  p.out = q.out; p.rows_total = q.rows_total; p.K = q.K; p.N = q.N; p.top_k = 1; p.limit = q.limit;
+  return launch_tiles(mode, p, stream, true);
 }
 
 template <int MODE>
@@ -823,12 +832,15 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
       const uint32_t sgroups = uint32_t((R + stm - 1) / stm);
       MxParams q{};
       q.rows_total = R; q.top_k = 1; q.limit = args->swiglu_limit;
+      // the tile kernel reads four scale bytes of a row block as one word; the slots only promise bytes
+      const bool mx_words = shared->slot[1] % 4 == 0 && shared->slot[3] % 4 == 0 && shared->slot[5] % 4 == 0;
       if (stages & 2) {
         q.a_codes = s + l.xq; q.a_scales = s + l.sx;
         q.w0_codes = shared->slot[0]; q.w0_scales = shared->slot[1]; q.w1_codes = shared->slot[2]; q.w1_scales = shared->slot[3];
         q.total_units = sgroups * uint32_t((SI + 127) / 128);
         q.out = (uint16_t*)(s + l.sh_act); q.K = H; q.N = SI;
-        FF_TRY(launch_mx_dense<0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
+        if (mx_words && use_tiles(0, R, SI)) FF_TRY(launch_tiles(0, q, stream));
+        else FF_TRY(launch_mx_dense<0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
       if (stages & 4) FF_TRY(ffmoe_act_quant_e8m0(s + l.sh_act, s + l.sh_aq, s + l.sh_sa, R, SI, stream_));
       if (stages & 8) {
@@ -836,7 +848,8 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
         q.w0_codes = shared->slot[4]; q.w0_scales = shared->slot[5]; q.w1_codes = 0; q.w1_scales = 0;
         q.total_units = sgroups * uint32_t((H + 255) / 256);
         q.out = (uint16_t*)args->shared_out; q.K = SI; q.N = H;
-        FF_TRY(launch_mx_dense<2>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
+        if (mx_words && use_tiles(2, R, H)) FF_TRY(launch_tiles(2, q, stream));
+        else FF_TRY(launch_mx_dense<2>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
     }
     return 0;

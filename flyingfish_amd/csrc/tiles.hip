@@ -8,8 +8,13 @@
 namespace ffmoe {
 
 int launch_w8a8_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
-  if (mode == 0) hipLaunchKernelGGL(k_w8a8_tile<0>, dim3(blocks), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL(k_w8a8_tile<2>, dim3(blocks), dim3(256), 0, stream, p);
+  if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, false>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((k_w8a8_tile<2, false>), dim3(blocks), dim3(256), 0, stream, p);
+  return ff_launch_status();
+}
+int launch_mx_dense_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
+  if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, true>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((k_w8a8_tile<2, true>), dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
 }
 

@@ -170,6 +170,23 @@ def test_e8m0_prefill_on_the_mx_matrix_cores(rows, top_k, experts, hidden, inter
     assert_close_bf16(so, want_sd, "shared down projection of the device activations")
 
 
+@pytest.mark.parametrize("rows,hidden,shared_inter", [(3, 128, 128), (65, 384, 256), (200, 256, 384), (300, 1280, 128)])
+def test_e8m0_shared_expert_tile_kernel_equals_the_row_group_kernel_bitwise(rows, hidden, shared_inter, monkeypatch):
+    routed, _, sh_table, _ = _tables(2, hidden, 128, shared_inter, 700 + rows)
+    x = rand_bf16((rows, hidden), 1.0, 710 + rows).to(DEV)
+    ids = torch.zeros((rows, 1), dtype=torch.int32, device=DEV)
+    wt = torch.ones((rows, 1), device=DEV)
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_TILE", switch)
+        op = PrefillOps(routed, rows, 1, swiglu=capi.SWIGLU_CLAMPED_ONCE, swiglu_limit=7.0, routed_weight=capi.WEIGHT_BEFORE_DOWN_F32, weights_f32=True,
+                        shared=sh_table.shared_struct(0), act_mode=capi.ACT_E4M3_E8M0_32)
+        op.contribute(x, ids, wt)
+        torch.cuda.synchronize()
+        out.append(op.shared_out.clone())
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("rows,hidden,inter", [(16, 128, 384), (33, 1280, 128), (65, 384, 640), (150, 768, 256)])
 def test_e8m0_prefill_rows_do_not_depend_on_their_group_bitwise(rows, hidden, inter):
     """Groups of one to 64 rows, contractions of one to five stages with and without a last half, columns past the end of a
