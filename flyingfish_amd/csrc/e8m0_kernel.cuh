@@ -789,10 +789,13 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
     if (is_shared) {
       exact = lo == 4096 || ms < pow2_f64(53 + lo - 18);  // units of 2^-18 below the smallest group's exponent
     } else {
-      // |group sum| < 2^27 units, G of them; the FP32 results stay away from both ends of the exponent range
+      // |group sum| < 2^27 units of 2^(scale codes - 264), G of them. The FP32 results stay away from both ends of the exponent
+      // range: 27 + 364 - 264 = 127 keeps a group's sum finite, 140 - 264 = -124 keeps its unit normal. A total that is not
+      // finite all the same holds a scale code of 255, which the contract reserves, over a group of zeros.
       const int xlo = range[2 * t], xhi = range[2 * t + 1];
       const int span = (xhi + hi) - (xlo + lo);
-      exact = lo > hi || xlo > xhi || (span + 27 + (32 - __builtin_clz(G)) <= 53 && xlo + lo >= 140 && xhi + hi <= 370 && hi <= 254);
+      exact = lo > hi || xlo > xhi || (span + 27 + (32 - __builtin_clz(G)) <= 53 && xlo + lo >= 140 && xhi + hi <= 364 && hi <= 254);
+      exact = exact && fabs(v) < __builtin_inf();
     }
     if (!exact) {
       const uint8_t* wrow = reinterpret_cast<const uint8_t*>(sl[2 * m]) + size_t(j) * (is_shared ? K : K >> 1);

@@ -314,3 +314,80 @@ def test_e8m0_matrix_core_tiles_bit_exact_on_any_code(hidden, inter, shared_inte
             assert np.array_equal(got[r, c], orc.expert_ffn_e8m0(1, xb[r], *ref[int(ids[r, c])], limit, float(wt[r, c]))), (r, c)
         assert np.array_equal(got_sh[r], orc.expert_ffn_e8m0(0, xb[r], *sh_ref, limit, 1.0)), r
     assert np.all(op.done.cpu().numpy() == 1)
+
+
+def _single_expert(hidden, inter, codes, scales):
+    """A table of one routed expert with these six tensors, gate codes, gate scales, up .., down .."""
+    routed = ExpertTable.allocate(capi.FMT_E2M1_E8M0, 1, hidden, inter, DEV)
+    for v, a in zip(routed.expert_views(0), [t for pair in zip(codes, scales) for t in pair]):
+        v.copy_(torch.from_numpy(a))
+    return routed
+
+
+def _pack(nibbles):
+    """[.., K] E2M1 nibbles to [.., K / 2] codes, low nibble first."""
+    return (nibbles[..., 0::2] | (nibbles[..., 1::2] << 4)).astype(np.uint8)
+
+
+def _one_choice(routed, x, weight=1.0, shared=None):
+    rows = x.shape[0]
+    op = E8m0DecodeOps(routed, shared, rows, 1, 7.0)
+    ids = torch.zeros((rows, 1), dtype=torch.int32, device=DEV)
+    contrib, shared_out = op.contribute(x.to(DEV), ids, torch.full((rows, 1), weight, device=DEV))
+    torch.cuda.synchronize()
+    return bits(contrib)[:, 0], None if shared is None else bits(shared_out)
+
+
+def _identity_down(n):
+    """Down projection that hands the (quantized) activations through: 1.0 on the diagonal."""
+    return _pack(2 * np.eye(n, dtype=np.uint8)), np.full((n, n // 32), 127, dtype=np.uint8)
+
+
+def test_e8m0_group_sums_at_the_ends_of_the_fp32_range():
+    """Two groups of 32 x 448 x 6.0 x 2^(code sum - 254) that cancel, or nearly do: from a code sum of 366 on one alone is
+    beyond FP32, while the contract's FP64 total is 0 or an ordinary multiple. Row j has weight scale 358 - 239 + j / 4 on a
+    token whose scale codes are 239; every second pair of rows leaves one product standing. Below, small sums: FP32 results
+    around the smallest normal number, which a large routing weight brings back to the output."""
+    n = 128
+    for xexp, first, weight in ((112, 119, 1.0), (-14, 0, 2.0 ** 120)):  # token codes 239 and 113; sums 358 .. 389 and 113 .. 144
+        x = np.zeros((3, n), dtype=np.float32)
+        x[:, :32] = 448.0
+        x[:, 32:64] = -448.0
+        xb = torch.from_numpy(x * np.float32(2.0 ** xexp)).to(torch.bfloat16)
+        up = np.zeros((n, n), dtype=np.uint8)
+        up[:, :64] = 7  # 6.0
+        up[2::4, 5] = 6   # one product of the pair stands: negative
+        up[3::4, 40] = 6  # positive
+        gate = np.zeros((n, n), dtype=np.uint8)
+        gate[:, :32] = 7
+        sup = np.repeat((first + np.arange(n) // 4).astype(np.uint8)[:, None], n // 32, 1)
+        sgate = np.full((n, n // 32), 127, dtype=np.uint8)
+        down, sdown = _identity_down(n)
+        m = [_pack(gate), sgate, _pack(up), sup, down, sdown]
+        got, _ = _one_choice(_single_expert(n, n, m[0::2], m[1::2]), xb, weight)
+        for r in range(3):
+            want = orc.expert_ffn_e8m0(1, bits(xb)[r], *m, 7.0, weight)
+            assert np.array_equal(got[r], want), (xexp, r, np.flatnonzero(got[r] != want))
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("code", [253, 254, 255])
+def test_e8m0_all_zero_group_adds_nothing_whatever_its_scale(code, rows):
+    """A weight group of zeros (of both signs) under the largest scales, and under the reserved code, on ordinary and on huge
+    activations: the result is that of any other scale."""
+    n = 128
+    rng = np.random.default_rng(code + rows)
+    _, ref, _, _ = _tables(1, n, n, n, 600)
+    m = [a.copy() for a in ref[0]]
+    for i in range(3):
+        m[2 * i][:, 16:32] = rng.choice(np.array([0x00, 0x08, 0x80, 0x88], dtype=np.uint8), (n, 16))
+        m[2 * i + 1][:, 1] = 100
+    x = rand_bf16((rows, n), 1.0, 601)
+    x[1:, 32:64] *= 2.0 ** 119
+    plain, _ = _one_choice(_single_expert(n, n, m[0::2], m[1::2]), x)
+    for r in range(rows):
+        assert np.array_equal(plain[r], orc.expert_ffn_e8m0(1, bits(x)[r], *m, 7.0, 1.0))
+    for i in range(3):
+        m[2 * i + 1][:, 1] = code
+    got, _ = _one_choice(_single_expert(n, n, m[0::2], m[1::2]), x)
+    assert np.array_equal(got, plain)
