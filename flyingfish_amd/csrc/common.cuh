@@ -14,6 +14,16 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int WAVE = 64;
 
+// Grids of more blocks than one dimension of a launch holds (fewer than 2^32 threads; the excess is dropped without an error):
+// blocks are numbered by flat_block(), rows of FLAT_ROW of them where they have to. The last row may run past the count asked for.
+constexpr uint32_t FLAT_ROW = 1u << 20;
+constexpr long long FLAT_BLOCKS_MAX = (1ll << 32) - FLAT_ROW;
+inline dim3 flat_grid(long long blocks, int threads) {
+  if (blocks * threads < (1ll << 32)) return dim3(unsigned(blocks));
+  return dim3(FLAT_ROW, unsigned((blocks + FLAT_ROW - 1) / FLAT_ROW));
+}
+__device__ __forceinline__ uint32_t flat_block() { return blockIdx.y * FLAT_ROW + blockIdx.x; }
+
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 __device__ __forceinline__ float bf16lo(uint32_t pair) { return __uint_as_float(pair << 16); }
 __device__ __forceinline__ float bf16hi(uint32_t pair) { return __uint_as_float(pair & 0xffff0000u); }

@@ -114,16 +114,17 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_decode_contribute_e8
     }
     const long long gs = shared ? (R + tokens - 1) / tokens : 0, gr = groups - gs;
     const long long b0 = gs * (SI / 16) + gr * (I / 32), b1 = gs * (H / 32) + gr * ((H + 127) / 128);
-    FF_REQUIRE(b0 < (1ll << 31) && b1 < (1ll << 31), FFMOE_ERR_SHAPE, "rows=%d top_k=%d exceed the launch grid", R, K);
+    FF_REQUIRE(b0 <= FLAT_BLOCKS_MAX && b1 <= FLAT_BLOCKS_MAX, FFMOE_ERR_SHAPE, "rows=%d top_k=%d exceed the launch grid", R, K);
+    const dim3 g0 = flat_grid(b0, FFMOE_E8M0_NT), g1 = flat_grid(b1, FFMOE_E8M0_NT);
     const size_t l0 = e8m0_tiles_lds(0, H, tokens), l1 = e8m0_tiles_lds(1, imax, tokens);
     if (R > 1) {
       hipLaunchKernelGGL(k_act_quant_e8m0, dim3((H / 32 + 63) / 64, R), dim3(256), 0, st, p.x, H, sc + l.xq, H, sc + l.xs, H / 32, H, (const uint32_t*)nullptr);
-      hipLaunchKernelGGL((k_e8m0_tiles<0, true>), dim3((unsigned)b0), dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
+      hipLaunchKernelGGL((k_e8m0_tiles<0, true>), g0, dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
     } else {
-      hipLaunchKernelGGL((k_e8m0_tiles<0, false>), dim3((unsigned)b0), dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
+      hipLaunchKernelGGL((k_e8m0_tiles<0, false>), g0, dim3(FFMOE_E8M0_NT), l0, st, q, tokens);
     }
     FF_TRY(ff_launch_status());
-    hipLaunchKernelGGL((k_e8m0_tiles<1, false>), dim3((unsigned)b1), dim3(FFMOE_E8M0_NT), l1, st, q, tokens);
+    hipLaunchKernelGGL((k_e8m0_tiles<1, false>), g1, dim3(FFMOE_E8M0_NT), l1, st, q, tokens);
     return ff_launch_status();
   }
   hipLaunchKernelGGL(k_act_quant_e8m0, dim3((H / 32 + 63) / 64, R), dim3(256), 0, st, p.x, H, sc + l.xq, H, sc + l.xs, H / 32, H, (const uint32_t*)nullptr);

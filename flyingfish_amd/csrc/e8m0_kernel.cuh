@@ -493,7 +493,7 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
   const int n_shared = p.groups ? load_uniform<int>(p.counters + 1) : (p.has_shared ? p.rows : 0);
   int group, tile;
   {
-    const uint32_t b = blockIdx.x, bs = uint32_t(n_shared) * uint32_t(tiles_s);
+    const uint32_t b = flat_block(), bs = uint32_t(n_shared) * uint32_t(tiles_s);
     if (b < bs) {
       group = int(b / uint32_t(tiles_s));
       tile = int(b) - group * tiles_s;

@@ -391,3 +391,24 @@ def test_e8m0_all_zero_group_adds_nothing_whatever_its_scale(code, rows):
         m[2 * i + 1][:, 1] = code
     got, _ = _one_choice(_single_expert(n, n, m[0::2], m[1::2]), x)
     assert np.array_equal(got, plain)
+
+
+def test_e8m0_call_larger_than_one_grid_dimension_bitwise():
+    """65535 rows, the most the entry takes, whose blocks hold more threads than one dimension of a launch counts: equal to the
+    same rows in four calls."""
+    hidden, inter, rows, top_k = 128, 512, 65535, 8
+    routed, _, sh_table, _ = _tables(16, hidden, inter, inter, 660)
+    sh = sh_table.shared_struct(0)
+    x = synth.normal((rows, hidden), 1.0, 661, device=DEV).to(torch.bfloat16)
+    ids = torch.stack([torch.arange(rows, device=DEV) % 9 + c for c in range(top_k)], 1).to(torch.int32)
+    wt = torch.linspace(0.05, 0.5, rows * top_k, device=DEV).view(rows, top_k)
+    op = E8m0DecodeOps(routed, sh, rows, top_k, 7.0)
+    contrib, shared_out = op.contribute(x, ids, wt)
+    part = 16384
+    for r0 in range(0, rows, part):
+        n = min(part, rows - r0)
+        few = E8m0DecodeOps(routed, sh, n, top_k, 7.0)
+        c, s = few.contribute(x[r0:r0 + n].contiguous(), ids[r0:r0 + n].contiguous(), wt[r0:r0 + n].contiguous())
+        assert torch.equal(c.view(torch.int16), contrib[r0:r0 + n].view(torch.int16)), r0
+        assert torch.equal(s.view(torch.int16), shared_out[r0:r0 + n].view(torch.int16)), r0
+    assert int(op.done.min()) == 1
