@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256) void k_decode_form_rows(const DecodeParams p) 
   const int n_shared = p.groups ? load_uniform<int>(p.counters + 1) : (p.has_shared ? p.rows : 0);
   int group, tile;
   {
-    const uint32_t b = blockIdx.x, bs = uint32_t(n_shared) * uint32_t(tiles_s);
+    const uint32_t b = flat_block(), bs = uint32_t(n_shared) * uint32_t(tiles_s);
     if (b < bs) {
       group = int(b / uint32_t(tiles_s));
       tile = int(b) - group * tiles_s;
@@ -586,14 +586,14 @@ bool form_rows_fit(const DecodeParams& p) {
 template <class F, int FORM, int T>
 int launch_form_rows(const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st) {
   const long long b0 = routed * ((p.inter + 63) / 64) + shared * ((p.shared_inter + 63) / 64), b1 = (routed + shared) * ((p.hidden + 127) / 128);
-  if (b0 >= (1ll << 31) || b1 >= (1ll << 31)) return ff_fail(FFMOE_ERR_SHAPE, "%lld groups exceed the launch grid", routed + shared);
+  if (b0 > FLAT_BLOCKS_MAX || b1 > FLAT_BLOCKS_MAX) return ff_fail(FFMOE_ERR_SHAPE, "%lld groups exceed the launch grid", routed + shared);
   constexpr size_t lds = 4 * FFMOE_FORM_WAVE_LDS + size_t(T) * FFMOE_FORM_SEG * 2;
   if (stage_mask & 1) {
-    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 0, T>), dim3((unsigned)b0), dim3(256), lds, st, p);
+    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 0, T>), flat_grid(b0, 256), dim3(256), lds, st, p);
     FF_TRY(ff_launch_status());
   }
   if (stage_mask & 2) {
-    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 1, T>), dim3((unsigned)b1), dim3(256), lds, st, p);
+    hipLaunchKernelGGL((k_decode_form_rows<F, FORM, 1, T>), flat_grid(b1, 256), dim3(256), lds, st, p);
     FF_TRY(ff_launch_status());
   }
   return 0;

@@ -207,3 +207,24 @@ def test_streamed_form_kernels_bit_exact(fmt, form, hidden, inter, rows, monkeyp
         assert np.array_equal(bits(contrib)[:, 0], want), grouped
         assert np.array_equal(bits(shared_out), want_sh), grouped
         assert np.all(op.done.cpu().numpy() == 1)
+
+
+def test_form_call_larger_than_one_grid_dimension_bitwise():
+    """65535 rows, whose blocks hold more threads than one dimension of a launch counts: equal to the same rows in four calls."""
+    hidden, inter, rows, top_k, experts = 64, 2048, 65535, 8, 16
+    table, _ = make_table(capi.FMT_BF16, experts + 1, hidden, inter, 7000)
+    sh = table.shared_struct(experts)
+    table.experts = experts
+    x = synth.normal((rows, hidden), 1.0, 7001, device=DEV).to(torch.bfloat16)
+    ids = torch.stack([torch.arange(rows, device=DEV) % 9 + c for c in range(top_k)], 1).to(torch.int32)
+    wt = torch.linspace(0.05, 0.5, rows * top_k, device=DEV).view(rows, top_k)
+    op = DecodeOps(table, sh, rows, top_k, weights_f32=True)
+    contrib, shared_out = op.contribute(x, ids, wt, form=capi.FORM_LANE16)
+    part = 16384
+    for r0 in range(0, rows, part):
+        n = min(part, rows - r0)
+        few = DecodeOps(table, sh, n, top_k, weights_f32=True)
+        c, s = few.contribute(x[r0:r0 + n].contiguous(), ids[r0:r0 + n].contiguous(), wt[r0:r0 + n].contiguous(), form=capi.FORM_LANE16)
+        assert torch.equal(c.view(torch.int16), contrib[r0:r0 + n].view(torch.int16)), r0
+        assert torch.equal(s.view(torch.int16), shared_out[r0:r0 + n].view(torch.int16)), r0
+    assert int(op.done.min()) == 1
