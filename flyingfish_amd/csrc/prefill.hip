@@ -776,6 +776,8 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   // cohorts): on its own it is a few dozen blocks per launch, which at small cohorts take longer than the routed experts'
   // thousands. FFMOE_PREFILL_SHARED_RIDE=0 keeps it in launches of its own (the results are the same bits either way).
   bool ride = a16 && shared && shared->format == table->format && SI == I;
+  // the NVFP4 tile kernel moves a row's 16 scale bytes straight to LDS in one piece; the shared slots only promise words
+  if (nv_tile && ride) ride = (shared->slot[1] | shared->slot[3] | shared->slot[5]) % 16 == 0;
   if (const char* f = getenv("FFMOE_PREFILL_SHARED_RIDE")) ride = ride && atoi(f) != 0;
 
   if (stages & 1) {

@@ -645,6 +645,34 @@ def test_prefill_nvfp4_tile_kernel_equals_the_line_kernel_bitwise(rows, mf, hidd
         assert torch.equal(out[0][2].view(torch.int16), out[1][2].view(torch.int16))
 
 
+def test_prefill_nvfp4_shared_expert_with_word_aligned_scales_bitwise(monkeypatch):
+    """A shared NVFP4 expert whose scale bytes start at any multiple of four, next to routed experts on the tile kernel."""
+    rows, hidden, inter = 70, 512, 256
+    monkeypatch.setenv("FFMOE_NVFP4_TILE", "1")
+    table, _ = make_table(capi.FMT_NVFP4, 6, hidden, inter, 520)
+    views = table.expert_views(5)
+    table.experts = 5
+    ids, w = _routing(rows, 2, 5, 521, 1.2)
+    x = synth.normal((rows, hidden), 1.0, 522).to(torch.bfloat16).cuda()
+    out = []
+    for shift in (0, 4, 8, 12):
+        sh = table.shared_struct(5)
+        copies = []
+        for i in (1, 3, 5):
+            n = views[i].numel()
+            copies.append(torch.empty(n + 16, dtype=torch.uint8, device="cuda"))
+            copies[-1][shift:shift + n].copy_(views[i].reshape(-1).view(torch.uint8))
+            assert copies[-1].data_ptr() % 16 == 0
+            sh.slot[i] = copies[-1].data_ptr() + shift
+        op = ops.PrefillOps(table, rows, 2, shared=sh, act_mode=capi.ACT_BF16)
+        op.contribute(x, torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda())
+        torch.cuda.synchronize()
+        out.append((bits(op.contributions), bits(op.shared_out)))
+    assert out[0][1].any()
+    for o in out[1:]:
+        assert np.array_equal(o[0], out[0][0]) and np.array_equal(o[1], out[0][1])
+
+
 @pytest.mark.parametrize("rows", [8, 16, 64, 65])
 @pytest.mark.parametrize("shared_inter", [256, 512])
 def test_decode_nvfp4_cohort_with_a_bf16_shared_expert(rows, shared_inter, monkeypatch):
