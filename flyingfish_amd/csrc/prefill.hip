@@ -871,14 +871,14 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
       p.a = (const uint16_t*)args->x; p.units = b.units0; p.unit_total = b.totals + 0;
       p.out = (uint16_t*)(s + l.act); p.K = H; p.N = I;
       p.a_sh = (const uint16_t*)args->x; p.out_sh = (uint16_t*)(s + l.sh_act);
-      if (nv_tile) FF_TRY(launch_nvfp4_tile(0, p, blocks / 2 * 3, stream));
+      if (nv_tile) FF_TRY(launch_nvfp4_tile(0, p, (blocks * 3 / 2 + 7u) & ~7u, stream));
       else FF_TRY(launch_w16_fmt<0>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
     }
     if (stages & 8) {
       p.a = (const uint16_t*)(s + l.act); p.units = b.units1; p.unit_total = b.totals + 1;
       p.out = (uint16_t*)args->contributions; p.done = args->done; p.weights = args->weights; p.K = I; p.N = H;
       p.a_sh = (const uint16_t*)(s + l.sh_act); p.out_sh = (uint16_t*)args->shared_out;
-      if (nv_tile) FF_TRY(launch_nvfp4_tile(1, p, blocks / 2 * 3, stream));
+      if (nv_tile) FF_TRY(launch_nvfp4_tile(1, p, (blocks * 3 / 2 + 7u) & ~7u, stream));
       else FF_TRY(launch_w16_fmt<1>(table->format, p, mf, wide ? blocks / 2 : blocks, stream, wide));
     }
     if (shared && !ride)
