@@ -79,6 +79,8 @@ __global__ __launch_bounds__(256, 2) void k_mx_tile(const MxParams p) {
     const uint8_t* wssrc = reinterpret_cast<const uint8_t*>(d.ws[0]);
     if (MODE == 0 && lane >= 32) wssrc = reinterpret_cast<const uint8_t*>(d.ws[1]);
     wssrc += size_t(min(column(lane >> 5), N - 16) + ((lane >> 1) & 15)) * SB + sdword * 4;
+    // the slots promise no alignment of scale bytes, a direct load of a word needs it: other addresses go through registers
+    const bool words = ((d.ws[0] | d.ws[1]) & 3u) == 0;
     auto token_row = [&](int m) {
       const int pos = d.start + min(m, d.n - 1);
       return MODE == 0 ? load_global<int>(p.perm + pos) / p.top_k : pos;
@@ -103,9 +105,16 @@ __global__ __launch_bounds__(256, 2) void k_mx_tile(const MxParams p) {
         for (int i = 0; i < MF; ++i)
           lds_load16(base + offsetof(MxStage<MF>, t) + uint32_t(i) * 4096u + uint32_t(wave) * 1024u, tsrc[i] + uint32_t(ks) * 256u - (half ? tback : 0));
         const int soff = ks * 8 - (half ? sdword * 4 : 0);  // signed: back to the row's first word where the only stage is a half
-        lds_load4(base + offsetof(MxStage<MF>, ws) + uint32_t(wave) * 256u, wssrc + soff);
 #pragma unroll
         for (int i = 0; i < SW; ++i) lds_load4(base + offsetof(MxStage<MF>, ts) + uint32_t(wave) * (SW * 256u) + i * 256u, tssrc[i] + soff);
+        if (words) {
+          lds_load4(base + offsetof(MxStage<MF>, ws) + uint32_t(wave) * 256u, wssrc + soff);
+        } else {  // one request fewer in flight: stage() then waits for all of them
+          uint32_t v = 0;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v |= uint32_t(load_global<uint8_t>(wssrc + soff + i)) << (8 * i);
+          reinterpret_cast<MxStage<MF>*>(lds + b * sizeof(MxStage<MF>))->ws[wave][lane] = v;
+        }
       };
       v4f acc[MF][2];
 #pragma unroll
@@ -116,7 +125,7 @@ __global__ __launch_bounds__(256, 2) void k_mx_tile(const MxParams p) {
       for (int b = 0; b < NS - 1; ++b)
         if (b < KS) request(b, b);
       auto stage = [&](int ks, int b) {
-        if (ks + NS - 1 <= KS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * LPS) : "memory");
+        if (words && ks + NS - 1 <= KS) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * LPS) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the stage is there for every wave, the buffer before it is free
         if (ks + NS - 1 < KS) request(ks + NS - 1, (b + NS - 1) % NS);

@@ -412,3 +412,30 @@ def test_e8m0_call_larger_than_one_grid_dimension_bitwise():
         assert torch.equal(c.view(torch.int16), contrib[r0:r0 + n].view(torch.int16)), r0
         assert torch.equal(s.view(torch.int16), shared_out[r0:r0 + n].view(torch.int16)), r0
     assert int(op.done.min()) == 1
+
+
+@pytest.mark.parametrize("rows,hidden,inter", [(9, 384, 256), (150, 640, 128)])
+def test_e8m0_prefill_takes_scales_at_any_address_bitwise(rows, hidden, inter):
+    """Scale bytes that start anywhere: the slots of a table promise 16-byte alignment of the codes only."""
+    routed, _, sh_table, _ = _tables(3, hidden, inter, 128, 680 + rows)
+    x = rand_bf16((rows, hidden), 1.0, 681).to(DEV)
+    g = synth.generator(682)
+    ids = torch.stack([torch.multinomial(torch.tensor([0.7, 0.2, 0.1]), 2, generator=g) for _ in range(rows)]).to(torch.int32).to(DEV)
+    wt = (torch.rand((rows, 2), generator=g) * 0.5 + 0.05).to(DEV)
+    moved = [[torch.empty(v.numel() + 16, dtype=torch.uint8, device=DEV) for v in routed.expert_views(e)[1::2]] for e in range(3)]
+    out = []
+    for shift in (0, 1, 2, 3, 4):
+        slots = routed.slots.tolist()
+        for e in range(3):
+            for i, (v, m) in enumerate(zip(routed.expert_views(e)[1::2], moved[e])):
+                m[shift:shift + v.numel()].copy_(v.reshape(-1))
+                slots[e][2 * i + 1] = m.data_ptr() + shift
+        table = ExpertTable(routed.format, 3, hidden, inter, routed.storage, torch.tensor(slots, dtype=torch.int64, device=DEV), None)
+        op = PrefillOps(table, rows, 2, swiglu=capi.SWIGLU_CLAMPED_ONCE, swiglu_limit=7.0, routed_weight=capi.WEIGHT_BEFORE_DOWN_F32, weights_f32=True,
+                        act_mode=capi.ACT_E4M3_E8M0_32)
+        op.contribute(x, ids, wt)
+        torch.cuda.synchronize()
+        out.append(bits(op.contributions))
+    assert out[0].any()
+    for shift in range(1, 5):
+        assert np.array_equal(out[shift], out[0]), shift
