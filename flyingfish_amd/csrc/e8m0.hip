@@ -2,6 +2,8 @@
 // kernels are in e8m0_kernel.cuh.
 #include "e8m0_kernel.cuh"
 #include <algorithm>
+#include <cmath>
+#include <cstdlib>
 
 namespace ffmoe {
 int decode_group_assignments(const DecodeParams& p, int rgmax, hipStream_t st);
@@ -29,6 +31,23 @@ E8m0Layout e8m0_layout(int rows, int top_k, int hidden, int inter, int shared_in
   l.counters = at; at = up(at + 8);
   l.total = at;
   return l;
+}
+}  // namespace
+
+namespace {
+// Pairing costs the grouping launch (5 us, and a scan of the assignments by every expert) and saves a pass over an expert's weights
+// per pair. us one at a time / in pairs (shared expert included): 2 rows, top-6 of 64 at 512 / 256: 20 / 26, 8 rows, top-8 of 64 at
+// 2048 / 768: 68 / 69, 16 rows 118 / 106; at 4096 / 1536 3 rows 73 / 71, 16 rows 292 / 218; 32 rows, top-8 of 256 at 1024 / 512:
+// 128 / 121; 256 rows, top-6 of 64 at 1024 / 512: 670 / 624. The line was fitted to 296 such shapes (within 9 % of the better side at all of them, 0.1 % on average): expected
+// passes saved, for an even routing, x weights of an expert against the assignments every expert's threads look through.
+// FFMOE_E8M0_PAIRS: 1 wherever it can be done, 0 never; same bits.
+bool pairs_pay(int rows, int top_k, int experts, int hidden, int inter, bool shared) {
+  if (const char* f = getenv("FFMOE_E8M0_PAIRS")) return atoi(f) != 0;
+  const double p = std::min(1.0, double(top_k) / experts);
+  double odd = 1.0;  // 1 - 2 x the probability that an expert is left with a single row
+  for (int i = 0; i < rows && std::abs(odd) > 1e-3; ++i) odd *= 1.0 - 2.0 * p;
+  const double saved = experts * (rows * p - (1.0 - odd) / 2.0) / 2.0 + (shared ? rows / 2 : 0);
+  return saved * 3e-6 * hidden * inter > 30.0 + 0.9 * std::min(1000, rows * top_k) * std::min(1.0, 64.0 / experts);
 }
 }  // namespace
 
@@ -96,11 +115,12 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_decode_contribute_e8
   hipStream_t st = (hipStream_t)stream;
   const int S = R * K + R;
   // Exact arithmetic on the matrix cores wherever the contractions are whole instructions (multiples of 128 columns) and a
-  // token's exponent planes fit LDS. Several rows: the assignments of an expert share a pass over its weights in pairs.
+  // token's exponent planes fit LDS. Several rows: the assignments of an expert may share a pass over its weights in pairs.
   auto tiles_lds = [&](int tokens) { return std::max(e8m0_tiles_lds(0, H, tokens), e8m0_tiles_lds(1, imax, tokens)); };
   constexpr size_t TWO_BLOCKS = 80 * 1024, ONE_BLOCK = 160 * 1024;  // LDS per CU: 160 KB
   if (exact && H % 128 == 0 && I % 128 == 0 && SI % 128 == 0 && tiles_lds(1) <= ONE_BLOCK) {
-    const bool pairs = R > 1 && K > 0 && (long long)R * K <= FFMOE_DECODE_MAX_ASSIGN && tiles_lds(FFMOE_E8M0_TOK) <= TWO_BLOCKS;
+    const bool can_pair = R > 1 && K > 0 && (long long)R * K <= FFMOE_DECODE_MAX_ASSIGN && tiles_lds(FFMOE_E8M0_TOK) <= TWO_BLOCKS;
+    const bool pairs = can_pair && pairs_pay(R, K, E, H, I, shared != nullptr);
     const int tokens = pairs ? FFMOE_E8M0_TOK : 1;
     long long groups = S;
     if (pairs) {

@@ -439,3 +439,32 @@ def test_e8m0_prefill_takes_scales_at_any_address_bitwise(rows, hidden, inter):
     assert out[0].any()
     for shift in range(1, 5):
         assert np.array_equal(out[shift], out[0]), shift
+
+
+@pytest.mark.parametrize("hidden,inter,rows,top_k", [
+    (128, 128, 2, 3), (384, 256, 5, 3), (640, 384, 9, 2),
+    (7168, 128, 3, 1),   # two tokens' planes beyond 64 KB of LDS
+    (7680, 128, 2, 2),   # the longest rows that pair
+    (7936, 128, 3, 1),   # one token at a time: two do not leave room for a second block
+    (15872, 128, 2, 1),  # the longest rows the entry takes
+    (128, 128, 700, 6),  # more assignments than the grouping launch holds
+])
+@pytest.mark.parametrize("pairs", ["0", "1"])
+def test_e8m0_launch_regimes_bit_exact(hidden, inter, rows, top_k, pairs, monkeypatch):
+    """Rows one at a time and in pairs, at the lengths where the one takes over from the other."""
+    monkeypatch.setenv("FFMOE_E8M0_PAIRS", pairs)
+    experts, limit = 7, 7.0
+    routed, ref, sh_table, sh_ref = _tables(experts, hidden, inter, inter, 650 + rows)
+    x = rand_bf16((rows, hidden), 1.0, 651)
+    g = synth.generator(652)
+    ids = torch.stack([torch.randperm(experts, generator=g)[:top_k] for _ in range(rows)]).to(torch.int32)
+    wt = torch.rand((rows, top_k), generator=g) * 0.5 + 0.05
+    op = E8m0DecodeOps(routed, sh_table.shared_struct(0), rows, top_k, limit)
+    contrib, shared_out = op.contribute(x.to(DEV), ids.to(DEV), wt.to(DEV))
+    torch.cuda.synchronize()
+    got, got_sh, xb = bits(contrib), bits(shared_out), bits(x)
+    for r in range(0, rows, max(1, rows // 20)):
+        for c in range(top_k):
+            assert np.array_equal(got[r, c], orc.expert_ffn_e8m0(1, xb[r], *ref[int(ids[r, c])], limit, float(wt[r, c]))), (r, c)
+        assert np.array_equal(got_sh[r], orc.expert_ffn_e8m0(0, xb[r], *sh_ref, limit, 1.0)), r
+    assert np.all(op.done.cpu().numpy() == 1)
