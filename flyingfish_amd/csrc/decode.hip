@@ -281,21 +281,30 @@ static int decode_impl(const ffmoe_expert_table* table, const ffmoe_shared_exper
     // one block per (row, group) kernels: it pays from about two rows per expert on (per-channel FP8, hidden 4096, 32 experts
     // top-4: 64 rows 0.89 against 1.56 ms in the Lane16 order, 512 rows 3.6 against 13.0 ms; 8 rows 0.41 against 0.30 ms)
     bool grouped = can_group && A >= 2 * E;
+    bool stream = rows_fit;
     if (rows_fit) {
-      // Streaming kernels: grouping costs its launch and 3 - 5 us of worse balance and saves the passes over weights that tokens
-      // share. Expected passes saved x bytes of an expert, per-channel FP8, Lane16, us grouped / not: 2 rows top-6 of 64 at
-      // 4096 / 1536 (25 MB) 79 / 68, 2 rows top-8 at 7168 / 2048 (83 MB) 152 / 151, 4 rows top-6 (92 MB) 119 / 107, 4 rows top-8
-      // (380 MB) 252 / 266, 8 rows top-6 (250 MB) 169 / 186, 32 rows (3.1 GB) 389 / 660.
+      // Streaming kernels: grouping costs its launch, a scan of the assignments by every expert's thread and worse balance; it saves
+      // the passes over weights that tokens share. The line, in expected passes saved (even routing) x bytes of an expert, was fitted to
+      // 876 shapes of both formats and orders, weights from HBM and from the caches: within 0.4 % of the better side on average and 22 %
+      // at worst, where one bound of 150 MB was 6 % off on average and up to 2.8 times. It rises with the tokens of a group, which are
+      // computed one by one, and with the scan. us grouped / not: per-channel FP8, 8 rows top-2 of 16 at 4096 / 1536 (236 MB) 117 / 82,
+      // 32 rows top-8 of 64 at 7168 / 2048 (3.1 GB) 389 / 660; BF16, 4 rows top-8 of 64 at 4096 / 1536 (321 MB) 178 / 198, 16 rows top-4
+      // of 64 at 1536 / 512 (178 MB) 67 / 52.
       double missed = 1.0;
       for (int i = 0; i < R && missed > 1e-3; ++i) missed *= 1.0 - double(K) / E;
       const double saved = double(A) - E * (1.0 - missed) + (shared ? R - 1 : 0);
-      grouped = can_group && saved * 3.0 * H * I * (fmt == FFMOE_FMT_BF16 ? 2 : 1) > 150e6;
+      const double expert = 3.0 * H * I * (fmt == FFMOE_FMT_BF16 ? 2 : 1);
+      grouped = can_group && saved * expert > (fmt == FFMOE_FMT_BF16 ? 0.0 : 75e6) + 30e6 * std::min(R, 12) + 1e6 * double(A) * std::min(1.0, 64.0 / E);
+      // Lane8 on BF16 rows of one LDS segment: with many passes in flight the kernel that reads them in accumulator order, all eight
+      // lanes' pieces of a line together, is ahead (us, streamed / not: 8 rows top-2 of 16 at 2048 / 1408 66 / 41, from HBM 66 / 65; top-8
+      // of 64 at 2048 / 768 107 / 101; but 2 rows of it 39 / 38, 4 rows 62 / 62, at 3072 / 1024 103 / 112)
+      stream = !(form == FFMOE_FORM_LANE8 && fmt == FFMOE_FMT_BF16 && H <= 2048 && !grouped && (double(A) + (shared ? R : 0)) * expert > 320e6);
     }
     if (const char* f = getenv("FFMOE_FORM_GROUPED")) grouped = can_group && atoi(f) != 0;
     if (!grouped) {
       p.groups = nullptr;
       p.counters = nullptr;
-      if (rows_fit) return decode_form_rows_launch(fmt, form, 1, p, (long long)A, shared ? R : 0, stage_mask, st);
+      if (stream) return decode_form_rows_launch(fmt, form, 1, p, (long long)A, shared ? R : 0, stage_mask, st);
       return decode_form_launch(fmt, form, p, stage_mask, st);
     }
     p.groups = (GroupDesc*)(sc + hbytes);

@@ -228,3 +228,19 @@ def test_form_call_larger_than_one_grid_dimension_bitwise():
         assert torch.equal(c.view(torch.int16), contrib[r0:r0 + n].view(torch.int16)), r0
         assert torch.equal(s.view(torch.int16), shared_out[r0:r0 + n].view(torch.int16)), r0
     assert int(op.done.min()) == 1
+
+
+def test_lane8_bf16_call_of_many_passes_equals_its_rows_bitwise():
+    """Eight rows whose passes over the weights leave the streaming kernels, against the rows one at a time."""
+    experts, hidden, inter, rows, top_k = 4, 2048, 1408, 8, 2
+    table, ref, sh, x, ids, wt = _case(capi.FMT_BF16, experts, hidden, inter, rows, top_k, 6100, True)
+    op = DecodeOps(table, sh, rows, top_k, weights_f32=True)
+    contrib, shared_out = op.contribute(x.to(DEV), ids.to(DEV), wt.to(DEV), form=capi.FORM_LANE8)
+    one = DecodeOps(table, sh, 1, top_k, weights_f32=True)
+    for r in range(rows):
+        c, s = one.contribute(x[r:r + 1].to(DEV), ids[r:r + 1].to(DEV), wt[r:r + 1].to(DEV), form=capi.FORM_LANE8)
+        assert torch.equal(c[0].view(torch.int16), contrib[r].view(torch.int16)), r
+        assert torch.equal(s[0].view(torch.int16), shared_out[r].view(torch.int16)), r
+    assert int(op.done.min()) == 1
+    want = orc.expert_ffn(bits(x)[0], *ref[int(ids[0, 0])], float(wt[0, 0]), orc.TWICE, 0.0, orc.AFTER_DOWN_BF16, orc.LANE8, orc.SILU_DIV)
+    assert np.array_equal(bits(contrib)[0, 0], want)
