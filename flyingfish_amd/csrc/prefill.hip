@@ -480,13 +480,21 @@ bool launch_w16_narrow(int format, const W16Params& p, int mf, unsigned blocks, 
   return false;
 }
 
-// Dense W8A8 rows on the 128 x 128 tile kernel (FFMOE_W8A8_TILE: 1 always, 0 never; same bits). It is ahead from about three
-// tiles for every four CUs: 400 x 2048 -> 7168 (224 tiles) 21.3 against 23.8 us, 512 x 7168 -> 7168 (224) 55 against 67,
-// 2048 x 2048 -> 7168 (896) 53 against 71; below, the 64-row kernel's smaller units spread further: 300 x 4096 -> 4096 (96)
-// 31.8 against 30.3 us.
-bool use_tiles(int mode, int rows, int n) {
+// Dense W8A8 rows on the 128 x 128 tile kernel (FFMOE_W8A8_TILE: 1 always, 0 never; same bits). Below about three tiles for every
+// four CUs the 64-row kernel's smaller units spread further: 300 x 4096 -> 4096 (96 tiles) 30.3 us against 31.8. Where that kernel
+// would need a second unit per CU the tiles are ahead: 2048 x 2048 -> 7168 (896) 53 us against 71, 1150 x 4096 -> 4096 (288) 44
+// against 50. With one unit per CU it is the other way round (1000 x 4096 -> 4096 34.7 against 33.3, 2048 x 2048 -> 2048 24.0
+// against 22.3), except where an XCD's units lie side by side over so many columns that every one of them streams its own weights:
+// from 22 column tiles on, two thirds of an XCD's CUs (512 x 7168 -> 7168 52 against 66, 700 x 7168 -> 5120 equal); more tiles than
+// CUs still lose there (700 x 7168 -> 5632, 264 tiles, 62 against 57). Contractions up to 1536, where start-up is a larger part of a
+// unit, from 15 column tiles on (850 x 1536 -> 4096 17.8 against 18.7, 1000 x 1536 -> 3072 equal).
+// mx: the E4M3 / E8M0 shared expert, whose 64-row kernel asks for its weights in operand order and is behind at every size.
+bool use_tiles(int mode, int rows, int n, int k, bool mx = false) {
   if (const char* f = getenv("FFMOE_W8A8_TILE")) return atoi(f) != 0;
-  return rows > 64 && 4ll * tile_units(mode, rows, n) >= 3ll * num_cus_p();
+  const long long cus = num_cus_p(), tiles = tile_units(mode, rows, n);
+  if (rows <= 64 || 4 * tiles < 3 * cus) return false;
+  const long long columns = (n + (mode == 0 ? 127 : 255)) / (mode == 0 ? 128 : 256);
+  return mx || (rows + 63) / 64 * columns > cus || (tiles <= cus && (k > 1536 ? 12 : 18) * columns > cus);
 }
 int launch_tiles(int mode, GemmParams& p, hipStream_t stream, bool mx = false) {
   p.total_units = tile_units(mode, p.rows_total, p.N);
@@ -558,7 +566,7 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_linear_fp8_block_w8a
   p.a_codes = (const uint8_t*)x_codes; p.a_scales = x_scales;
   p.w0_codes = (uint64_t)(uintptr_t)w_codes; p.w0_scales = (uint64_t)(uintptr_t)w_scales;
   p.out = (uint16_t*)y; p.rows_total = m; p.K = k; p.N = n; p.top_k = 1;
-  if (use_tiles(2, m, n)) return launch_tiles(2, p, (hipStream_t)stream);
+  if (use_tiles(2, m, n, k)) return launch_tiles(2, p, (hipStream_t)stream);
   p.total_units = uint32_t(((m + tm - 1) / tm) * ((n + 255) / 256));
   const unsigned blocks = (unsigned)std::min<uint32_t>((p.total_units + 7u) & ~7u, uint32_t(num_cus_p()) * 2u) & ~7u;
   return launch_gemm<2>(p, mf, blocks, (hipStream_t)stream);
@@ -841,7 +849,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
         q.w0_codes = shared->slot[0]; q.w0_scales = shared->slot[1]; q.w1_codes = shared->slot[2]; q.w1_scales = shared->slot[3];
         q.total_units = sgroups * uint32_t((SI + 127) / 128);
         q.out = (uint16_t*)(s + l.sh_act); q.K = H; q.N = SI;
-        if (mx_words && use_tiles(0, R, SI)) FF_TRY(launch_tiles(0, q, stream));
+        if (mx_words && use_tiles(0, R, SI, H, true)) FF_TRY(launch_tiles(0, q, stream));
         else FF_TRY(launch_mx_dense<0>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
       if (stages & 4) FF_TRY(ffmoe_act_quant_e8m0(s + l.sh_act, s + l.sh_aq, s + l.sh_sa, R, SI, stream_));
@@ -850,7 +858,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
         q.w0_codes = shared->slot[4]; q.w0_scales = shared->slot[5]; q.w1_codes = 0; q.w1_scales = 0;
         q.total_units = sgroups * uint32_t((H + 255) / 256);
         q.out = (uint16_t*)args->shared_out; q.K = SI; q.N = H;
-        if (mx_words && use_tiles(2, R, H)) FF_TRY(launch_tiles(2, q, stream));
+        if (mx_words && use_tiles(2, R, H, SI, true)) FF_TRY(launch_tiles(2, q, stream));
         else FF_TRY(launch_mx_dense<2>(q, smf, std::min<unsigned>(blocks, (q.total_units + 7u) & ~7u), stream));
       }
     }
@@ -922,7 +930,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
       q.w0_codes = shared->slot[0]; q.w0_scales = shared->slot[1]; q.w1_codes = shared->slot[2]; q.w1_scales = shared->slot[3];
       q.total_units = sgroups * uint32_t(snv ? (SI + 255) / 256 : (SI + 127) / 128);
       q.out = (uint16_t*)(s + l.sh_act); q.K = H; q.N = SI;
-      if (!snv && use_tiles(0, R, SI)) FF_TRY(launch_tiles(0, q, stream));
+      if (!snv && use_tiles(0, R, SI, H)) FF_TRY(launch_tiles(0, q, stream));
       else FF_TRY(launch_gemm<0>(q, smf, std::min<unsigned>(snv ? blocks / 2 : blocks, (q.total_units + 7u) & ~7u), stream, false, snv));
     }
     if (stages & 4)
@@ -933,7 +941,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
       q.w0_global = shared->global_scales[2];
       q.total_units = sgroups * uint32_t(snv ? (H + 511) / 512 : (H + 255) / 256);
       q.out = (uint16_t*)args->shared_out; q.K = SI; q.N = H;
-      if (!snv && use_tiles(2, R, H)) FF_TRY(launch_tiles(2, q, stream));
+      if (!snv && use_tiles(2, R, H, SI)) FF_TRY(launch_tiles(2, q, stream));
       else FF_TRY(launch_gemm<2>(q, smf, std::min<unsigned>(snv ? blocks / 2 : blocks, (q.total_units + 7u) & ~7u), stream, false, snv));
     }
   }
