@@ -397,13 +397,22 @@ bool nvfp4_lines_enabled() {
 }
 
 // NVFP4 cohorts of a prompt chunk on the tile kernel (nvfp4_tile.cuh; FFMOE_NVFP4_TILE: 1 wherever it can run, 0 never; same
-// bits). It multiplies the live rows of 64-row groups, which pays where some experts are popular (256 experts, Zipf-like: 100
-// tokens 1168 -> 1058 us a layer, 200 tokens 1608 -> 1423, 1021 tokens 3136 -> 2414); on the one or two rows per expert of a
-// decode step the line kernel's wider blocks are ahead (32 tokens of top-8 of 256: 934 against 978 us; 64 tokens of 64
-// experts, even: 468 against 474).
-bool nvfp4_tiles(int rows, int top_k, int experts) {
+// bits). It multiplies the live rows of 64-row groups; the line kernel's 16-row groups dequantize an expert once more for every 16
+// of its rows. Time against the line kernel's, mean of three seeded routings, even / Zipf-like, by rows per expert:
+//                                  4            6            8            10           12           14
+//   top-8 of 256, 7168 / 2048   1.07 / 0.98  1.07 / 0.95  1.06 / 0.92  1.04 / 0.88  0.97 / 0.86  0.89 / 0.84
+//   top-8 of 128, 4096 / 1024                1.07 / 0.95  0.98 / 0.94  0.95 / 0.86  0.96 / 0.90  0.87 / 0.85
+//   top-6 of 64, 4096 / 1536                              1.03 / 0.96  0.92 / 0.97  0.95 / 0.88  0.89 / 0.85
+//   top-4 of 128, 2048 / 768    1.02 / 1.01  1.02 / 0.99  0.96 / 0.97  0.92 / 0.95  0.94 / 0.92  0.82 / 0.81
+// Below 10 rows per expert it depends on the routing, which the host does not know, and an even one loses - unless the line kernel
+// has fewer gate/up units (128 activation columns of an expert) than two blocks per CU, of which the tile kernel makes twice as
+// many: top-4 of 64 at 7168 / 768, 5 rows 0.89 / 0.91, top-8 of 256 at 2048 / 256, 3 rows 0.95 / 0.97; it was behind at 3 rows and
+// below (64 tokens of 64 experts, even: 474 us against 468).
+bool nvfp4_tiles(int rows, int top_k, int experts, int inter) {
   if (const char* e = getenv("FFMOE_NVFP4_TILE")) return atoi(e) != 0;
-  return rows > 64 && (long long)rows * top_k > 3ll * experts;
+  const long long assignments = (long long)rows * top_k;
+  const bool few_units = (long long)experts * ((inter + 127) / 128) <= 2ll * num_cus_p();
+  return rows > 64 && (assignments >= 10ll * experts || (few_units && assignments > 3ll * experts));
 }
 
 // 16-row groups of the NVFP4 line kernel: one set of lines ahead and three blocks per CU (FFMOE_PREFILL_LINES_THREE_BLOCKS=0: two
@@ -773,7 +782,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   uint8_t* s = (uint8_t*)args->scratch;
   PrefillBook b{(uint32_t*)(s + l.counts), (uint32_t*)(s + l.offsets), (uint32_t*)(s + l.gbase), (uint32_t*)(s + l.totals),
                 (int*)(s + l.perm), (GemmGroup*)(s + l.groups), (u32x2*)(s + l.units0), (u32x2*)(s + l.units1)};
-  const bool nv_tile = a16 && table->format == FFMOE_FMT_NVFP4 && nvfp4_lines_enabled() && nvfp4_tiles(R, K, E) && H % 256 == 0 && I % 256 == 0;
+  const bool nv_tile = a16 && table->format == FFMOE_FMT_NVFP4 && nvfp4_lines_enabled() && nvfp4_tiles(R, K, E, I) && H % 256 == 0 && I % 256 == 0;
   const int mf = nv ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, (!mx && !a16) || mx || nv_tile);
   const int tm = 16 * mf;
   // W8A8 and W*A16 cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
