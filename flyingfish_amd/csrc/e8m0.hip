@@ -35,6 +35,16 @@ E8m0Layout e8m0_layout(int rows, int top_k, int hidden, int inter, int shared_in
 }  // namespace
 
 namespace {
+// LDS a block of the matrix-core kernels may ask for: the longest row of the entry takes 110 KB, beyond the 64 KB of a plain launch
+size_t tiles_lds_max() {
+  constexpr int most = 128 * 1024;
+  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_e8m0_tiles<0, true>), hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+                         hipFuncSetAttribute(reinterpret_cast<const void*>(k_e8m0_tiles<0, false>), hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+                         hipFuncSetAttribute(reinterpret_cast<const void*>(k_e8m0_tiles<1, false>), hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess;
+  if (!ok) (void)hipGetLastError();
+  return ok ? most : 64 * 1024;
+}
+
 // Pairing costs the grouping launch (5 us, and a scan of the assignments by every expert) and saves a pass over an expert's weights
 // per pair. us one at a time / in pairs (shared expert included): 2 rows, top-6 of 64 at 512 / 256: 20 / 26, 8 rows, top-8 of 64 at
 // 2048 / 768: 68 / 69, 16 rows 118 / 106; at 4096 / 1536 3 rows 73 / 71, 16 rows 292 / 218; 32 rows, top-8 of 256 at 1024 / 512:
@@ -117,9 +127,9 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_decode_contribute_e8
   // Exact arithmetic on the matrix cores wherever the contractions are whole instructions (multiples of 128 columns) and a
   // token's exponent planes fit LDS. Several rows: the assignments of an expert may share a pass over its weights in pairs.
   auto tiles_lds = [&](int tokens) { return std::max(e8m0_tiles_lds(0, H, tokens), e8m0_tiles_lds(1, imax, tokens)); };
-  constexpr size_t TWO_BLOCKS = 80 * 1024, ONE_BLOCK = 160 * 1024;  // LDS per CU: 160 KB
-  if (exact && H % 128 == 0 && I % 128 == 0 && SI % 128 == 0 && tiles_lds(1) <= ONE_BLOCK) {
-    const bool can_pair = R > 1 && K > 0 && (long long)R * K <= FFMOE_DECODE_MAX_ASSIGN && tiles_lds(FFMOE_E8M0_TOK) <= TWO_BLOCKS;
+  constexpr size_t TWO_BLOCKS = 80 * 1024;  // LDS per CU: 160 KB
+  if (exact && H % 128 == 0 && I % 128 == 0 && SI % 128 == 0 && tiles_lds(1) <= tiles_lds_max()) {
+    const bool can_pair = R > 1 && K > 0 && (long long)R * K <= FFMOE_DECODE_MAX_ASSIGN && tiles_lds(FFMOE_E8M0_TOK) <= std::min(TWO_BLOCKS, tiles_lds_max());
     const bool pairs = can_pair && pairs_pay(R, K, E, H, I, shared != nullptr);
     const int tokens = pairs ? FFMOE_E8M0_TOK : 1;
     long long groups = S;
