@@ -279,7 +279,8 @@ def test_e8m0_fp32_chain_variant_bit_exact(hidden, inter, shared_inter, rows, to
 def test_e8m0_matrix_core_tiles_bit_exact_on_any_code(hidden, inter, shared_inter, rows, top_k):
     """The matrix-core kernels of the exact arithmetic at the edges of their tiles, on weight codes drawn uniformly (every E2M1
     nibble, both zeros; every finite E4M3 code, so products over the whole exponent range) and on activations whose groups
-    mix the largest with the smallest E4M3 magnitudes, some groups all zero. Exact: any rounded product or sum is a failure."""
+    mix the largest with the smallest E4M3 magnitudes, some groups all zero. The outputs are BF16 behind a SwiGLU, so a lost last bit
+    shows only beside a tie here; test_e8m0_sums_that_cancel_to_their_last_bit isolates it."""
     rng = np.random.default_rng(9000 + hidden + rows)
     experts, limit = max(6, top_k), 7.0
     routed, ref, sh_table, sh_ref = _tables(experts, hidden, inter, shared_inter, 9100 + rows)
@@ -468,3 +469,73 @@ def test_e8m0_launch_regimes_bit_exact(hidden, inter, rows, top_k, pairs, monkey
             assert np.array_equal(got[r, c], orc.expert_ffn_e8m0(1, xb[r], *ref[int(ids[r, c])], limit, float(wt[r, c]))), (r, c)
         assert np.array_equal(got_sh[r], orc.expert_ffn_e8m0(0, xb[r], *sh_ref, limit, 1.0)), r
     assert np.all(op.done.cpu().numpy() == 1)
+
+
+_E4M3_INT = np.array([0 if c & 127 == 127 else ((8 + (c & 7)) << ((c >> 3 & 15) - 1) if c & 0x78 else c & 7) * (-1 if c & 128 else 1) for c in range(256)], dtype=np.int64)
+_E2M1_INT = np.array([0, 1, 2, 3, 4, 6, 8, 12, 0, -1, -2, -3, -4, -6, -8, -12], dtype=np.int64)
+
+
+@pytest.mark.parametrize("pairs", ["0", "1"])
+@pytest.mark.parametrize("weights", ["routed", "shared, small codes", "shared, large codes"])
+@pytest.mark.parametrize("low,high", [(1, 240), (1, 960), (9 << 5, 15 << 9), (9 << 7, 14 << 14), (9 << 10, 14 << 14)])
+def test_e8m0_sums_that_cancel_to_their_last_bit(weights, low, high, pairs, monkeypatch):
+    """Every dot is one smallest product of an exponent class (9 or 1 units times 1 or 3, or 9 or 11) beside large ones that cancel
+    exactly, anywhere in their group of 32 or (odd rows, sums of one sign) against the next group: a single bit lost from a
+    product or a sum changes the result outright. The parameters are the smallest and largest activation in units of 2^-9: the
+    exponent classes of the routed experts' tokens (bit 6 of the code) and of the shared expert's (0 .. 5, 6 .. 10, 11 .. 15). Three
+    rows, the second with every sign but the gate's turned, one at a time and two per instruction."""
+    monkeypatch.setenv("FFMOE_E8M0_PAIRS", pairs)
+    n = 128
+    packed = weights == "routed"
+    rng = np.random.default_rng(low + high + len(weights))
+    table = _E2M1_INT if packed else _E4M3_INT
+    code_of = {int(table[c]): c for c in reversed(range(len(table)))}
+    large, small = ([12, 8, 6], [1, 3]) if packed else ([960, 480, 832], [1, 3]) if "small" in weights else ([14 << 14, 15 << 13, 9 << 14], [9 << 7, 11 << 7])
+    ints = np.unique(np.abs(_E4M3_INT))
+    # groups 0 and 1: 448, which gives the group scale 1 and meets a zero weight, 26 large values in pairs, 5 small ones, the same
+    # magnitudes in both groups; group 2: 448, for the gate
+    pairs = np.repeat(rng.choice(ints[(ints >= high // 2) & (ints <= high)], 13), 2)
+    av, kind = np.zeros(n, dtype=np.int64), np.zeros(n, dtype=np.int64)  # kind: 0 zero weight, 1 .. 13 a pair, 14 small
+    for g in (0, 32):
+        order = rng.permutation(32)
+        av[g:g + 32] = (np.concatenate([[448 << 9], pairs, [low] * 5]) * rng.choice([-1, 1], 32))[order]
+        kind[g:g + 32] = np.concatenate([[0], np.repeat(np.arange(13) + 1, 2), [14] * 5])[order]
+    av[64] = 448 << 9
+    turn = np.where(np.arange(n) == 64, 1, -1)
+    x = torch.from_numpy((np.stack([av, av * turn, av]) * 2.0 ** -9).astype(np.float32)).to(torch.bfloat16)
+    codes, scales = orc.act_quant_e8m0(bits(x))
+    assert np.array_equal(_E4M3_INT[codes[0]], av) and np.all(scales[0, :3] == 127)
+    sign = np.sign(av)
+    w = np.zeros((n, n), dtype=np.int64)
+    for j in range(n):
+        if j % 2:
+            v = large[j // 2 % 3]
+            w[j, :64] = np.where((kind[:64] > 0) & (kind[:64] < 14), v * sign[:64], 0)
+            w[j, 32:64] *= -1
+        else:
+            for i in range(1, 14):
+                a, b = np.flatnonzero(kind[:32] == i)
+                v = int(rng.choice(large)) * int(rng.choice([-1, 1]))
+                w[j, a], w[j, b] = v * sign[a], -v * sign[b]
+        w[j, rng.choice(np.flatnonzero(kind[:32] == 14))] = int(rng.choice(small)) * int(rng.choice([-1, 1]))
+    total = w @ av
+    assert np.all(total != 0) and np.abs(total).max() <= 11 * low * max(small)
+    shift = int(np.floor(np.log2(float(np.abs(total).max()) * 2.0 ** (-10 if packed else -18))))  # the largest total lies between 1 and 2
+    up = np.vectorize(lambda v: code_of[int(v)], otypes=[np.uint8])(w)
+    gate = np.zeros((n, n), dtype=np.uint8)
+    gate[:, 64] = code_of[12 if packed else 960]
+    if packed:
+        down, sdown = _identity_down(n)
+        m = [_pack(gate), np.full((n, n // 32), 120, dtype=np.uint8), _pack(up), np.full((n, n // 32), 127 - shift, dtype=np.uint8), down, sdown]
+        got, _ = _one_choice(_single_expert(n, n, m[0::2], m[1::2]), x)
+    else:
+        blocks = lambda c: np.full((n // 32, n // 32), c, dtype=np.uint8)
+        m = [gate, blocks(120), up, blocks(127 - shift), (0x38 * np.eye(n)).astype(np.uint8), blocks(127)]
+        routed, _, sh_table, _ = _tables(1, n, n, n, 900)
+        for v, a in zip(sh_table.expert_views(0), m):
+            v.copy_(torch.from_numpy(a))
+        _, got = _one_choice(routed, x, shared=sh_table.shared_struct(0))
+    for r in range(3):
+        want = orc.expert_ffn_e8m0(packed, bits(x)[r], *m, 7.0, 1.0)
+        assert np.count_nonzero(want & 0x7fff) == n  # every total survives to the output
+        assert np.array_equal(got[r], want), (r, np.flatnonzero(got[r] != want))
