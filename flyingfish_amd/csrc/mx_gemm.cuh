@@ -9,8 +9,8 @@
 // bit for bit; the matrix core adds the 128 products of an instruction in its own FP32 tree, so this path is the
 // tolerance-checked variant (same quantized operands, same roundings between the stages).
 //
-// Work model, unit list and token staging are those of k_w8a8_grouped (w8a8_gemm.cuh); the token tile carries 128 code
-// bytes and the 4 scale bytes of the K block per row. Operand layout of the instruction, measured on the device with
+// Work model and token staging of the kernel here are those of k_w8a8_grouped (w8a8_gemm.cuh) over consecutive rows; the token tile
+// carries 128 code bytes and the 4 scale bytes of the K block per row. Operand layout of the instruction, measured on the device with
 // one-hot operands (the two element widths do NOT share it): with c = lane / 16,
 //   * a 4-bit operand holds columns 32 c .. 32 c + 31 of the K block in its 16 bytes (low nibble = even column);
 //   * an 8-bit operand holds columns 16 c .. 16 c + 15 in bytes 0-15 and columns 64 + 16 c .. 64 + 16 c + 15 in bytes 16-31;
@@ -28,16 +28,18 @@ namespace ffmoe {
 struct MxParams {
   const uint8_t* a_codes;    // activation E4M3 codes [*, K]
   const uint8_t* a_scales;   // activation E8M0 scales [*, K / 32]
-  const uint64_t* slots;     // [E, 6] expert table, or NULL: the four addresses below
-  uint64_t w0_codes, w0_scales, w1_codes, w1_scales;  // MODE 0: gate, up; MODE 1/2: w0 only
-  const GemmGroup* groups;   // NULL: rows split arithmetically into groups of TM
+  uint16_t* out;
+  // routed experts (mx_tile.cuh)
+  const uint64_t* slots;     // [E, 6] expert table
+  const GemmGroup* groups;
   const u32x2* units;
   const uint32_t* unit_total;
-  uint32_t total_units;
-  const int* perm;           // permuted position -> assignment index (NULL: identity)
-  const float* weights;      // routing weights per assignment (MODE 0 with perm; NULL: 1)
-  uint16_t* out;
+  const int* perm;           // permuted position -> assignment index
+  const float* weights;      // MODE 0: routing weights per assignment (NULL: 1)
   uint32_t* done;
+  // the shared expert (here and tile_gemm.cuh): all rows in order
+  uint64_t w0_codes, w0_scales, w1_codes, w1_scales;  // MODE 0: gate, up; MODE 2: w0 only
+  uint32_t total_units;
   int rows_total;
   int K, N, top_k;
   float limit;
@@ -51,7 +53,7 @@ __device__ __forceinline__ uint32_t mx_swiglu(float gate, float up, float weight
   return f32_to_bf16(__fmul_rn(__fmul_rn(silu, u), weight));
 }
 
-// E4M3 codes [N, K], E8M0 scales [N / 32, K / 32]: the always-on expert over all rows (E2M1 codes [N, K / 2], low nibble = even
+// E4M3 codes [N, K], E8M0 scales [N / 32, K / 32]: the always-on expert over all rows, MODE 0 and 2 (E2M1 codes [N, K / 2], low nibble = even
 // column, and scales [N, K / 32] of the routed experts are mx_tile.cuh's)
 template <int MF, int MODE, int P>
 __global__ __launch_bounds__(256, 2) void k_mx_dense(const MxParams p) {
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void k_mx_dense(const MxParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int K = p.K, N = p.N, KB = K >> 7, SB = K >> 5;
-  const uint32_t total = p.unit_total ? uint32_t(uni(int(load_global<uint32_t>(p.unit_total)))) : p.total_units;
+  const uint32_t total = p.total_units;
   const int ntiles = (N + gemm_tile_cols<MODE, NW>() - 1) / gemm_tile_cols<MODE, NW>();
   const int q4 = lane >> 4;  // this lane's scale block inside a K block
 
@@ -73,35 +75,8 @@ __global__ __launch_bounds__(256, 2) void k_mx_dense(const MxParams p) {
   const uint32_t span = (total + 7u) >> 3;
   const uint32_t span_end = min(total, (xcd + 1u) * span);
   for (uint32_t u = xcd * span + slot; u < span_end; u += per_xcd) {
-    int expert, start, n, t;
-    if (p.groups) {
-      const u32x2 un = load_global<u32x2>(p.units + u);
-      const int g = uni(int(un.x));
-      t = uni(int(un.y));
-      const int* gd = reinterpret_cast<const int*>(p.groups + g);
-      expert = uni(load_global<int>(gd));
-      start = uni(load_global<int>(gd + 1));
-      n = uni(load_global<int>(gd + 2));
-    } else {
-      const int g = int(u) / ntiles;
-      t = int(u) - g * ntiles;
-      expert = 0;
-      start = g * TM;
-      n = min(TM, p.rows_total - start);
-    }
-    uint64_t wc[2], ws[2];
-    if (p.slots) {
-      const uint64_t* sl = p.slots + size_t(expert) * 6;
-      if (MODE == 0) {
-        wc[0] = uni64(load_global<uint64_t>(sl + 0)); ws[0] = uni64(load_global<uint64_t>(sl + 1));
-        wc[1] = uni64(load_global<uint64_t>(sl + 2)); ws[1] = uni64(load_global<uint64_t>(sl + 3));
-      } else {
-        wc[0] = wc[1] = uni64(load_global<uint64_t>(sl + 4)); ws[0] = ws[1] = uni64(load_global<uint64_t>(sl + 5));
-      }
-    } else {
-      wc[0] = p.w0_codes; ws[0] = p.w0_scales;
-      wc[1] = MODE == 0 ? p.w1_codes : p.w0_codes; ws[1] = MODE == 0 ? p.w1_scales : p.w0_scales;
-    }
+    const int g = int(u) / ntiles, t = int(u) - g * ntiles, start = g * TM, n = min(TM, p.rows_total - start);
+    const uint64_t wc[2] = {p.w0_codes, MODE == 0 ? p.w1_codes : p.w0_codes}, ws[2] = {p.w0_scales, MODE == 0 ? p.w1_scales : p.w0_scales};
     int col0[4];
     const uint8_t* wrow[4];   // this lane's codes of K block 0
     const uint8_t* srow[4];   // this lane's scale byte of K block 0
@@ -120,18 +95,11 @@ __global__ __launch_bounds__(256, 2) void k_mx_dense(const MxParams p) {
     for (int i = 0; i < CPT; ++i) {
       const int q = min(tid + NT * i, CHUNKS - 1);
       const int m = q >> 3, c = q & 7;
-      const int pos = start + min(m, n - 1);
-      const int row = MODE == 0 && p.perm ? load_global<int>(p.perm + pos) / p.top_k : pos;
-      tsrc[i] = p.a_codes + size_t(row) * K + c * 16;
+      tsrc[i] = p.a_codes + size_t(start + min(m, n - 1)) * K + c * 16;
       tdst[i] = m * 128 + ((c ^ (m & 7)) << 4);
     }
     const bool stage_chunk = CHUNKS >= NT || tid < CHUNKS;
-    const uint8_t* ssrc;
-    {
-      const int pos = start + min(min(tid, TM - 1), n - 1);
-      const int row = MODE == 0 && p.perm ? load_global<int>(p.perm + pos) / p.top_k : pos;
-      ssrc = p.a_scales + size_t(row) * SB;
-    }
+    const uint8_t* ssrc = p.a_scales + size_t(start + min(min(tid, TM - 1), n - 1)) * SB;
 
     v4f acc[MF][4];
 #pragma unroll
@@ -229,30 +197,26 @@ __global__ __launch_bounds__(256, 2) void k_mx_dense(const MxParams p) {
       if (token < n) {
         const int pos = start + token;
         if (MODE == 0) {
-          float wk = 1.0f;
-          if (p.perm && p.weights) wk = load_global<float>(p.weights + load_global<int>(p.perm + pos));
 #pragma unroll
           for (int f = 0; f < 2; ++f) {
             const int col = col0[f] + sub;
             if (col0[f] + 16 <= N) {
               uint32_t o[4];
 #pragma unroll
-              for (int r = 0; r < 4; ++r) o[r] = mx_swiglu(acc[m][f][r], acc[m][f + 2][r], wk, p.limit);
+              for (int r = 0; r < 4; ++r) o[r] = mx_swiglu(acc[m][f][r], acc[m][f + 2][r], 1.0f, p.limit);
               const u32x2 v = {o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
               *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col) = v;
             }
           }
         } else {
-          const int a = (MODE == 1 && p.perm) ? load_global<int>(p.perm + pos) : pos;
 #pragma unroll
           for (int f = 0; f < 4; ++f) {
             const int col = col0[f] + sub;
             if (col0[f] + 16 <= N) {
               const u32x2 o = {pack_bf16x2(acc[m][f][0], acc[m][f][1]), pack_bf16x2(acc[m][f][2], acc[m][f][3])};
-              *reinterpret_cast<u32x2*>(p.out + size_t(a) * N + col) = o;
+              *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col) = o;
             }
           }
-          if (MODE == 1 && p.done && t == 0 && wave == 0 && lane < 16) p.done[a] = 1u;
         }
       }
     }
