@@ -315,7 +315,8 @@ __global__ __launch_bounds__(256) void k_e8m0_stage(const E8m0Params q) {
 // group sum (times the group's two scales, an exponent). Four groups x two halves are eight of the sixteen columns: two
 // tokens per instruction. The FP32 sums are added in FP64 in any order, which equals the contract's ascending chain as
 // long as nothing rounds: certain when the groups' exponents of a row span few enough binades (checked per row and
-// token from the scale codes of the groups that are not all zero); a row that fails is redone in the contract's order.
+// token from the sum of the groups' magnitudes and the smallest scale codes of the groups that are not all zero); a row that fails is
+// redone in the contract's order.
 // The shared expert's E4M3 x E4M3 products need 8 + 11 bits: v_mfma_f32_16x16x32_bf16 on codes widened to BF16, the token
 // in three exponent classes (at most 6 binades) by columns and the weights in two (bit 6) by instructions, group sums below
 // 2^24 units.
@@ -338,7 +339,7 @@ constexpr int FFMOE_E8M0_NT = 512;
 __host__ __device__ __forceinline__ int e8m0_plane(int k) { return k + (k % 256 == 0 ? 128 : 0); }
 struct E8m0Red {  // cross-lane and cross-wave hand-over of a tile, per wave
   double total[2][FFMOE_E8M0_TOK][16], mass[2][FFMOE_E8M0_TOK][16];
-  int smin[2][16], smax[2][16];  // routed: scale codes of the row's groups that are not all zero; shared: smin[m][token] = exponent
+  int smin[2][16];  // routed: smallest scale code of the row's groups that are not all zero; shared: [m][token], smallest exponent
 };
 static_assert(sizeof(E8m0Red) <= 2048, "a wave's hand-over lies in its weight buffer");
 // LDS of a block: per wave a weight buffer (2 KB per matrix, the hand-over behind it), the tokens' planes, their scales, the
@@ -374,8 +375,8 @@ __device__ __forceinline__ int e8m0_scale_exponent(float amax) {
 __device__ __forceinline__ float e8m0_scaled(float v, int exponent) { return fminf(448.0f, fmaxf(-448.0f, __builtin_amdgcn_ldexpf(v, -exponent))); }
 
 // The tokens of a group into LDS: E4M3 codes by exponent class (THREE: exponents 0..5, 6..10, 11..15; else bit 6 of the code)
-// and one E8M0 scale per 32. CODES: the source is quantized already, else BF16. range[2 t], [2 t + 1]: smallest and largest
-// scale code of token t over its groups that are not all zero. K is a multiple of 128: quads of lanes stay whole.
+// and one E8M0 scale per 32. CODES: the source is quantized already, else BF16. range[t]: smallest scale code of token t over its
+// groups that are not all zero. K is a multiple of 128: quads of lanes stay whole.
 template <bool THREE, bool CODES>
 __device__ __forceinline__ void e8m0_stage_tokens(const uint64_t (&src)[FFMOE_E8M0_TOK], const uint64_t (&ssrc)[FFMOE_E8M0_TOK], int n, int K, uint8_t* planes,
                                                   int ps, uint8_t* scales, int* range, int tid) {
@@ -384,7 +385,7 @@ __device__ __forceinline__ void e8m0_stage_tokens(const uint64_t (&src)[FFMOE_E8
 #pragma unroll
   for (int t = 0; t < FFMOE_E8M0_TOK; ++t) {
     if (t >= n) break;
-    int lo = 255, hi = 0;
+    int lo = 255;
     uint8_t* pl = planes + size_t(t) * NP * ps;
     for (int v = tid; v < per; v += FFMOE_E8M0_NT) {  // eight elements a lane, a quad of lanes a group
       uint32_t o[2];
@@ -429,15 +430,15 @@ __device__ __forceinline__ void e8m0_stage_tokens(const uint64_t (&src)[FFMOE_E8
       any |= uint32_t(dpp_or<DPP_QUAD_SWAP1, 0xf>(0, int(any)));
       any |= uint32_t(dpp_or<DPP_QUAD_SWAP2, 0xf>(0, int(any)));
       if ((v & 3) == 0) scales[size_t(t) * (K >> 5) + (v >> 2)] = uint8_t(code);
-      if (any) { lo = code < lo ? code : lo; hi = code > hi ? code : hi; }
+      if (any) lo = code < lo ? code : lo;
     }
-    // one LDS atomic per wave and bound
+    // one LDS atomic per wave
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
-      int u = __shfl_xor(lo, off, 64); lo = u < lo ? u : lo;
-      u = __shfl_xor(hi, off, 64); hi = u > hi ? u : hi;
+      const int u = __shfl_xor(lo, off, 64);
+      lo = u < lo ? u : lo;
     }
-    if ((tid & 63) == 0) { atomicMin(range + 2 * t, lo); atomicMax(range + 2 * t + 1, hi); }
+    if ((tid & 63) == 0) atomicMin(range + t, lo);
   }
 }
 
@@ -522,8 +523,8 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
   uint8_t* xsc = lds + 8 * WB;                    // [token][G]
   uint8_t* wsc = xsc + ((size_t(lds_tokens) * G + 15) & ~size_t(15));
   uint8_t* planes = wsc + size_t(is_shared ? 4 : (STAGE == 0 ? 64 : 128)) * G;
-  __shared__ int range[2 * T];
-  if (tid < 2 * T) range[tid] = (tid & 1) ? 0 : 255;
+  __shared__ int range[T];
+  if (tid < T) range[tid] = 255;
 
   uint64_t sl[2 * NMAT];
 #pragma unroll
@@ -592,12 +593,13 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
     const int wr = (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
     const int rd0 = i * 128 + ((c ^ (i & 7)) << 4), rd1 = i * 128 + (((4 + c) ^ (i & 7)) << 4);
     double acc[NMAT][4];
-    int smin[NMAT], smax[NMAT];
+    float mass[NMAT][4];  // sum of |group sum|
+    int smin[NMAT];
 #pragma unroll
     for (int m = 0; m < NMAT; ++m) {
-      smin[m] = 255; smax[m] = 0;
+      smin[m] = 255;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[m][r] = 0.0;
+      for (int r = 0; r < 4; ++r) { acc[m][r] = 0.0; mass[m][r] = 0.0f; }
     }
     for (int kpo = k0; kpo < k1; kpo += D) {
 #pragma unroll
@@ -633,11 +635,10 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
             const u32x4 v = a[m][h];
             const bool nz = ((v[0] | v[1] | v[2] | v[3]) & 0x77777777u & in) != 0u;
             smin[m] = nz && sw < smin[m] ? sw : smin[m];
-            smax[m] = nz && sw > smax[m] ? sw : smax[m];
             const e8_i32x8 wf = {int(v[0]), int(v[1]), int(v[2]), int(v[3]), 0, 0, 0, 0};
             const e8_f32x4 r = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, tk, e8_f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 4, 0, 0, sw, 0, sx);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[m][e] += double(r[e]);
+            for (int e = 0; e < 4; ++e) { acc[m][e] += double(r[e]); mass[m][e] += fabsf(r[e]); }
           }
         }
       }
@@ -646,13 +647,14 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
     for (int m = 0; m < NMAT; ++m) {
       int o = __shfl_xor(smin[m], 16, 64); smin[m] = o < smin[m] ? o : smin[m];
       o = __shfl_xor(smin[m], 32, 64); smin[m] = o < smin[m] ? o : smin[m];
-      o = __shfl_xor(smax[m], 16, 64); smax[m] = o > smax[m] ? o : smax[m];
-      o = __shfl_xor(smax[m], 32, 64); smax[m] = o > smax[m] ? o : smax[m];
-      if (lane < 16) { red.smin[m][lane] = smin[m]; red.smax[m][lane] = smax[m]; }
+      if (lane < 16) red.smin[m][lane] = smin[m];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const double t = sum8_f64(acc[m][r]);
-        if ((lane & 7) == r) red.total[m][(lane >> 3) & 1][4 * c + r] = t;
+        const double t = sum8_f64(acc[m][r]), ms = sum8_f64(double(mass[m][r]));
+        if ((lane & 7) == r) {
+          red.total[m][(lane >> 3) & 1][4 * c + r] = t;
+          red.mass[m][(lane >> 3) & 1][4 * c + r] = ms;
+        }
       }
     }
   } else {
@@ -773,29 +775,26 @@ __global__ __launch_bounds__(FFMOE_E8M0_NT, 4) void k_e8m0_tiles(const E8m0Param
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) {
     double v = 0.0, ms = 0.0;
-    int lo = is_shared ? 4096 : 255, hi = 0;
+    int lo = is_shared ? 4096 : 255;
     for (int u = w_lo; u < w_hi; ++u) {
       const E8m0Red& ru = *reinterpret_cast<const E8m0Red*>(lds + size_t(u) * WB);
       v += ru.total[m][t][row];
+      ms += ru.mass[m][t][row];
       if (is_shared) {
-        ms += ru.mass[m][t][row];
         lo = ru.smin[m][t] < lo ? ru.smin[m][t] : lo;
       } else {
         lo = ru.smin[m][row] < lo ? ru.smin[m][row] : lo;
-        hi = ru.smax[m][row] > hi ? ru.smax[m][row] : hi;
       }
     }
     bool exact;
     if (is_shared) {
       exact = lo == 4096 || ms < pow2_f64(53 + lo - 18);  // units of 2^-18 below the smallest group's exponent
     } else {
-      // |group sum| < 2^27 units of 2^(scale codes - 264), G of them. The FP32 results stay away from both ends of the exponent
-      // range: 27 + 364 - 264 = 127 keeps a group's sum finite, 140 - 264 = -124 keeps its unit normal. A total that is not
-      // finite all the same holds a scale code of 255, which the contract reserves, over a group of zeros.
-      const int xlo = range[2 * t], xhi = range[2 * t + 1];
-      const int span = (xhi + hi) - (xlo + lo);
-      exact = lo > hi || xlo > xhi || (span + 27 + (32 - __builtin_clz(G)) <= 53 && xlo + lo >= 140 && xhi + hi <= 364 && hi <= 254);
-      exact = exact && fabs(v) < __builtin_inf();
+      // Units of 2^(smallest scale codes - 264), normal in FP32 from 140 on. The mass is an FP32 sum of up to 2^10 terms, off by less
+      // than one part in a thousand; a group sum beyond FP32 (scale codes from 366 on can: 32 x 448 x 6 x 2^(codes - 254)) or a scale
+      // code of 255, which the contract reserves, makes it infinite or NaN, and the comparison fails.
+      const int unit = range[t] + lo;
+      exact = ms * 1.001 < pow2_f64(53 + unit - 264) && unit >= 140;
     }
     if (!exact) {
       const uint8_t* wrow = reinterpret_cast<const uint8_t*>(sl[2 * m]) + size_t(j) * (is_shared ? K : K >> 1);

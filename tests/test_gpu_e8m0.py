@@ -539,3 +539,38 @@ def test_e8m0_sums_that_cancel_to_their_last_bit(weights, low, high, pairs, monk
         want = orc.expert_ffn_e8m0(packed, bits(x)[r], *m, 7.0, 1.0)
         assert np.count_nonzero(want & 0x7fff) == n  # every total survives to the output
         assert np.array_equal(got[r], want), (r, np.flatnonzero(got[r] != want))
+
+
+@pytest.mark.parametrize("up", [0, 6, 8, 14, 30])
+def test_e8m0_activations_over_many_binades_bit_exact(up):
+    """Group scales from the quantizer's floor up to 2^`up` times an ordinary token's: FP64 sums of any order, or the ordered chain
+    where those would round. Up to 25 binades, which tokens with near-silent and with outlying channels reach, a call takes about
+    as long as any other (the ordered chain is a hundred times slower)."""
+    experts, hidden, inter, rows = 2, 7168, 256, 2
+    routed, ref, _, _ = _tables(experts, hidden, inter, inter, 690)
+    rng = np.random.default_rng(691 + up)
+    f = np.exp2(up - rng.uniform(0, up + 14, (rows, hidden // 32, 1)))
+    f[:, 0], f[:, 1] = 2.0 ** up, 2.0 ** -14
+    x = torch.from_numpy((rng.standard_normal((rows, hidden // 32, 32)) * f).reshape(rows, hidden).astype(np.float32)).to(torch.bfloat16)
+    _, scales = orc.act_quant_e8m0(bits(x))
+    assert np.all(scales.max(1).astype(int) - scales.min(1) >= up + 14)
+    op = E8m0DecodeOps(routed, None, rows, 1, 7.0)
+    ids, wt = torch.tensor([[0], [1]], dtype=torch.int32, device=DEV), torch.ones((rows, 1), device=DEV)
+
+    def us(x):
+        op.contribute(x, ids, wt)
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(20):
+            op.contribute(x, ids, wt)
+        b.record()
+        b.synchronize()
+        return a.elapsed_time(b) * 50
+    plain = us(rand_bf16((rows, hidden), 1.0, 692).to(DEV))
+    wide = us(x.to(DEV))
+    got = bits(op.contributions)[:, 0]
+    for r in range(rows):
+        assert np.array_equal(got[r], orc.expert_ffn_e8m0(1, bits(x)[r], *ref[r], 7.0, 1.0)), r
+    print("up=%d: %.1f us against %.1f" % (up, wide, plain))
+    if up <= 8:
+        assert wide < 8 * plain
