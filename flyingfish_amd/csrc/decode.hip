@@ -298,7 +298,8 @@ static int decode_impl(const ffmoe_expert_table* table, const ffmoe_shared_exper
       // Lane8 on BF16 rows of one LDS segment: with many passes in flight the kernel that reads them in accumulator order, all eight
       // lanes' pieces of a line together, is ahead (us, streamed / not: 8 rows top-2 of 16 at 2048 / 1408 66 / 41, from HBM 66 / 65; top-8
       // of 64 at 2048 / 768 107 / 101; but 2 rows of it 39 / 38, 4 rows 62 / 62, at 3072 / 1024 103 / 112)
-      stream = !(form == FFMOE_FORM_LANE8 && fmt == FFMOE_FMT_BF16 && H <= 2048 && !grouped && (double(A) + (shared ? R : 0)) * expert > 320e6);
+      stream = !(form == FFMOE_FORM_LANE8 && fmt == FFMOE_FMT_BF16 && H <= 2048 && !grouped && (double(A) + (shared ? R : 0)) * expert > 320e6) ||
+               R > 65535 || imax > 32 * 1024;  // what its grid and a row in LDS hold
     }
     if (const char* f = getenv("FFMOE_FORM_GROUPED")) grouped = can_group && atoi(f) != 0;
     if (!grouped) {
