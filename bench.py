@@ -471,14 +471,14 @@ def prefill_main(args, torch, capi, ops, synth, prebuilt=None):
         "cohort_mfma_frac": flop_total / (ms * 1e-3) / 1e12 / peak,
         "weight_bytes_once": touched * per,
         "cohort_weight_gbps": touched * per / (ms * 1e-3) / 1e9,
-        "roofline": {"kernel": ("ffmoe::k_w16_grouped<F, MF, 0, P>" if a16 else "ffmoe::k_mx_tile<0>" if mx else "ffmoe::k_w8a8_grouped<MF, 0, P>") + " (gate/up grouped GEMM + SwiGLU)", "bound": "mfma",
+        "roofline": {"kernel": ("ffmoe::k_nvfp4_tile<0>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 0, P>" if a16 else "ffmoe::k_mx_tile<0>" if mx else "ffmoe::k_w8a8_grouped<MF, 0, P>") + " (gate/up grouped GEMM + SwiGLU)", "bound": "mfma",
                      "achieved": flop0 / (k0_avg * 1e-3) / 1e12, "peak": peak, "unit": "TFLOP/s",
                      "frac": flop0 / (k0_avg * 1e-3) / 1e12 / peak,
                      "traffic": PREFILL_GATE_UP_TRAFFIC_BYTES if default_cohort else None,
                      "traffic_source": PREFILL_TRAFFIC_SOURCE if default_cohort else None,
                      "flop_per_launch": flop0, "avg_ms": k0_avg, "min_ms": k0[0],
                      "weight_bytes_once": touched * per * 2 // 3, "weight_gbps": touched * per * 2 / 3 / (k0_avg * 1e-3) / 1e9},
-        "down_kernel": {"kernel": "ffmoe::k_w16_grouped<F, MF, 1, P>" if a16 else "ffmoe::k_mx_tile<1>" if mx else "ffmoe::k_w8a8_grouped<MF, 1, P>", "avg_ms": k1_avg, "min_ms": k1[0],
+        "down_kernel": {"kernel": "ffmoe::k_nvfp4_tile<1>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 1, P>" if a16 else "ffmoe::k_mx_tile<1>" if mx else "ffmoe::k_w8a8_grouped<MF, 1, P>", "avg_ms": k1_avg, "min_ms": k1[0],
                         "tflops": A * 2.0 * H * I / (k1_avg * 1e-3) / 1e12},
     }
     out["router_logits"] = {"kernel": "ffmoe::k_route_logits_f32_rows (FP32 logits of all token rows, vector ALUs, the oracle's summation order)",

@@ -1,5 +1,5 @@
 // Grouped W4A16 GEMM of NVFP4 experts with K a multiple of 256: 128 weight rows x up to 64 tokens per block of four waves,
-// both operands through LDS by direct loads, two blocks per CU. Arithmetic (dequantization to the decode path's BF16 effective
+// both operands through LDS by direct loads, three blocks per CU. Arithmetic (dequantization to the decode path's BF16 effective
 // weights, operand order, epilogue) is that of k_w16_grouped<FmtNvfp4>, results equal bit for bit.
 //
 // What bounds it: the weight stream next to two VALU instructions of dequantization per weight and row group, which want

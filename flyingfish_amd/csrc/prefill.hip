@@ -345,16 +345,17 @@ inline uint64_t up256(uint64_t v) { return (v + 255) & ~uint64_t(255); }
 
 // rows per group for an average of `avg` rows per expert
 // (cap: the largest group a path's kernels are built for, in units of 16 rows; anything else in the variable is ignored)
-int pick_mf(double avg, int cap, bool w8a8 = false) {
+int pick_mf(double avg, int cap, bool groups64) {
   if (const char* f = getenv("FFMOE_PREFILL_MF")) {
     const int v = atoi(f);
     if (v == 1 || v == 2 || v == 4 || v == 8) return std::min(v, cap);
   }
-  // W8A8: the 64-row kernel with eight waves per block is ahead at every cohort size measured (top-8 of 256 experts at
+  // groups64: the W8A8, MX and NVFP4 tile kernels take 64-row groups whatever the average. W8A8: the 64-row kernel with eight waves per block is ahead at every cohort size measured (top-8 of 256 experts at
   // hidden 7168, 32 / 128 / 512 / 2048 tokens: 0.74 / 1.42 / 2.04 / 2.65 ms against 0.77 / 1.54 / 2.30 / 4.17 ms with 32-row
-  // groups and 0.77 / 1.55 / 2.71 / 6.79 ms with 16-row groups). The W*A16 and MX kernels dequantize per row group
-  // and keep the short groups for short segments (64 rows, 16-row groups: 1.89 ms, 64-row groups: 2.17 ms).
-  if (w8a8) return 4;
+  // groups and 0.77 / 1.55 / 2.71 / 6.79 ms with 16-row groups); the tile kernels move and multiply the live rows of a group only.
+  // The other W*A16 kernels dequantize per row group and keep short groups for short segments (64 rows, 16-row groups: 1.89 ms,
+  // 64-row groups: 2.17 ms).
+  if (groups64) return 4;
   return avg > 24.0 ? 4 : avg > 12.0 ? 2 : 1;
 }
 

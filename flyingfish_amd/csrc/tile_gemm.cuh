@@ -10,7 +10,7 @@
 // registers on its way in, and a wave's 16 instructions read 16 KB; the 32 KB of a K block are requested one K block ahead
 // and land while the previous one is multiplied. Two independent blocks per CU (66 KB of LDS each) cover each other's
 // barriers, first loads and epilogues. Measured: 4096 x 7168 -> 4096 in 142 us = 1.69 PFLOP/s (matrix cores busy 40 % of
-// the cycles at the 2.0 GHz the chip holds here), 2048 x 2048 -> 7168 66 -> 47 us. The same loop without its loads takes
+// the cycles at the 2.05 GHz the chip holds here), 2048 x 2048 -> 7168 66 -> 47 us. The same loop without its loads takes
 // 105 us. Not faster: 256 x 128 tiles with three stages and one block per CU (145 us), 256 x 256 tiles (144), the next K block's
 // operands read into registers under the matrix work (155).
 #pragma once
@@ -20,8 +20,8 @@
 namespace ffmoe {
 
 // Waves: wave / 2 is the weight half (64 rows), wave % 2 the token half (64 tokens). LDS rows are 128 bytes, 16-byte piece
-// c of row r at c ^ (r / 2 & 7), so that the 16 rows of an operand read cover all 64 banks (keyed by r & 7 half of the LDS cycles
-// were conflicts); the swizzle is applied to the source address, since a direct load writes its lanes in order.
+// c of row r at c ^ (r / 2 & 7), so that the 16 rows of an operand read cover all 64 banks (the counters report 47 % of the LDS
+// cycles as conflicts all the same, as they do with r & 7 for the key); the swizzle is applied to the source address, since a direct load writes its lanes in order.
 // MX: E4M3 weights with one E8M0 scale per 32 x 32 block against E4M3 activations with one per 32 columns (mx_gemm.cuh's dense form, the
 // same bits): the matrix core applies the scales and sums over the whole contraction. 1500 tokens at hidden 7168 / intermediate 2048:
 // gate/up 142 -> 88 us, down 70 -> 39 us against 64-row units with the weights requested in operand order.
