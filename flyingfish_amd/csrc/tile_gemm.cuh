@@ -20,8 +20,7 @@
 namespace ffmoe {
 
 // Waves: wave / 2 is the weight half (64 rows), wave % 2 the token half (64 tokens). LDS rows are 128 bytes, 16-byte piece
-// c of row r at c ^ (r / 2 & 7), so that the 16 rows of an operand read cover all 64 banks (the counters report 47 % of the LDS
-// cycles as conflicts all the same, as they do with r & 7 for the key); the swizzle is applied to the source address, since a direct load writes its lanes in order.
+// c of row r at c ^ lds_key(r); the swizzle is applied to the source address, since a direct load writes its lanes in order.
 // MX: E4M3 weights with one E8M0 scale per 32 x 32 block against E4M3 activations with one per 32 columns (mx_gemm.cuh's dense form, the
 // same bits): the matrix core applies the scales and sums over the whole contraction. 1500 tokens at hidden 7168 / intermediate 2048:
 // gate/up 142 -> 88 us, down 70 -> 39 us against 64-row units with the weights requested in operand order.
@@ -42,11 +41,11 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
   const uint32_t lds_w[2] = {lds_address(stage[0].w) + uint32_t(wave) * 4096u, lds_address(stage[1].w) + uint32_t(wave) * 4096u};
   const uint32_t lds_t[2] = {lds_address(stage[0].t) + uint32_t(wave) * 4096u, lds_address(stage[1].t) + uint32_t(wave) * 4096u};
   const uint32_t lds_s[2] = {lds_address(stage[0].sx[wave]), lds_address(stage[1].sx[wave])};
-  const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ (lane >> 4)) << 4);  // odd requests: piece ^ 4
+  const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ lds_key(lane >> 3)) << 4);  // odd requests: piece ^ 4
   // operand reads: row lane % 16, bytes 32 c .. 32 c + 31 of the K block for lane group c
   // (MX: bytes 16 c .. 16 c + 15 and 64 + 16 c .. 64 + 16 c + 15, the operand form whose scales sit in lane group column / 32)
   const int r16 = lane & 15, c = lane >> 4, c_lo = MX ? c : 2 * c, c_hi = MX ? c + 4 : 2 * c + 1;
-  const int rd_lo = r16 * 128 + ((c_lo ^ (r16 >> 1)) << 4), rd_hi = r16 * 128 + ((c_hi ^ (r16 >> 1)) << 4);
+  const int rd_lo = r16 * 128 + ((c_lo ^ lds_key(r16)) << 4), rd_hi = r16 * 128 + ((c_hi ^ lds_key(r16)) << 4);
 
   for (uint32_t u = xcd * span + slot; u < span_end; u += per_xcd) {
     // blocks of eight column tiles, row groups inside: the blocks of an XCD run an 8 x 8 window of tiles (4096 x 7168 -> 4096:
@@ -68,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
     const float* ssrc;       // the scales of this wave's 64 tokens
     auto token_row = [&](int m) { return start + min(m, n - 1); };
 #pragma unroll
-    for (int i = 0; i < 4; ++i) tsrc[i] = p.a_codes + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * K + (((lane & 7) ^ (lane >> 4) ^ 4 * (i & 1)) << 4);
+    for (int i = 0; i < 4; ++i) tsrc[i] = p.a_codes + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * K + (((lane & 7) ^ lds_key(lane >> 3) ^ 4 * (i & 1)) << 4);
     ssrc = p.a_scales + size_t(token_row(wt * 64 + lane)) * KB;  // MX: the four scale bytes of a K block are one word
     // Block scales, one word per K block; lane l keeps K block l (+ 64). A wave's columns sit inside one 128-row block; MX: four
     // bytes per 32 rows, which are the wave's fragments 0, 1 and its fragments 2, 3.

@@ -86,9 +86,9 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int K = p.K, N = p.N, KB = K >> 7;
-  const int wr_off = (lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) << 4);                 // rows 0..7; rows 8..15 at + 1024
-  const int rd_lo = (lane & 15) * 128 + (((2 * (lane >> 4)) ^ (lane & 7)) << 4);
-  const int rd_hi = (lane & 15) * 128 + (((2 * (lane >> 4) + 1) ^ (lane & 7)) << 4);
+  const int wr_off = (lane >> 3) * 128 + (((lane & 7) ^ lds_key(lane >> 3)) << 4);  // rows 0..7; rows 8..15 at + 1024, key ^ 4
+  const int rd_lo = (lane & 15) * 128 + (((2 * (lane >> 4)) ^ lds_key(lane & 15)) << 4);
+  const int rd_hi = (lane & 15) * 128 + (((2 * (lane >> 4) + 1) ^ lds_key(lane & 15)) << 4);
   const uint32_t total = p.unit_total ? uint32_t(uni(int(load_global<uint32_t>(p.unit_total)))) : p.total_units;
   const int ntiles = (N + gemm_tile_cols<MODE, NW>() - 1) / gemm_tile_cols<MODE, NW>();
 
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
                               : TW ? uint32_t(lane >> 3) * uint32_t(K) + uint32_t(lane & 7) * 16u : uint32_t(lane & 15) * uint32_t(K) + uint32_t(lane >> 4) * 32u;
     const uint32_t woff1 = NV ? uint32_t(lane >> 2) * uint32_t(K >> 4) + uint32_t((lane & 3) >> 1) * 4u : woff0 + (TW ? 8u * uint32_t(K) : 16u);
     const int nv_wr = ((lane >> 2) & 7) * 128 + (lane >> 5) * 1024;  // NV: this lane's row of the fragment in the buffer
-    const int nv_key = (lane >> 2) & 7, nv_piece = (lane & 3) * 2;
+    const int nv_key = lds_key(lane >> 2), nv_piece = (lane & 3) * 2;
     // block-scale rows: one per wave (its fragments sit inside one 128-row block), lane l keeps K block l (+64)
     const int srow = min(MODE == 0 ? t * (32 * NW) + wave * 32 : t * (64 * NW) + wave * 64, N - 16) >> 7;
     const float* sw0 = reinterpret_cast<const float*>(NV ? uint64_t(p.a_scales) : ws[0]) + (NV ? 0 : size_t(srow) * KB);  // NV: any readable floats, never used
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
       const int pos = start + min(m, n - 1);
       const int row = MODE == 0 && p.perm ? load_global<int>(p.perm + pos) / p.top_k : pos;
       tsrc[i] = p.a_codes + size_t(row) * K + c * 16;
-      tdst[i] = m * 128 + ((c ^ (m & 7)) << 4);
+      tdst[i] = m * 128 + ((c ^ lds_key(m)) << 4);
     }
     const bool stage_chunk = CHUNKS >= NT || tid < CHUNKS;
     const float* ssrc;
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
             nv_store(wl + f * 2048, w[0][f][0], wsc[0][f]);
           } else {
             *reinterpret_cast<u32x4*>(wl + f * 2048 + wr_off) = w[0][f][0];
-            *reinterpret_cast<u32x4*>(wl + f * 2048 + 1024 + wr_off) = w[0][f][1];
+            *reinterpret_cast<u32x4*>(wl + f * 2048 + 1024 + (wr_off ^ 64)) = w[0][f][1];
           }
         }
 #pragma unroll
@@ -329,8 +329,8 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
     // token address is one of three lane values plus a compile-time constant.
     static_assert(P % 2 == 0, "token buffer = stage parity");
     const int trow0 = lane & 15, q2 = (lane >> 4) * 2;
-    const int tlo0 = trow0 * 128 + (((q2) ^ (trow0 & 7)) << 4);
-    const int thi0 = trow0 * 128 + (((q2 + 1) ^ (trow0 & 7)) << 4);
+    const int tlo0 = trow0 * 128 + ((q2 ^ lds_key(trow0)) << 4);
+    const int thi0 = trow0 * 128 + (((q2 + 1) ^ lds_key(trow0)) << 4);
     const int tsx0 = TM * 128 + trow0 * 4;
 
     // 64-row groups keep LDS latency off the matrix core's path: the operand-order weight fragments of a stage are read at
@@ -432,12 +432,12 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
                     FF_REQUEST_WEIGHTS(s, kw, m);
                     wait_loads<CPT + 1 + 8>(w[o][m][0], w[o][m][1]);
                     *reinterpret_cast<u32x4*>(wl + m * 2048 + wr_off) = w[o][m][0];
-                    *reinterpret_cast<u32x4*>(wl + m * 2048 + 1024 + wr_off) = w[o][m][1];
+                    *reinterpret_cast<u32x4*>(wl + m * 2048 + 1024 + (wr_off ^ 64)) = w[o][m][1];
                   } else {
                     if (m & 1) load16_async(w[s][m >> 1][1], wfrag[m >> 1] + kw * 128u, woff1);
                     else load16_async(w[s][m >> 1][0], wfrag[m >> 1] + kw * 128u, woff0);
                     wait_loads<CPT + 1 + 8>(w[o][m >> 1][m & 1]);
-                    *reinterpret_cast<u32x4*>(wl + (m >> 1) * 2048 + (m & 1) * 1024 + wr_off) = w[o][m >> 1][m & 1];
+                    *reinterpret_cast<u32x4*>(wl + (m >> 1) * 2048 + (m & 1) * 1024 + (wr_off ^ 64 * (m & 1))) = w[o][m >> 1][m & 1];
                   }
                 }
               }
