@@ -8,11 +8,9 @@
 // the weights through registers into a wave-private transposition buffer and so passes 24 KB through LDS per 16 matrix
 // instructions; its cache-resident rate stays near 1.2 PFLOP/s. Here two waves share each operand half, nothing goes through
 // registers on its way in, and a wave's 16 instructions read 16 KB; the 32 KB of a K block are requested one K block ahead
-// and land while the previous one is multiplied. Two independent blocks per CU (66 KB of LDS each) cover each other's
-// barriers, first loads and epilogues. Measured: 4096 x 7168 -> 4096 in 142 us = 1.69 PFLOP/s (matrix cores busy 40 % of
-// the cycles at the 2.05 GHz the chip holds here), 2048 x 2048 -> 7168 66 -> 47 us. The same loop without its loads takes
-// 105 us. Not faster: 256 x 128 tiles with three stages and one block per CU (145 us), 256 x 256 tiles (144), the next K block's
-// operands read into registers under the matrix work (155).
+// and land while the previous one is multiplied. Two independent blocks per CU (72 KB of LDS each) cover each other's
+// barriers, first loads and epilogues. Measured, steady clocks: 4096 x 7168 -> 4096 in 122 us = 1.97 PFLOP/s (129 while a wave fetched its
+// 64 token scales per K block, a line look-up per token; 157 with that and bank conflicts in every operand read), 2048 x 2048 -> 7168 41 us.
 #pragma once
 #include "mx_gemm.cuh"
 #include "lds_load.cuh"
@@ -26,8 +24,9 @@ namespace ffmoe {
 // gate/up 142 -> 88 us, down 70 -> 39 us against 64-row units with the weights requested in operand order.
 template <int MODE, bool MX>
 __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
-  struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; float sx[4][64]; };
+  struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; };
   __shared__ __attribute__((aligned(16))) Stage stage[2];
+  __shared__ float sx_lds[2][128][8];  // token scales of eight K blocks
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int wr = wave >> 1, wt = wave & 1;
@@ -40,7 +39,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
   const uint32_t span_end = min(total, (xcd + 1u) * span);
   const uint32_t lds_w[2] = {lds_address(stage[0].w) + uint32_t(wave) * 4096u, lds_address(stage[1].w) + uint32_t(wave) * 4096u};
   const uint32_t lds_t[2] = {lds_address(stage[0].t) + uint32_t(wave) * 4096u, lds_address(stage[1].t) + uint32_t(wave) * 4096u};
-  const uint32_t lds_s[2] = {lds_address(stage[0].sx[wave]), lds_address(stage[1].sx[wave])};
+  const uint32_t lds_s = lds_address(sx_lds) + uint32_t(wave) * 1024u;
   const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ lds_key(lane >> 3)) << 4);  // odd requests: piece ^ 4
   // operand reads: row lane % 16, bytes 32 c .. 32 c + 31 of the K block for lane group c
   // (MX: bytes 16 c .. 16 c + 15 and 64 + 16 c .. 64 + 16 c + 15, the operand form whose scales sit in lane group column / 32)
@@ -64,11 +63,9 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       wbase[i] = uni64((MODE == 0 ? wc[f >> 1] : wc[0]) + uint64_t(min(column(wr, f), N - 16) + (i & 1) * 8) * uint64_t(K));
     }
     const uint8_t* tsrc[4];  // request i: token rows 32 wave + 8 i + lane / 8
-    const float* ssrc;       // the scales of this wave's 64 tokens
     auto token_row = [&](int m) { return start + min(m, n - 1); };
 #pragma unroll
     for (int i = 0; i < 4; ++i) tsrc[i] = p.a_codes + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * K + (((lane & 7) ^ lds_key(lane >> 3) ^ 4 * (i & 1)) << 4);
-    ssrc = p.a_scales + size_t(token_row(wt * 64 + lane)) * KB;  // MX: the four scale bytes of a K block are one word
     // Block scales, one word per K block; lane l keeps K block l (+ 64). A wave's columns sit inside one 128-row block; MX: four
     // bytes per 32 rows, which are the wave's fragments 0, 1 and its fragments 2, 3.
     const float* sw0 = reinterpret_cast<const float*>(ws[0]) + size_t(min(column(wr, 0), N - 16) >> (MX ? 5 : 7)) * KB;
@@ -79,7 +76,13 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       for (int i = 0; i < 4; ++i) lds_load16(lds_w[b] + i * 1024u, wbase[i] + uint64_t(uint32_t(kb) * 128u), woff ^ (64u * (i & 1)));
 #pragma unroll
       for (int i = 0; i < 4; ++i) lds_load16(lds_t[b] + i * 1024u, tsrc[i] + uint32_t(kb) * 128u);
-      lds_load4(lds_s[b], ssrc + kb);
+      // Token scales, a row of KB words per token (MX: the four scale bytes of a K block are one word): a request takes eight K blocks of
+      // eight tokens. One K block of 64 tokens per request touches a line per lane, as many line look-ups as the operands themselves.
+      if ((kb & 7) == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          lds_load4(lds_s + uint32_t((kb >> 3) & 1) * 4096u + i * 256u, p.a_scales + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * KB + min(kb + (lane & 7), KB - 1));
+      }
     };
     __syncthreads();  // the previous unit's last tile has been read
     request(0, 0);
@@ -98,7 +101,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       if (kb + 1 < KB) request(kb + 1, b ^ 1);
       const uint8_t* wl = stage[b].w + wr * 8192;
       const uint8_t* tl = stage[b].t + wt * 8192;
-      const float* sl = stage[b].sx[wave] + r16;
+      const float* sl = &sx_lds[(kb >> 3) & 1][wt * 64 + r16][kb & 7];
       v8i wf[4];
 #pragma unroll
       for (int f = 0; f < 4; ++f) {
@@ -108,7 +111,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       u32x4 tlo[2], thi[2];
       float sx[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) sx[m] = sl[16 * m];
+      for (int m = 0; m < 4; ++m) sx[m] = sl[16 * 8 * m];
       tlo[0] = *reinterpret_cast<const u32x4*>(tl + rd_lo);
       thi[0] = *reinterpret_cast<const u32x4*>(tl + rd_hi);
       if constexpr (MX) {
