@@ -506,7 +506,22 @@ bool use_tiles(int mode, int rows, int n, int k, bool mx = false) {
   const long long columns = (n + (mode == 0 ? 127 : 255)) / (mode == 0 ? 128 : 256);
   return mx || (rows + 63) / 64 * columns > cus || (tiles <= cus && (k > 1536 ? 12 : 18) * columns > cus);
 }
+// The 256 x 256 tile kernel (FFMOE_W8A8_WIDE: 1 wherever the tiles are used, 0 never; same bits) takes 1.83 us per K block and round of one
+// tile per CU, the 128 x 128 one 1.09 per round of two tiles per CU, and its start and end are longer: it wants rounds of the small tiles
+// to fall from at least 8 to 5. 2048 x 2048 -> 7168 (2 rounds to 1) 41.1 -> 32.3 us, 4096 x 2048 -> 7168 (4 to 2) 69.5 -> 62.2; 1024 x 7168 ->
+// 7168 (1 to 1) 59.8 against 85.1. Its token addresses are 32-bit offsets.
+bool use_wide(int mode, const GemmParams& p) {
+  if (uint64_t(p.rows_total) * uint64_t(p.K) >= (uint64_t(1) << 32)) return false;
+  if (const char* f = getenv("FFMOE_W8A8_WIDE")) return atoi(f) != 0;
+  const uint32_t cus = uint32_t(num_cus_p());
+  const uint32_t small = (tile_units(mode, p.rows_total, p.N) + 2 * cus - 1) / (2 * cus), large = (wide_units(mode, p.rows_total, p.N) + cus - 1) / cus;
+  return 5 * small >= 8 * large;
+}
 int launch_tiles(int mode, GemmParams& p, hipStream_t stream, bool mx = false) {
+  if (!mx && use_wide(mode, p)) {
+    p.total_units = wide_units(mode, p.rows_total, p.N);
+    return launch_w8a8_wide(mode, p, std::min<unsigned>((p.total_units + 7u) & ~7u, unsigned(num_cus_p()) & ~7u), stream);
+  }
   p.total_units = tile_units(mode, p.rows_total, p.N);
   const unsigned blocks = std::min<unsigned>((p.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u);
   return mx ? launch_mx_dense_tile(mode, p, blocks, stream) : launch_w8a8_tile(mode, p, blocks, stream);

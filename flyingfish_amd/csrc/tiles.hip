@@ -1,5 +1,6 @@
-// Launches of the kernels whose operand tiles go straight to LDS (tile_gemm.cuh, mx_tile.cuh, nvfp4_tile.cuh)
+// Launches of the kernels whose operand tiles go straight to LDS (tile_gemm.cuh, wide_gemm.cuh, mx_tile.cuh, nvfp4_tile.cuh)
 #include "tile_gemm.cuh"
+#include "wide_gemm.cuh"
 #include "mx_tile.cuh"
 #include "nvfp4_tile.cuh"
 #include "tiles.h"
@@ -16,6 +17,17 @@ int launch_mx_dense_tile(int mode, const GemmParams& p, unsigned blocks, hipStre
   if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, true>), dim3(blocks), dim3(256), 0, stream, p);
   else hipLaunchKernelGGL((k_w8a8_tile<2, true>), dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
+}
+
+template <int MODE>
+static int launch_wide(const GemmParams& p, unsigned blocks, hipStream_t stream) {
+  static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_w8a8_wide<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, WIDE_LDS);
+  if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", WIDE_LDS, hipGetErrorString(ok));
+  hipLaunchKernelGGL(k_w8a8_wide<MODE>, dim3(blocks), dim3(512), WIDE_LDS, stream, p);
+  return ff_launch_status();
+}
+int launch_w8a8_wide(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
+  return mode == 0 ? launch_wide<0>(p, blocks, stream) : launch_wide<2>(p, blocks, stream);
 }
 
 template <int MODE>

@@ -72,6 +72,39 @@ def test_prefill_shared_expert_tile_kernel_equals_the_group_kernel_bitwise(rows,
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 16, 128), (255, 144, 256), (257, 272, 384), (130, 272, 8320), (300, 1168, 1024), (600, 528, 1152), (4200, 4400, 128)])
+def test_linear_w8a8_wide_tile_kernel_equals_the_tile_kernel_bitwise(m, n, k, monkeypatch):
+    """Ragged rows and columns, one K block, two, the ends of a fetch of eight token scales, more tiles than CUs."""
+    wc, ws = _fp8_matrix(n, k, m * 5 + n)
+    x = synth.normal((m, k), 1.0, 3 + m, dtype=torch.bfloat16)
+    monkeypatch.setenv("FFMOE_W8A8_TILE", "1")
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_WIDE", switch)
+        out.append(ops.Fp8Ops.linear(wc.cuda(), ws.cuda(), x.cuda(), capi.ACT_FP8_BLOCK128))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,inter", [(65, 128), (300, 384)])
+def test_prefill_shared_expert_wide_tile_kernel_equals_the_tile_kernel_bitwise(rows, inter, monkeypatch):
+    table, _ = make_table(capi.FMT_FP8_BLOCK128, 4, 256, inter, 79)
+    shared = table.shared_struct(3)
+    table.experts = 3
+    x = synth.normal((rows, 256), 1.0, 80).to(torch.bfloat16).cuda()
+    ids = torch.randint(0, 3, (rows, 1), generator=torch.Generator().manual_seed(5)).to(torch.int32).cuda()
+    w = torch.rand((rows, 1), generator=torch.Generator().manual_seed(6)).cuda()
+    monkeypatch.setenv("FFMOE_W8A8_TILE", "1")
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_WIDE", switch)
+        op = ops.PrefillOps(table, rows, 1, shared=shared)
+        op.contribute(x, ids, w)
+        torch.cuda.synchronize()
+        out.append(op.shared_out.clone())
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
 def test_linear_w8a8_device_quantizer_chain():
     """ffmoe_linear_fp8_block(act_mode = FP8_BLOCK128) = device quantizer + W8A8 linear."""
     m, n, k = 9, 256, 640
