@@ -2,6 +2,7 @@
 // (W8A16 / W4A16 arithmetic: BF16-rounded effective weights, FP32 accumulation, BF16 output),
 // the per-128 E4M3 activation quantizer and the elementwise SwiGLU.
 #include "gemv.cuh"
+#include "lds_load.cuh"
 #include "api.h"
 #include <cstdlib>
 
@@ -297,6 +298,102 @@ __global__ __launch_bounds__(512) void k_linear_mfma(const LinearParams p, int m
   }
 }
 
+// The block-FP8 linear for more than four rows, K a multiple of 128: TR weight rows x 16 tokens per block of eight waves that split the
+// contraction, arithmetic of k_linear_mfma.
+//
+// What bounds it: not the weights (14.7 MB are 2.3 us) but the way of 16 token rows into every CU, 229 KB at K 7168, and the
+// round trips in front of the matrix work. k_linear_mfma copies the tokens through registers into a panel that the block shares, half
+// of them at a time, with a barrier and a latency in front of each: 13.5 us for 16 x 7168 -> 2048. A wave's share of the tokens is its
+// own, so nothing needs sharing: here each wave moves its K blocks of tokens and weights straight into a ring of its own in LDS
+// (D blocks, 160 KB per CU in flight at once) and waits by count; the only barrier is the one in front of the eight partial sums.
+// us per call, weights cold, against k_linear_mfma (7.5 us of either is a call's way through the host): 16 rows 7168 -> 2048 13.6 -> 7.8,
+// 7168 -> 7168 28.8 -> 13.0, 4096 -> 4096 12.4 -> 7.7; 64 rows (four launches there) 7168 -> 2048 54 -> 11.0, 7168 -> 7168 115 -> 44.5.
+// LDS: token row r 256 bytes, 16-byte piece c at c ^ r ^ (r & 4) << 1; weight row r 128 bytes, piece c at c ^ lds_key(r).
+template <int TR>
+__global__ __launch_bounds__(512) void k_linear_fp8_split(const LinearParams p) {
+  constexpr int NW = 8, NF = TR > 16 ? TR / 16 : 1, WREQ = TR / 8, REQ = 4 + WREQ;  // requests of a wave per K block
+  constexpr int BYTES = 4096 + TR * 128, D = TR == 8 ? 4 : TR == 16 ? 3 : 2;
+  extern __shared__ __align__(16) uint8_t lds[];
+  static_assert(NW * D * BYTES <= 160 * 1024, "one block per CU");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int K = p.k, N = p.n, KB = K >> 7;
+  const int n0 = blockIdx.x * TR, m0 = blockIdx.y * 16;
+  const int mcount = min(16, p.m - m0);
+  const int i = lane & 15, c = lane >> 4;
+  const int mine = (KB - wave + NW - 1) / NW;  // K blocks wave, wave + 8, ..; none when there are fewer than waves
+  const uint32_t ring = lds_address(lds) + uint32_t(wave) * (D * BYTES);
+  uint32_t toff[4];  // request q: token rows 4 q + lane / 16 (rows past the last one repeat it and are dropped at the store)
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = 4 * q + c;
+    toff[q] = uint32_t(min(r, mcount - 1)) * uint32_t(K) * 2u + uint32_t((i ^ r ^ (r & 4) << 1) << 4);
+  }
+  const uint64_t xbase = uint64_t(uintptr_t(p.x)) + uint64_t(m0) * uint64_t(K) * 2u;
+  const uint64_t wbase = p.codes + uint64_t(n0) * uint64_t(K);
+  const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ lds_key(lane >> 3)) << 4);  // odd requests: rows + 8, piece ^ 4
+  const float* scales = reinterpret_cast<const float*>(p.scales) + size_t(n0 >> 7) * KB;
+  auto request = [&](int j) {
+    const uint32_t kb = uint32_t(wave + NW * j), at = ring + uint32_t(j % D) * BYTES;
+#pragma unroll
+    for (int q = 0; q < WREQ; ++q) lds_load16_nt(at + 4096u + q * 1024u, wbase + uint64_t(8 * q) * uint64_t(K) + kb * 128u, woff ^ (64u * (q & 1)));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) lds_load16(at + q * 1024u, xbase + kb * 256u, toff[q]);
+  };
+  f32x4 acc[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int j = 0; j < D; ++j)
+    if (j < mine) request(j);
+  const int xkey = i ^ (i & 4) << 1;
+  for (int j = 0; j < mine; ++j) {
+    const float s = load_uniform<float>(scales + wave + NW * j);
+    const int younger = mine - 1 - j;  // K blocks requested behind this one
+    if (younger >= D - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * REQ) : "memory");
+    else if (D > 3 && younger == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * REQ) : "memory");
+    else if (D > 2 && younger == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(REQ) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const uint8_t* xb = lds + wave * (D * BYTES) + (j % D) * BYTES + i * 256;
+    const uint8_t* wb = lds + wave * (D * BYTES) + (j % D) * BYTES + 4096;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {  // columns 64 h + 16 c .. + 15
+      const u32x4 b0 = *reinterpret_cast<const u32x4*>(xb + (((8 * h + 2 * c) ^ xkey) << 4));
+      const u32x4 b1 = *reinterpret_cast<const u32x4*>(xb + (((8 * h + 2 * c + 1) ^ xkey) << 4));
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const int r = 16 * f + (i & (TR - 1));
+        const u32x4 codes = *reinterpret_cast<const u32x4*>(wb + r * 128 + (((4 * h + c) ^ lds_key(r)) << 4));
+        uint32_t w[8];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) dequant4_e4m3(codes[q], s, w[2 * q], w[2 * q + 1]);
+        const u32x4 a0 = {w[0], w[1], w[2], w[3]}, a1 = {w[4], w[5], w[6], w[7]};
+        acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a0), __builtin_bit_cast(bf16x8_t, b0), acc[f], 0, 0, 0);
+        acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a1), __builtin_bit_cast(bf16x8_t, b1), acc[f], 0, 0, 0);
+      }
+    }
+    if (j + D < mine) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block has been read: its place is free
+      request(j + D);
+    }
+  }
+  // lane (token i, group c) holds weight rows 4 c .. 4 c + 3 of a fragment; the waves' tiles are added in wave order
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(lds);  // [wave][row][token]
+#pragma unroll
+  for (int f = 0; f < NF; ++f)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[((wave * NF + f) * 16 + 4 * c + r) * 16 + i] = acc[f][r];
+  __syncthreads();
+  for (int t = tid; t < 16 * TR; t += 512) {
+    const int j = t / TR, r = t - j * TR;
+    float v = red[r * 16 + j];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v = __fadd_rn(v, red[(w * NF * 16 + r) * 16 + j]);
+    if (j < mcount) p.y[size_t(m0 + j) * N + n0 + r] = f32_to_bf16(v);
+  }
+}
+
 // Per (row, 128-group): scale = amax * (1/448), code = e4m3(clamp(x / max(scale, 1e-12), +-448))
 // (kernels/fp8_linear.cu:12-48 of the reference). One wave per 4 cells, 16 lanes x 8 elements per cell.
 __global__ __launch_bounds__(256) void k_quant_fp8_128(const uint16_t* __restrict__ x, uint8_t* __restrict__ codes,
@@ -422,6 +519,26 @@ int launch_linear_mfma(const LinearParams& p, hipStream_t st) {
   return ff_launch_status();
 }
 
+template <int TR>
+int launch_linear_split_rows(const LinearParams& p, hipStream_t st) {
+  constexpr int lds = 8 * (TR == 8 ? 4 : TR == 16 ? 3 : 2) * (4096 + TR * 128);
+  static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_linear_fp8_split<TR>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", lds, hipGetErrorString(ok));
+  hipLaunchKernelGGL(k_linear_fp8_split<TR>, dim3(p.n / TR, (p.m + 15) / 16), dim3(512), lds, st, p);
+  return ff_launch_status();
+}
+// Weight rows per block: what a CU moves is 32 bytes of tokens and TR bytes of weights per column and block, so the fewest rounds of blocks
+// over the chip times that (7168 -> 2048, 16 rows with 8 / 16 / 32: 7.8 / 8.5 / 11.4 us; 64 rows 26.0 / 15.2 / 11.0).
+int launch_linear_split(const LinearParams& p, hipStream_t st) {
+  const long long cus = num_cus_l(), mb = (p.m + 15) / 16;
+  auto cost = [&](int tr) { return p.n % tr != 0 ? ~0ull >> 1 : (unsigned long long)((p.n / tr * mb + cus - 1) / cus * (32 + tr)); };
+  int tr = 8;
+  if (cost(16) < cost(tr)) tr = 16;
+  if (cost(32) < cost(tr)) tr = 32;
+  if (const char* e = getenv("FFMOE_LINEAR_ROWS")) { const int v = atoi(e); if ((v == 8 || v == 16 || v == 32) && p.n % v == 0) tr = v; }
+  return tr == 32 ? launch_linear_split_rows<32>(p, st) : tr == 16 ? launch_linear_split_rows<16>(p, st) : launch_linear_split_rows<8>(p, st);
+}
+
 int check_linear(const void* w, const void* x, const void* y, int m, int n, int k, int kgran) {
   FF_REQUIRE(m >= 1 && n >= 1 && k >= kgran && k % kgran == 0, FFMOE_ERR_SHAPE, "linear m=%d n=%d k=%d (k must be a positive multiple of %d)", m, n, k, kgran);
   FF_REQUIRE(size_t(k) * 2 <= 64 * 1024, FFMOE_ERR_SHAPE, "linear k=%d exceeds the LDS row staging (32768)", k);
@@ -459,7 +576,10 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_linear_fp8_block(con
   }
   FF_REQUIRE(act_mode == FFMOE_ACT_BF16, FFMOE_ERR_UNSUPPORTED, "unknown act_mode %d", act_mode);
   LinearParams p{(const uint16_t*)x, (uint16_t*)y, (uint64_t)(uintptr_t)w_codes, (uint64_t)(uintptr_t)w_scales, nullptr, m, n, k};
-  if (m > 4 && n % 16 == 0 && mfma_linear_fits<FmtFp8>(k)) return launch_linear_mfma<FmtFp8>(p, (hipStream_t)stream);
+  if (m > 4 && n % 16 == 0 && mfma_linear_fits<FmtFp8>(k)) {
+    if (k % 128 == 0 && !getenv("FFMOE_LINEAR_NO_SPLIT") && m <= 16 * 65535) return launch_linear_split(p, (hipStream_t)stream);
+    return launch_linear_mfma<FmtFp8>(p, (hipStream_t)stream);
+  }
   return launch_linear<FmtFp8>(p, (hipStream_t)stream);
 }
 

@@ -649,6 +649,26 @@ def test_linear_fp8_block_matrix_core_path(m, k, n):
     assert orc.rel_l2(y, y2) < 1e-3
 
 
+@pytest.mark.parametrize("rows", ["8", "16", "32"])
+@pytest.mark.parametrize("m,k,n", [
+    (5, 128, 32),      # one K block for eight waves
+    (16, 1152, 160),   # nine K blocks: one wave takes two; more than one scale row
+    (17, 4224, 64),    # 33 K blocks, past every ring's length, a second token block of one row
+    (64, 7168, 32),
+])
+def test_linear_fp8_block_split_kernel_edges(m, k, n, rows, monkeypatch):
+    """Every number of weight rows per block against the FP64 sum and against the panel kernel (another order of the same sum)."""
+    w = synth.normal((n, k), 0.02, 720 + m)
+    codes, scales = synth.quant_fp8_block(w)
+    x = rand_bf16((m, k), 1.0, 730 + m)
+    monkeypatch.setenv("FFMOE_LINEAR_ROWS", rows)
+    y = bits(Fp8Ops.linear(codes.to(DEV), scales.to(DEV), x.to(DEV)))
+    assert_close_bf16(y, orc.linear_skinny(orc.dequant_fp8_block(codes.numpy(), scales.numpy()), bits(x), 2), "fp8 linear (split) vs f64")
+    monkeypatch.setenv("FFMOE_LINEAR_NO_SPLIT", "1")
+    y2 = bits(Fp8Ops.linear(codes.to(DEV), scales.to(DEV), x.to(DEV)))
+    assert orc.rel_l2(y, y2) < 1e-3
+
+
 @pytest.mark.parametrize("m,k,n", [(40, 2048, 192), (17, 3712, 48), (21, 128, 4096)])
 def test_linear_nvfp4_and_bf16_matrix_core_path(m, k, n):
     """NVFP4 beyond 16 rows (the reference switches to its MMA kernel there, nvfp4_linear.cu:262-573, bounded by
