@@ -124,6 +124,40 @@ __device__ __forceinline__ float det_expf(float x) {
   return y;
 }
 
+// The same for x <= 0, without branches; a NaN stays one.
+__device__ __forceinline__ float det_expf_neg(float x) {
+  const float magic = 12582912.0f;
+  const float c = fmaxf(x, -105.0f);  // in range for the arithmetic; the result is replaced below
+  const float t = __fmaf_rn(c, 1.44269502162933349609375f, magic);
+  const float n = __fsub_rn(t, magic);
+  float r = __fmaf_rn(n, -0.693145751953125f, c);
+  r = __fmaf_rn(n, -1.428606765330187045037746429443359375e-06f, r);
+  float p = 1.9875691500e-4f;
+  p = __fmaf_rn(p, r, 1.3981999507e-3f);
+  p = __fmaf_rn(p, r, 8.3334519073e-3f);
+  p = __fmaf_rn(p, r, 4.1665795894e-2f);
+  p = __fmaf_rn(p, r, 1.6666665459e-1f);
+  p = __fmaf_rn(p, r, 5.0000001201e-1f);
+  float y = __fmaf_rn(p, __fmul_rn(r, r), r);
+  y = __fadd_rn(y, 1.0f);
+  // n from the low bits of t: t = 1.5 * 2^23 + n
+  const int ni = int(__float_as_uint(t)) - 0x4b400000;
+  const int a = ni >> 1;
+  y = __fmul_rn(y, __uint_as_float(uint32_t(a + 127) << 23));
+  y = __fmul_rn(y, __uint_as_float(uint32_t(ni - a + 127) << 23));
+  return x > -104.0f ? y : 0.0f;
+}
+// n / d correctly rounded for d in [1, 2] and n = 1 or n = d - 1 before its rounding: reciprocal, one Newton step, and the quotient
+// corrected twice by its exact remainder (Markstein). No operand needs scaling: where n is too small for an exact remainder, d is 1
+// and the quotient n itself.
+__device__ __forceinline__ float div_by_1_to_2(float n, float d) {
+  float y = __builtin_amdgcn_rcpf(d);
+  y = __fmaf_rn(__fmaf_rn(-d, y, 1.0f), y, y);
+  float q = __fmul_rn(n, y);
+  q = __fmaf_rn(__fmaf_rn(-d, q, n), y, q);
+  return __fmaf_rn(__fmaf_rn(-d, q, n), y, q);
+}
+
 // log(1+u), 0 <= u <= 1.
 __device__ __forceinline__ float det_log1pf_unit(float u) {
   const float w = __fadd_rn(1.0f, u);
@@ -183,11 +217,12 @@ __device__ __forceinline__ float gelu_tanh(float g) {
 // SiLU as x * sigmoid(x) with the two-branch sigmoid of the reference's dense activation kernels
 // (kernels/q38_contract.cuh:17-21, kernels/act.cu:152-156).
 __device__ __forceinline__ float silu_two_branch(float g) {
-  // both branches are exp(-|g|) and a quotient over 1 + exp(-|g|): one of each instead of two under divergence (a 4096 x 7168 gate/up
-  // product on 256 x 256 tiles 117 -> 112 us)
+  // Both branches are exp(-|g|) and a quotient over 1 + exp(-|g|): one of each instead of two under divergence (a 4096 x 7168 gate/up
+  // product on 256 x 256 tiles 117 -> 112 us).
   const bool pos = g >= 0.0f;
-  const float e = det_expf(pos ? -g : g);
-  return __fmul_rn(g, __fdiv_rn(pos ? 1.0f : e, __fadd_rn(1.0f, e)));
+  const float e = det_expf_neg(pos ? -g : g);
+  const float y = __fmul_rn(g, div_by_1_to_2(pos ? 1.0f : e, __fadd_rn(1.0f, e)));
+  return g == g ? y : __fadd_rn(g, g);  // the remainders negate a NaN
 }
 __device__ __forceinline__ uint16_t swiglu_bf16_two_branch(float g, float u, int mode, float limit) {
   if (mode >= 2) {
