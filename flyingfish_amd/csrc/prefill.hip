@@ -24,7 +24,7 @@ struct PrefillBook {
   uint32_t* counts;   // [E]
   uint32_t* offsets;  // [E + 1]
   uint32_t* gbase;    // [E + 1] first group of each expert
-  uint32_t* totals;   // [0] units of the gate/up GEMM, [1] units of the down GEMM, [2] groups, [3] active assignments
+  uint32_t* totals;   // [0] units of the gate/up GEMM, [1] units of the down GEMM, [2] groups, [3] active assignments, [4] groups of 256 rows; [8 + 16 s + x]: claims of stage s on span x
   int* perm;          // [A]
   GemmGroup* groups;
   u32x2* units0;
@@ -73,24 +73,58 @@ __global__ __launch_bounds__(256) void k_prefill_count(const LiveTest t, uint32_
 // shared_rows > 0 appends the always-on expert as groups of expert id `experts` over rows 0 .. shared_rows - 1, their units
 // behind the routed ones (column tile outermost, so the row groups of a tile are neighbours and share its weights in L2):
 // the launches that run the routed experts then run the shared one as well.
+// Row groups of an expert with c rows: of tm rows, or (tm == 0) of 256 rows while more than 128 are left and of 64 rows for the rest. A
+// 256-row tile takes 3500 cycles per K block whatever its group holds, a 64-row group 2100 to 2600 (its share of the weight stream, or less where
+// it follows another of its expert): 4096 tokens 3.70 ms, with 64-row groups up to 192 rows 3.88.
+// The 256-row groups of all experts come first in the group and unit lists, the 64-row groups behind them; an expert's two counts share a
+// word (at most two small groups per expert), and so do their prefix sums.
+constexpr uint32_t SMALL_BITS = 12;
+static_assert(2 * FFMOE_MAX_EXPERTS < (1 << SMALL_BITS), "prefix sums of the small groups");
+__device__ __forceinline__ uint32_t big_groups(uint32_t c) { return (c + 127u) / 256u; }
+__device__ __forceinline__ uint32_t group_count(uint32_t c, int tm) {
+  if (tm > 0) return (c + tm - 1) / tm;
+  const uint32_t big = big_groups(c);
+  return (big << SMALL_BITS) | (big * 256u >= c ? 0u : (c - big * 256u + 63u) / 64u);
+}
+// first row (of the expert's) and rows of group q among `total` groups, its expert and that expert's first row
+__device__ __forceinline__ GemmGroup group_of(const uint32_t* s_rows, const uint32_t* s_groups, int experts, int tm, uint32_t q) {
+  const uint32_t big_total = tm > 0 ? 0u : s_groups[experts] >> SMALL_BITS;
+  const bool big = q < big_total;
+  const uint32_t key = q - (big ? 0u : big_total);
+  auto field = [&](uint32_t v) { return tm > 0 ? v : big ? v >> SMALL_BITS : v & ((1u << SMALL_BITS) - 1u); };
+  int lo = 0, hi = experts;  // last e with its first group <= key
+  while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (field(s_groups[mid]) <= key) lo = mid; else hi = mid; }
+  const uint32_t i = key - field(s_groups[lo]), c = s_rows[lo + 1] - s_rows[lo];
+  const uint32_t size = tm > 0 ? uint32_t(tm) : big ? 256u : 64u;
+  const uint32_t first = (tm > 0 || big ? 0u : big_groups(c) * 256u) + i * size;
+  GemmGroup gd;
+  gd.expert = lo; gd.start = int(s_rows[lo] + first); gd.n = int(min(size, c - first)); gd.pad = 0;
+  return gd;
+}
+__device__ __forceinline__ uint32_t group_total(uint32_t packed, int tm) { return tm > 0 ? packed : (packed >> SMALL_BITS) + (packed & ((1u << SMALL_BITS) - 1u)); }
+
 struct PlanShared { uint32_t rows[1025], groups[1025], tmp[1024]; };
 
 // unit u of a list with `tiles` column tiles per group -> (group, tile); s_groups = exclusive scan of the experts' group
 // counts, G routed groups, GS groups of the riding shared expert behind them
-__device__ __forceinline__ u32x2 plan_unit(const uint32_t* s_groups, int experts, uint32_t tiles, int rgb, int tgb, uint32_t G, uint32_t GS, uint32_t u) {
+__device__ __forceinline__ u32x2 plan_unit(const uint32_t* s_groups, int experts, int tm, uint32_t tiles, int rgb, int tgb, uint32_t G, uint32_t GS, uint32_t u) {
   if (u >= G * tiles) {
     const uint32_t v = u - G * tiles;
     return u32x2{G + v % GS, v / GS};
   }
-  const uint32_t key = u / tiles;
-  int lo = 0, hi = experts;  // last e with s_groups[e] <= key
-  while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (s_groups[mid] <= key) lo = mid; else hi = mid; }
+  const uint32_t big_total = tm > 0 ? 0u : s_groups[experts] >> SMALL_BITS;
+  const bool big = u < big_total * tiles;
+  const uint32_t base = big ? 0u : big_total;  // first group of the list's part
+  auto field = [&](uint32_t v) { return tm > 0 ? v : big ? v >> SMALL_BITS : v & ((1u << SMALL_BITS) - 1u); };
+  const uint32_t key = u / tiles - base;
+  int lo = 0, hi = experts;  // last e with its first group <= key
+  while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (field(s_groups[mid]) <= key) lo = mid; else hi = mid; }
   // An expert's units run over blocks of rgb row groups, inside a row block over blocks of tgb column tiles, inside those
   // over the tiles, innermost over the row groups. The blocks of an XCD work on neighbouring units at the same time (64 of
   // them with two blocks per CU), so a window of rgb x tgb units fetches rgb token tiles and tgb weight tiles into that
   // XCD's L2 and shares each among tgb resp. rgb blocks.
-  const uint32_t ge = s_groups[lo + 1] - s_groups[lo];
-  const uint32_t v = u - s_groups[lo] * tiles;
+  const uint32_t g0 = field(s_groups[lo]), ge = field(s_groups[lo + 1]) - g0;
+  const uint32_t v = u - (base + g0) * tiles;
   const uint32_t per = uint32_t(rgb) * tiles;
   const uint32_t j = min(v / per, (ge - 1u) / uint32_t(rgb));
   const uint32_t w = v - j * per;
@@ -99,7 +133,7 @@ __device__ __forceinline__ u32x2 plan_unit(const uint32_t* s_groups, int experts
   const uint32_t per2 = rb * tg;
   const uint32_t q = min(w / per2, (tiles - 1u) / tg);
   const uint32_t w2 = w - q * per2;
-  return u32x2{s_groups[lo] + j * uint32_t(rgb) + w2 % rb, q * tg + w2 / rb};
+  return u32x2{base + g0 + j * uint32_t(rgb) + w2 % rb, q * tg + w2 / rb};
 }
 
 __device__ __forceinline__ void prefill_plan_body(PlanShared& sh, const PrefillBook& b, int experts, int tm, int tiles0, int tiles1, int rgb,
@@ -108,7 +142,7 @@ __device__ __forceinline__ void prefill_plan_body(PlanShared& sh, const PrefillB
   uint32_t* s_groups = sh.groups;
   uint32_t* s_tmp = sh.tmp;
   const int tid = threadIdx.x;
-  const uint32_t g = (c + tm - 1) / tm;
+  const uint32_t g = group_count(c, tm);
   // Inclusive scans of the row and group counts over the block's 1024 threads: inside each wave by six cross-lane steps,
   // then the sixteen wave totals by the first wave, two barriers for both scans (forty barrier pairs as a block-wide
   // Hillis-Steele scan, which was most of this block's time)
@@ -139,8 +173,10 @@ __device__ __forceinline__ void prefill_plan_body(PlanShared& sh, const PrefillB
   __syncthreads();
   if (tid < experts) { b.offsets[tid] = s_rows[tid]; b.gbase[tid] = s_groups[tid]; }
   if (tid == 0) { b.offsets[experts] = s_rows[experts]; b.gbase[experts] = s_groups[experts]; }
-  const uint32_t G = s_groups[experts];
+  const uint32_t G = group_total(s_groups[experts], tm);
   const uint32_t GS = shared_rows > 0 ? uint32_t((shared_rows + tm - 1) / tm) : 0u;
+  if (tid < 32) b.totals[8 + tid] = 0u;
+  if (tid == 32) b.totals[4] = tm > 0 ? 0u : s_groups[experts] >> SMALL_BITS;
   if (tid == 0) { b.totals[0] = (G + GS) * tiles0; b.totals[1] = (G + GS) * tiles1; b.totals[2] = G; b.totals[3] = s_rows[experts]; }
   for (uint32_t q = tid; q < GS; q += 1024) {
     GemmGroup gd;
@@ -148,21 +184,13 @@ __device__ __forceinline__ void prefill_plan_body(PlanShared& sh, const PrefillB
     b.groups[G + q] = gd;
   }
   // group descriptors
-  for (uint32_t q = tid; q < G; q += 1024) {
-    int lo = 0, hi = experts;  // last e with s_groups[e] <= q
-    while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (s_groups[mid] <= q) lo = mid; else hi = mid; }
-    const uint32_t i = q - s_groups[lo];
-    const uint32_t cnt = s_rows[lo + 1] - s_rows[lo];
-    GemmGroup gd;
-    gd.expert = lo; gd.start = int(s_rows[lo] + i * tm); gd.n = int(min(uint32_t(tm), cnt - i * tm)); gd.pad = 0;
-    b.groups[q] = gd;
-  }
+  for (uint32_t q = tid; q < G; q += 1024) b.groups[q] = group_of(s_rows, s_groups, experts, tm, q);
   // unit lists
   if (!with_units) return;
   for (int pass = 0; pass < 2; ++pass) {
     const uint32_t tiles = pass == 0 ? tiles0 : tiles1;
     u32x2* units = pass == 0 ? b.units0 : b.units1;
-    for (uint32_t u = tid; u < (G + GS) * tiles; u += 1024) units[u] = plan_unit(s_groups, experts, tiles, rgb, tgb, G, GS, u);
+    for (uint32_t u = tid; u < (G + GS) * tiles; u += 1024) units[u] = plan_unit(s_groups, experts, tm, tiles, rgb, tgb, G, GS, u);
   }
 }
 
@@ -181,10 +209,10 @@ __global__ __launch_bounds__(256) void k_prefill_units(PrefillBook b, int expert
   for (int e = threadIdx.x; e <= experts; e += 256) s_groups[e] = b.gbase[e];
   __syncthreads();
   if (u >= n0 + n1) return;
-  const uint32_t G = s_groups[experts];
+  const uint32_t G = group_total(s_groups[experts], tm);
   const uint32_t GS = shared_rows > 0 ? uint32_t((shared_rows + tm - 1) / tm) : 0u;
-  if (u < n0) b.units0[u] = plan_unit(s_groups, experts, uint32_t(tiles0), rgb, tgb, G, GS, u);
-  else b.units1[u - n0] = plan_unit(s_groups, experts, uint32_t(tiles1), rgb, tgb, G, GS, u - n0);
+  if (u < n0) b.units0[u] = plan_unit(s_groups, experts, tm, uint32_t(tiles0), rgb, tgb, G, GS, u);
+  else b.units1[u - n0] = plan_unit(s_groups, experts, tm, uint32_t(tiles1), rgb, tgb, G, GS, u - n0);
 }
 
 // Small cohorts (at most FFMOE_BOOK_SMALL_MAX assignments, one per thread): count, plan and stable fill in ONE launch of one
@@ -535,6 +563,28 @@ int launch_tiles(int mode, const MxParams& q, hipStream_t stream) {
   return launch_tiles(mode, p, stream, true);
 }
 
+// A W8A8 prompt chunk's routed experts on the cohort kernel (wide_gemm.cuh; FFMOE_W8A8_COHORT: 1 wherever it can run, 0 never; same bits).
+// Its units are large and a CU runs one at a time: it wants contractions that outlast a unit's start and end (about ten K blocks of time)
+// and enough units per CU. us per layer, 64-row kernel / this one, Zipf-like routing:
+//   rows                              65            128           256           512           1024          4096
+//   top-8 of 256, 7168 / 2048    1022 /  935   1425 / 1266   1649 / 1475   2014 / 1875   2347 / 2184   4027 / 3634
+//   top-6 of 64, 4096 / 1536      311 /  283    336 /  315    354 /  345    413 /  376    504 /  482   1100 /  985
+//   top-8 of 128, 2048 / 1408     181 /  176    200 /  199    253 /  237    320 /  295    398 /  344
+//   top-6 of 64, 3072 / 1024      188 /  187    203 /  206    242 /  228    264 /  246    341 /  303     (2.0 - 2.8 gate/up units per CU)
+//   top-4 of 64, 4096 / 768       188 /  192    200 /  205    223 /  238    242 /  267    306 /  289     (1.6 - 1.9)
+//   top-8 of 256, 2048 / 768      136 /  157    150 /  172    200 /  197    232 /  233    309 /  300     (16 and 6 K blocks)
+// The group sizes and orders that the environment asks for are the 64-row kernel's.
+bool use_cohort(int rows, int top_k, int experts, int hidden, int inter) {
+  const uint64_t A = uint64_t(rows) * uint64_t(top_k), limit = uint64_t(1) << 32;
+  if (uint64_t(rows) * uint64_t(hidden) >= limit || A * uint64_t(inter) >= limit) return false;  // token addresses are 32-bit offsets
+  if (A >= (uint64_t(1) << 27)) return false;  // the prefix sums of both kinds of groups share a word
+  if (const char* f = getenv("FFMOE_W8A8_COHORT")) return atoi(f) != 0;
+  if (getenv("FFMOE_PREFILL_MF") || getenv("FFMOE_PREFILL_WIDE")) return false;
+  if (rows <= 64 || hidden + inter < 26 * 128) return false;
+  const uint64_t groups = std::min<uint64_t>(experts, A / 3) + A / 256;  // about: the routing is not known here
+  return groups * uint64_t((inter + 127) / 128) * uint64_t(hidden / 128) >= 64ull * uint64_t(num_cus_p());
+}
+
 template <int MODE>
 int launch_mx_dense(const MxParams& p, int mf, unsigned blocks, hipStream_t stream) {
   switch (mf) {
@@ -563,7 +613,7 @@ PrefillLayout prefill_layout(int rows, int top_k, int experts, int hidden, int i
   l.counts = take(uint64_t(experts) * 4);
   l.offsets = take(uint64_t(experts + 1) * 4);
   l.gbase = take(uint64_t(experts + 1) * 4);
-  l.totals = take(16);
+  l.totals = take(40 * 4);
   l.perm = take(A * 4);
   l.groups = take(l.max_groups * sizeof(GemmGroup));
   l.units0 = take(l.max_groups * uint64_t((inter + 127) / 128) * 8);
@@ -800,9 +850,11 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
                 (int*)(s + l.perm), (GemmGroup*)(s + l.groups), (u32x2*)(s + l.units0), (u32x2*)(s + l.units1)};
   const bool nv_tile = a16 && table->format == FFMOE_FMT_NVFP4 && nvfp4_lines_enabled() && nvfp4_tiles(R, K, E, I) && H % 256 == 0 && I % 256 == 0;
   const int mf = nv ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, (!mx && !a16) || mx || nv_tile);
-  const int tm = 16 * mf;
   // W8A8 and W*A16 cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
-  bool wide = mf == 4 && !mx && !nv_tile;
+  // W8A8 of a prompt chunk: groups of up to 256 and 64 rows on the cohort kernel (wide_gemm.cuh)
+  const bool cohort = !mx && !a16 && !nv && use_cohort(R, K, E, H, I);
+  const int tm = cohort ? 0 : 16 * mf;  // 0: k_prefill_plan's groups of 256 and 64
+  bool wide = mf == 4 && !mx && !nv_tile && !cohort;
   if (const char* f = getenv("FFMOE_PREFILL_WIDE")) wide = (wide && atoi(f) != 0) || nv;
   const int tiles0 = wide ? (I + 255) / 256 : (I + 127) / 128, tiles1 = wide ? (H + 511) / 512 : (H + 255) / 256;
   // A shared expert of the routed experts' format and width rides in the routed launches as further row groups (W*A16
@@ -926,7 +978,8 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   if (stages & 2) {  // gate/up + SwiGLU
     p.a_codes = s + l.xq; p.a_scales = (const float*)(s + l.sx); p.units = b.units0; p.unit_total = b.totals + 0;
     p.out = (uint16_t*)(s + l.act); p.K = H; p.N = I;
-    FF_TRY(launch_gemm<0>(p, mf, wide ? blocks / 2 : blocks, stream, wide, nv));
+    if (cohort) FF_TRY(launch_w8a8_cohort(0, p, b.totals + 4, b.totals + 8, blocks / 2 & ~7u, stream));
+    else FF_TRY(launch_gemm<0>(p, mf, wide ? blocks / 2 : blocks, stream, wide, nv));
   }
   if (stages & 4) {  // re-quantize the activations of the live rows
     const long long cells = (long long)A * (I / 128);
@@ -937,7 +990,8 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   if (stages & 8) {  // down x routing weight, scattered to contributions[assignment]
     p.a_codes = s + l.aq; p.a_scales = (const float*)(s + l.sa); p.units = b.units1; p.unit_total = b.totals + 1;
     p.out = (uint16_t*)args->contributions; p.done = args->done; p.weights = args->weights; p.K = I; p.N = H;
-    FF_TRY(launch_gemm<1>(p, mf, wide ? blocks / 2 : blocks, stream, wide, nv));
+    if (cohort) FF_TRY(launch_w8a8_cohort(1, p, b.totals + 4, b.totals + 24, blocks / 2 & ~7u, stream));
+    else FF_TRY(launch_gemm<1>(p, mf, wide ? blocks / 2 : blocks, stream, wide, nv));
   }
   if (shared) {
     // the always-on expert: the same three steps over all rows in their own order (no grouping, no routing weight),

@@ -31,6 +31,17 @@ int launch_w8a8_wide(int mode, const GemmParams& p, unsigned blocks, hipStream_t
 }
 
 template <int MODE>
+static int launch_cohort(const GemmParams& p, const uint32_t* big_groups, uint32_t* queue, unsigned blocks, hipStream_t stream) {
+  static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_w8a8_cohort<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, COHORT_LDS);
+  if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", COHORT_LDS, hipGetErrorString(ok));
+  hipLaunchKernelGGL(k_w8a8_cohort<MODE>, dim3(blocks), dim3(512), COHORT_LDS, stream, p, big_groups, queue);
+  return ff_launch_status();
+}
+int launch_w8a8_cohort(int mode, const GemmParams& p, const uint32_t* big_groups, uint32_t* queue, unsigned blocks, hipStream_t stream) {
+  return mode == 0 ? launch_cohort<0>(p, big_groups, queue, blocks, stream) : launch_cohort<1>(p, big_groups, queue, blocks, stream);
+}
+
+template <int MODE>
 static int launch_mx(const MxParams& p, unsigned blocks, hipStream_t stream) {
   static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mx_tile<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, MX_TILE_LDS);
   if (ok != hipSuccess) return ff_fail(FFMOE_ERR_UNSUPPORTED, "%d bytes of LDS per block: %s", MX_TILE_LDS, hipGetErrorString(ok));

@@ -47,6 +47,11 @@ struct GemmParams {
   float limit;
 };
 
+// a down output times its routing weight, at either rounding boundary
+__device__ __forceinline__ float w8a8_weighted(float v, float rw, int routed_weight) {
+  return routed_weight == FFMOE_WEIGHT_AFTER_DOWN_BF16 ? __fmul_rn(bround(v), rw) : __fmul_rn(v, rw);
+}
+
 // output columns per unit: every wave owns 32 activation columns (gate and up rows) or 64 down columns
 template <int MODE, int NW = 4>
 __device__ __forceinline__ constexpr int gemm_tile_cols() { return (MODE == 0 ? 32 : 64) * NW; }
@@ -538,7 +543,7 @@ __global__ __launch_bounds__(64 * NW, (NW == 4 && MF <= 4) ? 2 : 1) void k_w8a8_
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
                 if (MODE == 1 && p.weights)
-                  v[r] = p.routed_weight == FFMOE_WEIGHT_AFTER_DOWN_BF16 ? __fmul_rn(bround(acc[m][f][r]), rw) : __fmul_rn(acc[m][f][r], rw);
+                  v[r] = w8a8_weighted(acc[m][f][r], rw, p.routed_weight);
                 else
                   v[r] = acc[m][f][r];
               }

@@ -105,6 +105,37 @@ def test_prefill_shared_expert_wide_tile_kernel_equals_the_tile_kernel_bitwise(r
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("hidden,inter,counts", [
+    (384, 256, [1, 16, 17, 0, 32, 33, 64, 65]),       # every number of live fragments; output columns past the last tile
+    (1152, 128, [128, 129, 0, 256, 257, 3]),          # both sides of a 256-row group; nine K blocks, then one
+    (256, 384, [1000, 385, 2, 448]),                  # several 256-row groups, with and without a rest
+    (8320, 128, [5, 130, 40]),                        # 65 K blocks
+    (128, 2048, [300] * 24 + [20] * 40),              # more units of both kinds than blocks start on
+])
+def test_prefill_cohort_kernel_equals_the_group_kernel_bitwise(hidden, inter, counts, monkeypatch):
+    """The groups of 256 and 64 rows at their edges; a stage repeated without a plan finds its claim counters at zero again."""
+    experts, rows = len(counts), sum(counts) + 3
+    table, _ = make_table(capi.FMT_FP8_BLOCK128, experts, hidden, inter, 91)
+    x = synth.normal((rows, hidden), 1.0, 92).to(torch.bfloat16).cuda()
+    ids = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)] + [torch.full((3,), -1, dtype=torch.int32)])
+    ids = ids[torch.randperm(rows, generator=torch.Generator().manual_seed(7))][:, None].cuda()
+    w = torch.rand((rows, 1), generator=torch.Generator().manual_seed(8)).cuda()
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_COHORT", switch)
+        op = ops.PrefillOps(table, rows, 1)
+        op.done.zero_()
+        live = ids[:, 0] >= 0
+        first = op.contribute(x, ids, w).clone()
+        for stage in (1, 2, 3):
+            op.contribute(x, ids, w, stage=stage)
+        torch.cuda.synchronize()
+        assert torch.equal(op.done != 0, live.reshape(op.done.shape))
+        assert torch.equal(first.view(torch.int16).reshape(rows, -1)[live], op.contributions.view(torch.int16).reshape(rows, -1)[live])
+        out.append(first.view(torch.int16).reshape(rows, -1)[live])
+    assert torch.equal(out[0], out[1])
+
+
 def test_linear_w8a8_device_quantizer_chain():
     """ffmoe_linear_fp8_block(act_mode = FP8_BLOCK128) = device quantizer + W8A8 linear."""
     m, n, k = 9, 256, 640
