@@ -1,6 +1,7 @@
 // Router kernels: logits (BF16 chain contract / FP32 wave-reduced) and deterministic top-k.
 // Behaviour follows kernels/moe_route.cu of the reference; the mapping to wave64 is new.
 #include "common.cuh"
+#include "lds_load.cuh"
 #include "route_select.cuh"
 #include "api.h"
 #include <stdlib.h>
@@ -402,6 +403,148 @@ __global__ __launch_bounds__(256 * LG_TEAMS) void k_route_logits_f32_rows(const 
   }
 }
 
+// The same logits on the matrix cores. v_mfma_f32_16x16x1_4b_f32 is one fused multiply-add, rounded like any other, for 16 rows x 64
+// experts: a chain step of 1024 logits in 32 cycles, twice the vector ALUs' rate (checked against fmaf chains bit for bit, with
+// subnormals, infinities and NaN), and it needs one unpacking instruction per operand and lane instead of four per lane and fma.
+// A block of four waves takes 16 rows x 64 experts, wave w the chains 64 w .. 64 w + 63 in groups of four: four accumulators per
+// lane and output hide each other's latency. The group's vectors of one turn (64 contiguous bytes of 80 rows) come by direct loads into
+// a ring of the wave's own, up to four turns ahead; the groups' sums meet in the tree's order, the four waves' in LDS. Two blocks share a CU.
+// What bounds it: the matrix cores' FP32 rate, and that the vector ALUs stand still while such an instruction runs (unpacked in front of
+// each one: 100 us for a round of two blocks per CU, in pieces of sixteen 92; 59 without any). us, k_route_logits_f32_rows / here, 256
+// experts at hidden 7168: 1024 rows 75 / 57, 2048 132 / 92, 4096 257 / 170.
+constexpr int LGM_RING = 4, LGM_STAGE = 80 * 64, LGM_LDS = 4 * LGM_RING * LGM_STAGE;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__global__ __launch_bounds__(256, 2) void k_route_logits_f32_mfma(const uint16_t* __restrict__ x, const uint16_t* __restrict__ router,
+                                                                  float* __restrict__ logits, int rows, int experts, int hidden) {
+  extern __shared__ __align__(16) uint8_t lg_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = uni(tid >> 6);
+  const int r0 = blockIdx.x * 16, e0 = blockIdx.y * 64;
+  const int words = hidden >> 3;
+  const uint32_t row_bytes = uint32_t(hidden) * 2u;
+  uint8_t* const ring = lg_lds + wave * (LGM_RING * LGM_STAGE);
+  const uint32_t ring0 = lds_address(lg_lds) + uint32_t(wave) * (LGM_RING * LGM_STAGE);
+  // request 0: the token rows, 1 .. 4: sixteen experts each; four lanes per row, 16-byte piece c of row r at c ^ (r / 4 & 3)
+  const uint32_t piece = uint32_t(((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  const uint32_t xoff = uint32_t(min(r0 + (lane >> 2), rows - 1) - r0) * row_bytes + piece;
+  uint32_t eoff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) eoff[q] = uint32_t(min(e0 + 16 * q + (lane >> 2), experts - 1)) * row_bytes + piece;
+  const uint64_t xbase = uint64_t(uintptr_t(x)) + uint64_t(r0) * row_bytes, ebase = uint64_t(uintptr_t(router));
+  const int p0 = wave * 64;
+  auto turns = [&](int g) { const int p = p0 + 4 * g; return p < words ? (words - p + 255) >> 8 : 0; };  // vectors of group g's chains
+  int rg = 0, ri = 0, rn = turns(0), asked = 0;  // the next request: group, turn, its group's turns; requests so far
+  auto advance = [&]() { while (rg < 16 && ri >= rn) { ++rg; ri = 0; rn = rg < 16 ? turns(rg) : 0; } };
+  auto request = [&]() {
+    const uint32_t at = ring0 + uint32_t(asked % LGM_RING) * LGM_STAGE, off = uint32_t(p0 + 4 * rg + 256 * ri) * 16u;
+    lds_load16(at, xbase + off, xoff);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) lds_load16(at + 1024u + q * 1024u, ebase + off, eoff[q]);
+    ++asked;
+    ++ri;
+    advance();
+  };
+  advance();
+#pragma unroll 1
+  for (int i = 0; i < LGM_RING; ++i)
+    if (rg < 16) request();
+  const int key = (lane >> 2) & 3;
+  const uint8_t* const xl = ring + (lane & 15) * 64;
+  const uint8_t* const el = ring + 1024 + lane * 64;
+  f32x16 l0, l1, l2, l3, total;  // partial sums of 4, 8, 16 and 32 chains that wait for their partners
+#pragma unroll
+  for (int r = 0; r < 16; ++r) l0[r] = l1[r] = l2[r] = l3[r] = total[r] = 0.0f;
+  auto add = [](const f32x16& a, const f32x16& b) {
+    f32x16 o;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[r] = __fadd_rn(a[r], b[r]);
+    return o;
+  };
+  int used = 0;
+  u32x4 xv[4], ev[4];  // the turn at hand, as it lies in LDS
+  auto fetch = [&]() {
+    const int younger = asked - used - 1;
+    if (younger < 0) return;  // that was the last turn
+    if (younger >= 3) asm volatile("s_waitcnt vmcnt(15)" ::: "memory");
+    else if (younger == 2) asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    else if (younger == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int at = (used % LGM_RING) * LGM_STAGE;
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+      xv[ch] = *reinterpret_cast<const u32x4*>(xl + at + ((ch ^ key) << 4));
+      ev[ch] = *reinterpret_cast<const u32x4*>(el + at + ((ch ^ key) << 4));
+    }
+  };
+  fetch();
+#pragma unroll 1
+  for (int g = 0; g < 16; ++g) {
+    f32x16 acc[4];
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[ch][r] = 0.0f;
+    const int n = turns(g);
+#pragma unroll 1
+    for (int i = 0; i < n; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // four elements of every chain at a time: the vector ALUs wait while an FP32 matrix instruction runs, so the unpacking comes in one
+        // piece, and the next turn's reads go out in front of the second half's instructions
+        float xf[4][4], ef[4][4];
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch)
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            xf[ch][2 * q] = bf16lo(xv[ch][2 * h + q]); xf[ch][2 * q + 1] = bf16hi(xv[ch][2 * h + q]);
+            ef[ch][2 * q] = bf16lo(ev[ch][2 * h + q]); ef[ch][2 * q + 1] = bf16hi(ev[ch][2 * h + q]);
+          }
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(xf[ch][e]), "+v"(ef[ch][e]));
+        if (h == 1) {
+          ++used;
+          if (rg < 16) request();  // into the place of the turn just unpacked
+          fetch();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int ch = 0; ch < 4; ++ch) acc[ch] = __builtin_amdgcn_mfma_f32_16x16x1f32(xf[ch][e], ef[ch][e], acc[ch], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    f32x16 s = add(add(acc[0], acc[1]), add(acc[2], acc[3]));
+    if (!(g & 1)) l0 = s;
+    else {
+      s = add(l0, s);
+      if (!(g & 2)) l1 = s;
+      else {
+        s = add(l1, s);
+        if (!(g & 4)) l2 = s;
+        else {
+          s = add(l2, s);
+          if (!(g & 8)) l3 = s;
+          else total = add(l3, s);
+        }
+      }
+    }
+  }
+  // lane (16 a + b): rows 4 a .. 4 a + 3 (register r % 4) of experts 16 (r / 4) + b
+  __syncthreads();  // the rings have been read
+  float* part = reinterpret_cast<float*>(lg_lds);  // [wave][row][expert]
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part[(wave * 16 + 4 * (lane >> 4) + (r & 3)) * 64 + 16 * (r >> 2) + (lane & 15)] = total[r];
+  __syncthreads();
+  for (int t = tid; t < 1024; t += 256) {
+    const int row = t >> 6, e = t & 63;
+    const float v = __fadd_rn(__fadd_rn(part[t], part[1024 + t]), __fadd_rn(part[2048 + t], part[3072 + t]));
+    if (r0 + row < rows && e0 + e < experts) logits[size_t(r0 + row) * experts + e0 + e] = v;
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Selection by rank. The reference runs top_k rounds of a block-wide arg-max under (score desc, id asc)
 // (kernels/moe_route.cu:205-235); that order is total, so the r-th pick is the candidate with exactly r
@@ -617,6 +760,24 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_route_logits_f32(con
   FF_PTR16(x); FF_PTR16(router); FF_PTR4(logits);
   FF_NO_OVERLAP(logits, size_t(rows) * experts * 4, x, size_t(rows) * hidden * 2);
   FF_NO_OVERLAP(logits, size_t(rows) * experts * 4, router, size_t(experts) * hidden * 2);
+  // Very many rows: the matrix cores (FFMOE_ROUTE_LOGITS_MFMA: 1 wherever they can run, 0 never; same bits). A tile of 16 rows x 64 experts
+  // takes 4 us + 7.3 ns per column where a CU has one, 1.62 times that where it has two; the vector kernel 6 us + 3.4 us per 100 M fmas. us,
+  // vector / matrix: 64 experts at 7168, 2048 rows (one tile on half the CUs) 42 / 56, 4096 77 / 57; 128 at 2048, 1500 rows 21.0 / 21.0,
+  // 2048 29 / 21; 256 at 7168, 768 rows 56 / 57, 1024 75 / 57, 1500 97 / 92.
+  {
+    const char* e = getenv("FFMOE_ROUTE_LOGITS_MFMA");
+    const long long tiles = (long long)((rows + 15) / 16) * ((experts + 63) / 64), cus = decode_cus();
+    const double matrix = (4.0 + 0.0073 * hidden) * (tiles <= cus ? 1.0 : 1.62 * double((tiles + 2 * cus - 1) / (2 * cus)));
+    const double vector = 6.0 + 3.4e-8 * double(rows) * double(experts) * double(hidden);
+    if (hidden % 32 == 0 && uint64_t(experts) * uint64_t(hidden) * 2 < (uint64_t(1) << 32) && (e ? atoi(e) != 0 : vector > 1.05 * matrix)) {
+      static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_route_logits_f32_mfma), hipFuncAttributeMaxDynamicSharedMemorySize, LGM_LDS);
+      if (ok == hipSuccess) {
+        hipLaunchKernelGGL(k_route_logits_f32_mfma, dim3((rows + 15) / 16, (experts + 63) / 64), dim3(256), LGM_LDS, (hipStream_t)stream,
+                           (const uint16_t*)x, (const uint16_t*)router, logits, rows, experts, hidden);
+        return ff_launch_status();
+      }
+    }
+  }
   // Many rows: the kernel that keeps a tile of router rows in LDS (from FFMOE_ROUTE_LOGITS_TILE_ROWS rows on, default 96 - 15.8 against 18.4 us there at 256 x 7168, 13.2 against 15.5 us at 64 rows;
   // 0 = never), when the tile and the partial sums fit. Same bits either way.
   {

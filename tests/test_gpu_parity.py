@@ -168,6 +168,22 @@ def test_route_logits_f32_bit_exact_and_close_to_f64(rows, experts, hidden):
     assert np.max(np.abs(got - f64)) <= 16 * 2.0 ** -24 * np.max(np.abs(x.double().numpy()) @ np.abs(w.double().numpy()).T)
 
 
+@pytest.mark.parametrize("rows,experts,hidden", [(1, 1, 32), (17, 65, 1024), (16, 64, 2048), (33, 100, 2080), (5, 256, 7168), (40, 8, 8224)])
+def test_route_logits_f32_matrix_core_path_bit_exact(rows, experts, hidden, monkeypatch):
+    """Ragged rows and experts, chains without an element, of one, and of several turns of different lengths; subnormal products, an
+    infinity and a NaN among them. Against the oracle and, over all of it, the kernel it replaces."""
+    monkeypatch.setenv("FFMOE_ROUTE_LOGITS_MFMA", "1")
+    x, r = rand_bf16((rows, hidden), 1.0, 61 + rows), rand_bf16((experts, hidden), 0.02, 62 + rows)
+    out = lambda: RouteOps.logits_f32(x.to(DEV), r.to(DEV)).cpu().numpy().view(np.uint32)
+    assert np.array_equal(out(), orc.route_logits_f32(bits(x), bits(r)).view(np.uint32))
+    x[0, ::7] *= 2.0 ** -70
+    r[0, ::5] *= 2.0 ** -60
+    x[-1, 3], r[-1, 11] = float("inf"), float("nan")
+    got = out()
+    monkeypatch.setenv("FFMOE_ROUTE_LOGITS_MFMA", "0")
+    assert np.array_equal(got, out())
+
+
 @pytest.mark.parametrize("score", [capi.SCORE_SOFTMAX, capi.SCORE_SIGMOID])
 @pytest.mark.parametrize("rows,experts,top_k", [(4, 64, 4), (3, 256, 8), (2, 1000, 32), (5, 48, 6)])
 def test_route_topk_bit_exact(score, rows, experts, top_k):
