@@ -595,6 +595,18 @@ int launch_mx_dense(const MxParams& p, int mf, unsigned blocks, hipStream_t stre
   return ff_launch_status();
 }
 
+// A dense BF16 expert (the shared expert next to experts of another format) over many rows on the same tiles (FFMOE_BF16_TILE: 1 always,
+// 0 never). The blocks that split the contraction (dense_splitk.cuh) pass the whole token panel through every block, and the grouped
+// kernel has a wave per SIMD. us gate/up + down, those / tiles: hidden 7168 / intermediate 2048, 128 rows 86 + 36 / 80 + 25, 192 126 + 52 /
+// 80 + 27, 768 494 + 180 / 80 + 33, 1021 122 + 78 / 85 + 36; 7168 / 768, 128 rows 45 + 35 / 80 + 13, 192 85 + 51 / 81 + 14; 2048 / 768, 128
+// rows 18 + 19 / 29 + 13, 192 33 + 19 / 29 + 13. Distance from the rounded FP64 sums at 7168 / 2048, 512 rows: 1.69e-4 / 1.23e-4.
+// An expert that could ride in the routed launches keeps their sums wherever it runs.
+bool use_bf16_tiles(int rows, bool rides) {
+  if (const char* f = getenv("FFMOE_BF16_TILE")) return atoi(f) != 0;
+  const char* se = getenv("FFMOE_SHARED_SPLITK");  // 0 asks for the grouped kernels
+  return rows > 128 && !rides && !(se && atoi(se) == 0);
+}
+
 struct PrefillLayout {
   uint64_t xq, sx, act, aq, sa, counts, offsets, gbase, totals, perm, groups, units0, units1, sh_act, sh_aq, sh_sa, total;
   uint64_t max_groups;
@@ -660,7 +672,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
 // activations between the two launches; stage_mask bit 0 = gate/up + SwiGLU, bit 1 = down. Arguments are checked by the
 // callers.
 int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, int H, int swiglu, float limit, void* act, void* shared_out,
-                      int stage_mask, void* stream_) {
+                      int stage_mask, void* stream_, bool rides) {
   hipStream_t stream = (hipStream_t)stream_;
   const int SI = shared->inter;
   const unsigned blocks = ((unsigned)num_cus_p() * 2u) & ~7u;
@@ -675,6 +687,23 @@ int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, i
   const char* ne = getenv("FFMOE_PREFILL_SHARED_NARROW");
   const bool may_narrow = (shared->format == FFMOE_FMT_BF16 || shared->format == FFMOE_FMT_FP8_BLOCK128) && !(ne && atoi(ne) == 0);
   const unsigned nblocks = ((unsigned)num_cus_p() * 8u) & ~7u;
+  if (shared->format == FFMOE_FMT_BF16 && use_bf16_tiles(R, rides)) {
+    GemmParams g{};
+    g.rows_total = R; g.top_k = 1; g.swiglu = swiglu; g.limit = limit;
+    auto run = [&](int mode) {
+      g.total_units = tile_units(mode, R, g.N);
+      return launch_bf16_tile(mode, g, std::min<unsigned>((g.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
+    };
+    if (stage_mask & 1) {
+      g.a_codes = (const uint8_t*)x; g.w0_codes = shared->slot[0]; g.w1_codes = shared->slot[2]; g.out = (uint16_t*)act; g.K = H; g.N = SI;
+      FF_TRY(run(0));
+    }
+    if (stage_mask & 2) {
+      g.a_codes = (const uint8_t*)act; g.w0_codes = shared->slot[4]; g.w1_codes = 0; g.out = (uint16_t*)shared_out; g.K = SI; g.N = H;
+      FF_TRY(run(2));
+    }
+    return 0;
+  }
   // A BF16 expert over so few rows that the grouped kernels would give it fewer tiles than CUs: blocks of eight waves that
   // split the contraction (dense_splitk.cuh; FFMOE_SHARED_SPLITK=0 keeps the grouped kernels). Hidden 7168 / intermediate
   // 2048, 32 rows: 62 + 19 us on one-wave tiles.
@@ -968,7 +997,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
     }
     if (shared && !ride)
       FF_TRY(shared_expert_w16(shared, args->x, R, H, args->swiglu, args->swiglu_limit, s + l.sh_act, args->shared_out,
-                               (stages & 2 ? 1 : 0) | (stages & 8 ? 2 : 0), stream_));
+                               (stages & 2 ? 1 : 0) | (stages & 8 ? 2 : 0), stream_, shared->format == table->format && SI == I));
     return 0;
   }
   GemmParams p{};

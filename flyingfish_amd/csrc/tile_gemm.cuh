@@ -13,6 +13,7 @@
 // 64 token scales per K block, a line look-up per token; 157 with that and bank conflicts in every operand read), 2048 x 2048 -> 7168 41 us.
 #pragma once
 #include "mx_gemm.cuh"
+#include "w16_gemm.cuh"
 #include "lds_load.cuh"
 
 namespace ffmoe {
@@ -22,7 +23,11 @@ namespace ffmoe {
 // MX: E4M3 weights with one E8M0 scale per 32 x 32 block against E4M3 activations with one per 32 columns (mx_gemm.cuh's dense form, the
 // same bits): the matrix core applies the scales and sums over the whole contraction. 1500 tokens at hidden 7168 / intermediate 2048:
 // gate/up 142 -> 88 us, down 70 -> 39 us against 64-row units with the weights requested in operand order.
-template <int MODE, bool MX>
+// BF: BF16 weights and activations, no scales: a stage is 64 columns, two matrix instructions. The accumulators are added to totals every
+// four stages, so that a sum over K has about as many roundings as the eight partial sums of dense_splitk.cuh, whose rows this takes over
+// (in one chain its outputs were 1.5 times as far from the rounded FP64 sums). 1021 tokens, hidden 7168 / intermediate 2048: 122 + 78 ->
+// 85 + 36 us against the 64-row kernel.
+template <int MODE, bool MX, bool BF = false>
 __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
   struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; };
   __shared__ __attribute__((aligned(16))) Stage stage[2];
@@ -30,7 +35,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int wr = wave >> 1, wt = wave & 1;
-  const int K = p.K, N = p.N, KB = K >> 7;
+  const int K = BF ? 2 * p.K : p.K, N = p.N, KB = K >> 7;  // bytes of a row, 128 per stage
   const uint32_t total = p.total_units;
   const int ntiles = (N + (MODE == 0 ? 63 : 127)) / (MODE == 0 ? 64 : 128);
   const int groups = (p.rows_total + 127) / 128;
@@ -68,8 +73,8 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
     for (int i = 0; i < 4; ++i) tsrc[i] = p.a_codes + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * K + (((lane & 7) ^ lds_key(lane >> 3) ^ 4 * (i & 1)) << 4);
     // Block scales, one word per K block; lane l keeps K block l (+ 64). A wave's columns sit inside one 128-row block; MX: four
     // bytes per 32 rows, which are the wave's fragments 0, 1 and its fragments 2, 3.
-    const float* sw0 = reinterpret_cast<const float*>(ws[0]) + size_t(min(column(wr, 0), N - 16) >> (MX ? 5 : 7)) * KB;
-    const float* sw1 = reinterpret_cast<const float*>(ws[1]) + size_t(min(column(wr, MX ? 2 : 0), N - 16) >> (MX ? 5 : 7)) * KB;
+    [[maybe_unused]] const float* sw0 = reinterpret_cast<const float*>(ws[0]) + size_t(min(column(wr, 0), N - 16) >> (MX ? 5 : 7)) * KB;
+    [[maybe_unused]] const float* sw1 = reinterpret_cast<const float*>(ws[1]) + size_t(min(column(wr, MX ? 2 : 0), N - 16) >> (MX ? 5 : 7)) * KB;
 
     auto request = [&](int kb, int b) {
 #pragma unroll
@@ -78,7 +83,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       for (int i = 0; i < 4; ++i) lds_load16(lds_t[b] + i * 1024u, tsrc[i] + uint32_t(kb) * 128u);
       // Token scales, a row of KB words per token (MX: the four scale bytes of a K block are one word): a request takes eight K blocks of
       // eight tokens. One K block of 64 tokens per request touches a line per lane, as many line look-ups as the operands themselves.
-      if ((kb & 7) == 0) {
+      if (!BF && (kb & 7) == 0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           lds_load4(lds_s + uint32_t((kb >> 3) & 1) * 4096u + i * 256u, p.a_scales + size_t(token_row(wave * 32 + i * 8 + (lane >> 3))) * KB + min(kb + (lane & 7), KB - 1));
@@ -94,6 +99,14 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       for (int f = 0; f < 4; ++f)
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[m][f][r] = 0.0f;
+
+    float tot[BF ? 4 : 1][4][4];
+#pragma unroll
+    for (int m = 0; m < (BF ? 4 : 1); ++m)
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tot[m][f][r] = 0.0f;
 
     auto block = [&](int kb, int b, float s0, float s1) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -111,9 +124,39 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       u32x4 tlo[2], thi[2];
       float sx[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) sx[m] = sl[16 * 8 * m];
+      for (int m = 0; m < 4; ++m) sx[m] = BF ? 1.0f : sl[16 * 8 * m];
       tlo[0] = *reinterpret_cast<const u32x4*>(tl + rd_lo);
       thi[0] = *reinterpret_cast<const u32x4*>(tl + rd_hi);
+      if constexpr (BF) {
+        auto half = [](const v8i& v, int h) { return __builtin_bit_cast(w16_bf16x8, u32x4{uint32_t(v[4 * h]), uint32_t(v[4 * h + 1]), uint32_t(v[4 * h + 2]), uint32_t(v[4 * h + 3])}); };
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          if (m + 1 < 4) {
+            tlo[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_lo);
+            thi[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_hi);
+          }
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            v4f t4 = {acc[m][f][0], acc[m][f][1], acc[m][f][2], acc[m][f][3]};
+            t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[f], 0), __builtin_bit_cast(w16_bf16x8, tlo[m & 1]), t4, 0, 0, 0);
+            t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[f], 1), __builtin_bit_cast(w16_bf16x8, thi[m & 1]), t4, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[m][f][r] = t4[r];
+          }
+        }
+        if ((kb & 3) == 3 || kb + 1 == KB) {
+#pragma unroll
+          for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int f = 0; f < 4; ++f)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                tot[m][f][r] = __fadd_rn(tot[m][f][r], acc[m][f][r]);
+                acc[m][f][r] = 0.0f;
+              }
+        }
+        return;
+      }
       if constexpr (MX) {
         const int w0 = int((__float_as_uint(s0) >> (8 * c)) & 0xffu), w1 = int((__float_as_uint(s1) >> (8 * c)) & 0xffu);
 #pragma unroll
@@ -166,8 +209,8 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
     };
     for (int kb0 = 0; kb0 < KB; kb0 += 64) {
       const int kl = min(kb0 + lane, KB - 1);
-      const float swl0 = landed(load_global<float>(sw0 + kl));
-      const float swl1 = MODE == 0 || MX ? landed(load_global<float>(sw1 + kl)) : swl0;
+      const float swl0 = BF ? 1.0f : landed(load_global<float>(sw0 + kl));
+      const float swl1 = !BF && (MODE == 0 || MX) ? landed(load_global<float>(sw1 + kl)) : swl0;
       const int kend = min(KB, kb0 + 64);
       auto scale = [&](float v, int kb) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), kb - kb0)); };
       for (int kb = kb0; kb < kend; kb += 2) {  // kb0 is even: buffer = parity of the K block
@@ -176,6 +219,14 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       }
     }
 
+    if constexpr (BF) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][f][r] = tot[m][f][r];
+    }
     const int sub = (lane >> 4) * 4;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -189,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
             if (col + 16 <= N) {
               uint32_t o[4];
 #pragma unroll
-              for (int r = 0; r < 4; ++r) o[r] = MX ? mx_swiglu(acc[m][f][r], acc[m][f + 2][r], 1.0f, p.limit) : swiglu_bf16_two_branch(bround(acc[m][f][r]), bround(acc[m][f + 2][r]), p.swiglu, p.limit);
+              for (int r = 0; r < 4; ++r) o[r] = MX ? mx_swiglu(acc[m][f][r], acc[m][f + 2][r], 1.0f, p.limit) : BF ? swiglu_bf16(bround(acc[m][f][r]), bround(acc[m][f + 2][r]), p.swiglu, p.limit) : swiglu_bf16_two_branch(bround(acc[m][f][r]), bround(acc[m][f + 2][r]), p.swiglu, p.limit);
               *reinterpret_cast<u32x2*>(p.out + size_t(pos) * N + col + sub) = u32x2{o[0] | (o[1] << 16), o[2] | (o[3] << 16)};
             }
           }

@@ -19,6 +19,12 @@ int launch_mx_dense_tile(int mode, const GemmParams& p, unsigned blocks, hipStre
   return ff_launch_status();
 }
 
+int launch_bf16_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
+  if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, false, true>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((k_w8a8_tile<2, false, true>), dim3(blocks), dim3(256), 0, stream, p);
+  return ff_launch_status();
+}
+
 template <int MODE>
 static int launch_wide(const GemmParams& p, unsigned blocks, hipStream_t stream) {
   static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_w8a8_wide<MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, WIDE_LDS);

@@ -105,6 +105,29 @@ def test_prefill_shared_expert_wide_tile_kernel_equals_the_tile_kernel_bitwise(r
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("rows,hidden,inter", [(1, 256, 128), (129, 192, 128), (130, 320, 192), (300, 1024, 256)])
+def test_prefill_bf16_shared_expert_tile_kernel_matches_the_float64_sums(rows, hidden, inter, monkeypatch):
+    """Ragged rows and columns, one stage and numbers of stages that do not fill a fold; stage by stage against FP64 with the same BF16
+    boundaries, where an FP32 sum's error leaves at most a neighbouring BF16 value."""
+    table = ops.ExpertTable.allocate(capi.FMT_FP8_CHANNEL, 1, hidden, inter)
+    sh = ops.ExpertTable.allocate(capi.FMT_BF16, 1, hidden, inter)
+    w = [synth.normal(s, 0.02, 95 + i).to(torch.bfloat16) for i, s in enumerate([(inter, hidden), (inter, hidden), (hidden, inter)])]
+    for i in range(3):
+        sh.expert_views(0)[2 * i].copy_(w[i])
+    x = synth.normal((rows, hidden), 1.0, 98).to(torch.bfloat16)
+    ids, wt = torch.full((rows, 1), -1, dtype=torch.int32).cuda(), torch.ones((rows, 1)).cuda()
+    monkeypatch.setenv("FFMOE_BF16_TILE", "1")
+    op = ops.PrefillOps(table, rows, 1, shared=sh.shared_struct(0), act_mode=capi.ACT_BF16)
+    op.contribute(x.cuda(), ids, wt)
+    torch.cuda.synchronize()
+    act = op.scratch_views()["sh_act"].cpu().view(torch.bfloat16).reshape(rows, inter)
+    r = lambda v: v.float().to(torch.bfloat16).double()
+    g, u = r(x.double() @ w[0].double().t()), r(x.double() @ w[1].double().t())
+    want = r(r(g / (1 + torch.exp(-g))) * u)
+    assert_close_bf16(bits(act), bits(want.to(torch.bfloat16)), "shared activations", max_ulp=3)
+    assert_close_bf16(bits(op.shared_out), bits((act.double() @ w[2].double().t()).float().to(torch.bfloat16)), "shared expert", max_ulp=1)
+
+
 @pytest.mark.parametrize("hidden,inter,counts", [
     (384, 256, [1, 16, 17, 0, 32, 33, 64, 65]),       # every number of live fragments; output columns past the last tile
     (1152, 128, [128, 129, 0, 256, 257, 3]),          # both sides of a 256-row group; nine K blocks, then one
