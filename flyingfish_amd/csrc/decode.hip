@@ -29,7 +29,7 @@ bool decode_form_rows_fit(int fmt, const DecodeParams& p);
 int decode_form_rows_launch(int fmt, int form, int rg, const DecodeParams& p, long long routed, long long shared, int stage_mask, hipStream_t st);
 int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int stages, void* stream);
 int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, int H, int swiglu, float limit, void* act, void* shared_out,
-                      int stage_mask, void* stream_, bool rides);
+                      int stage_mask, void* stream_);
 }  // namespace ffmoe
 
 namespace ffmoe {
@@ -474,7 +474,7 @@ static int decode_dispatch(const ffmoe_expert_table* table, const ffmoe_shared_e
       const uint64_t own = (((A + R) * imax * 2 + 255) & ~uint64_t(255)) + (((A + R + 2) * sizeof(GroupDesc) + 255) & ~uint64_t(255)) + 256;
       uint8_t* act = (uint8_t*)args->scratch + own;
       FF_REQUIRE(own + act_bytes <= args->scratch_bytes, FFMOE_ERR_SCRATCH, "decode scratch too small for the shared expert's activations");
-      return shared_expert_w16(shared, args->x, R, H, args->swiglu, args->swiglu_limit, act, args->shared_out, stage_mask, stream, true);
+      return shared_expert_w16(shared, args->x, R, H, args->swiglu, args->swiglu_limit, act, args->shared_out, stage_mask, stream);
     }
   }
   if (!table || !args || !shared || shared->format == table->format) return decode_impl(table, shared, args, stage_mask, stream);

@@ -596,15 +596,14 @@ int launch_mx_dense(const MxParams& p, int mf, unsigned blocks, hipStream_t stre
 }
 
 // A dense BF16 expert (the shared expert next to experts of another format) over many rows on the same tiles (FFMOE_BF16_TILE: 1 always,
-// 0 never). The blocks that split the contraction (dense_splitk.cuh) pass the whole token panel through every block, and the grouped
+// 0 never; same bits). The blocks that split the contraction (dense_splitk.cuh) pass the whole token panel through every block, and the grouped
 // kernel has a wave per SIMD. us gate/up + down, those / tiles: hidden 7168 / intermediate 2048, 128 rows 86 + 36 / 80 + 25, 192 126 + 52 /
 // 80 + 27, 768 494 + 180 / 80 + 33, 1021 122 + 78 / 85 + 36; 7168 / 768, 128 rows 45 + 35 / 80 + 13, 192 85 + 51 / 81 + 14; 2048 / 768, 128
-// rows 18 + 19 / 29 + 13, 192 33 + 19 / 29 + 13. Distance from the rounded FP64 sums at 7168 / 2048, 512 rows: 1.69e-4 / 1.23e-4.
-// An expert that could ride in the routed launches keeps their sums wherever it runs.
-bool use_bf16_tiles(int rows, bool rides) {
+// rows 18 + 19 / 29 + 13, 192 33 + 19 / 29 + 13.
+bool use_bf16_tiles(int rows) {
   if (const char* f = getenv("FFMOE_BF16_TILE")) return atoi(f) != 0;
   const char* se = getenv("FFMOE_SHARED_SPLITK");  // 0 asks for the grouped kernels
-  return rows > 128 && !rides && !(se && atoi(se) == 0);
+  return rows > 128 && !(se && atoi(se) == 0);
 }
 
 struct PrefillLayout {
@@ -672,7 +671,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
 // activations between the two launches; stage_mask bit 0 = gate/up + SwiGLU, bit 1 = down. Arguments are checked by the
 // callers.
 int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, int H, int swiglu, float limit, void* act, void* shared_out,
-                      int stage_mask, void* stream_, bool rides) {
+                      int stage_mask, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
   const int SI = shared->inter;
   const unsigned blocks = ((unsigned)num_cus_p() * 2u) & ~7u;
@@ -687,12 +686,19 @@ int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, i
   const char* ne = getenv("FFMOE_PREFILL_SHARED_NARROW");
   const bool may_narrow = (shared->format == FFMOE_FMT_BF16 || shared->format == FFMOE_FMT_FP8_BLOCK128) && !(ne && atoi(ne) == 0);
   const unsigned nblocks = ((unsigned)num_cus_p() * 8u) & ~7u;
-  if (shared->format == FFMOE_FMT_BF16 && use_bf16_tiles(R, rides)) {
+  // A BF16 expert over so few rows that the grouped kernels would give it fewer tiles than CUs: blocks of eight waves that
+  // split the contraction (dense_splitk.cuh; FFMOE_SHARED_SPLITK=0 keeps the grouped kernels). Hidden 7168 / intermediate
+  // 2048, 32 rows: 62 + 19 us on one-wave tiles.
+  const char* se = getenv("FFMOE_SHARED_SPLITK");
+  const bool splitk = shared->format == FFMOE_FMT_BF16 && !(se && atoi(se) == 0) && H % 256 == 0 && SI % 256 == 0 &&
+                      sgroups * uint32_t((SI + 127) / 128) < (unsigned)num_cus_p();
+  // Many rows of either: 128 x 128 tiles, which sum in the order of the kernel that they stand in for
+  if (shared->format == FFMOE_FMT_BF16 && use_bf16_tiles(R)) {
     GemmParams g{};
     g.rows_total = R; g.top_k = 1; g.swiglu = swiglu; g.limit = limit;
     auto run = [&](int mode) {
       g.total_units = tile_units(mode, R, g.N);
-      return launch_bf16_tile(mode, g, std::min<unsigned>((g.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
+      return launch_bf16_tile(mode, splitk, g, std::min<unsigned>((g.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
     };
     if (stage_mask & 1) {
       g.a_codes = (const uint8_t*)x; g.w0_codes = shared->slot[0]; g.w1_codes = shared->slot[2]; g.out = (uint16_t*)act; g.K = H; g.N = SI;
@@ -704,12 +710,6 @@ int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, i
     }
     return 0;
   }
-  // A BF16 expert over so few rows that the grouped kernels would give it fewer tiles than CUs: blocks of eight waves that
-  // split the contraction (dense_splitk.cuh; FFMOE_SHARED_SPLITK=0 keeps the grouped kernels). Hidden 7168 / intermediate
-  // 2048, 32 rows: 62 + 19 us on one-wave tiles.
-  const char* se = getenv("FFMOE_SHARED_SPLITK");
-  const bool splitk = shared->format == FFMOE_FMT_BF16 && !(se && atoi(se) == 0) && H % 256 == 0 && SI % 256 == 0 &&
-                      sgroups * uint32_t((SI + 127) / 128) < (unsigned)num_cus_p();
   if (splitk) {
     // 8 activation columns (gate + up rows in one fragment) or 16 output columns per block; tiles of half that size, for
     // twice the blocks, measured slower (32 rows: 52 + 34 against 32 + 20 us): every block reads the whole token panel
@@ -997,7 +997,7 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
     }
     if (shared && !ride)
       FF_TRY(shared_expert_w16(shared, args->x, R, H, args->swiglu, args->swiglu_limit, s + l.sh_act, args->shared_out,
-                               (stages & 2 ? 1 : 0) | (stages & 8 ? 2 : 0), stream_, shared->format == table->format && SI == I));
+                               (stages & 2 ? 1 : 0) | (stages & 8 ? 2 : 0), stream_));
     return 0;
   }
   GemmParams p{};

@@ -23,12 +23,15 @@ namespace ffmoe {
 // MX: E4M3 weights with one E8M0 scale per 32 x 32 block against E4M3 activations with one per 32 columns (mx_gemm.cuh's dense form, the
 // same bits): the matrix core applies the scales and sums over the whole contraction. 1500 tokens at hidden 7168 / intermediate 2048:
 // gate/up 142 -> 88 us, down 70 -> 39 us against 64-row units with the weights requested in operand order.
-// BF: BF16 weights and activations, no scales: a stage is 64 columns, two matrix instructions. The accumulators are added to totals every
-// four stages, so that a sum over K has about as many roundings as the eight partial sums of dense_splitk.cuh, whose rows this takes over
-// (in one chain its outputs were 1.5 times as far from the rounded FP64 sums). 1021 tokens, hidden 7168 / intermediate 2048: 122 + 78 ->
-// 85 + 36 us against the 64-row kernel.
-template <int MODE, bool MX, bool BF = false>
+// BF16: BF16 weights and activations, no scales: a stage is 64 columns, two matrix instructions, summed in one chain as in w16_gemm.cuh.
+// BF16_SPLIT: the same, summed as dense_splitk.cuh does: eight partial sums over the columns that its waves take, added in their order.
+// A tile walks the partial sums one behind the other: K a multiple of 1024, two stages of every sixteen, else contiguous eighths, whose
+// ends may halve a stage (K a multiple of 256). So either takes over rows of its kernel with the same bits. 1021 tokens, hidden
+// 7168 / intermediate 2048: 122 + 78 -> 85 + 36 us against the 64-row kernel.
+enum TileForm { TILE_W8A8, TILE_MX, TILE_BF16, TILE_BF16_SPLIT };
+template <int MODE, TileForm FORM>
 __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
+  constexpr bool MX = FORM == TILE_MX, SPLIT = FORM == TILE_BF16_SPLIT, BF = FORM == TILE_BF16 || SPLIT;
   struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; };
   __shared__ __attribute__((aligned(16))) Stage stage[2];
   __shared__ float sx_lds[2][128][8];  // token scales of eight K blocks
@@ -47,8 +50,9 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
   const uint32_t lds_s = lds_address(sx_lds) + uint32_t(wave) * 1024u;
   const uint32_t woff = uint32_t(lane >> 3) * uint32_t(K) + uint32_t(((lane & 7) ^ lds_key(lane >> 3)) << 4);  // odd requests: piece ^ 4
   // operand reads: row lane % 16, bytes 32 c .. 32 c + 31 of the K block for lane group c
-  // (MX: bytes 16 c .. 16 c + 15 and 64 + 16 c .. 64 + 16 c + 15, the operand form whose scales sit in lane group column / 32)
-  const int r16 = lane & 15, c = lane >> 4, c_lo = MX ? c : 2 * c, c_hi = MX ? c + 4 : 2 * c + 1;
+  // (MX: bytes 16 c .. 16 c + 15 and 64 + 16 c .. 64 + 16 c + 15, the operand form whose scales sit in lane group column / 32;
+  // BF16: 16 columns of a lane, the first eight in the first instruction; BF16_SPLIT: 32 columns of the stage per instruction)
+  const int r16 = lane & 15, c = lane >> 4, c_lo = MX || SPLIT ? c : 2 * c, c_hi = MX || SPLIT ? c + 4 : 2 * c + 1;
   const int rd_lo = r16 * 128 + ((c_lo ^ lds_key(r16)) << 4), rd_hi = r16 * 128 + ((c_hi ^ lds_key(r16)) << 4);
 
   for (uint32_t u = xcd * span + slot; u < span_end; u += per_xcd) {
@@ -100,18 +104,31 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[m][f][r] = 0.0f;
 
-    float tot[BF ? 4 : 1][4][4];
+    // SPLIT: the sum of the partial sums so far (the first one is added to -0.0, which leaves it as it is), the stage asked for last, as the
+    // j-th of partial sum w, and the 32-column steps since the last partial sum ended
+    [[maybe_unused]] float tot[SPLIT ? 4 : 1][4][4];
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int m = 0; m < (BF ? 4 : 1); ++m)
+      for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int f = 0; f < 4; ++f)
+        for (int f = 0; f < 4; ++f)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tot[m][f][r] = 0.0f;
+          for (int r = 0; r < 4; ++r) tot[m][f][r] = -0.0f;
+    }
+    [[maybe_unused]] const int part_steps = KB >> 2;       // of 32 columns
+    [[maybe_unused]] const bool dealt = part_steps % 4 == 0;
+    [[maybe_unused]] int ask_w = 0, ask_j = 0, steps = 0;
+    auto next_stage = [&](int q) {  // where the q-th stage of the walk is
+      if constexpr (!SPLIT) return q;
+      if (!dealt) return q;
+      if (++ask_j == part_steps >> 1) { ask_j = 0; ++ask_w; }
+      return ((ask_j >> 1) * 8 + ask_w) * 2 + (ask_j & 1);
+    };
 
     auto block = [&](int kb, int b, float s0, float s1) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();  // K block kb is there for every wave, and nobody reads the other buffer any more
-      if (kb + 1 < KB) request(kb + 1, b ^ 1);
+      if (kb + 1 < KB) request(next_stage(kb + 1), b ^ 1);
       const uint8_t* wl = stage[b].w + wr * 8192;
       const uint8_t* tl = stage[b].t + wt * 8192;
       const float* sl = &sx_lds[(kb >> 3) & 1][wt * 64 + r16][kb & 7];
@@ -129,31 +146,49 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       thi[0] = *reinterpret_cast<const u32x4*>(tl + rd_hi);
       if constexpr (BF) {
         auto half = [](const v8i& v, int h) { return __builtin_bit_cast(w16_bf16x8, u32x4{uint32_t(v[4 * h]), uint32_t(v[4 * h + 1]), uint32_t(v[4 * h + 2]), uint32_t(v[4 * h + 3])}); };
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          if (m + 1 < 4) {
-            tlo[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_lo);
-            thi[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_hi);
-          }
+        auto multiply = [&](const u32x4& token, int m, int h) {
 #pragma unroll
           for (int f = 0; f < 4; ++f) {
             v4f t4 = {acc[m][f][0], acc[m][f][1], acc[m][f][2], acc[m][f][3]};
-            t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[f], 0), __builtin_bit_cast(w16_bf16x8, tlo[m & 1]), t4, 0, 0, 0);
-            t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[f], 1), __builtin_bit_cast(w16_bf16x8, thi[m & 1]), t4, 0, 0, 0);
+            t4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[f], h), __builtin_bit_cast(w16_bf16x8, token), t4, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[m][f][r] = t4[r];
           }
-        }
-        if ((kb & 3) == 3 || kb + 1 == KB) {
+        };
+        if constexpr (SPLIT) {
+          u32x4 tok[4];
 #pragma unroll
-          for (int m = 0; m < 4; ++m)
+          for (int m = 0; m < 4; ++m) tok[m] = *reinterpret_cast<const u32x4*>(tl + m * 2048 + rd_lo);
 #pragma unroll
-            for (int f = 0; f < 4; ++f)
+          for (int h = 0; h < 2; ++h) {
 #pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                tot[m][f][r] = __fadd_rn(tot[m][f][r], acc[m][f][r]);
-                acc[m][f][r] = 0.0f;
-              }
+            for (int m = 0; m < 4; ++m) {
+              multiply(tok[m], m, h);
+              if (h == 0) tok[m] = *reinterpret_cast<const u32x4*>(tl + m * 2048 + rd_hi);
+            }
+            if (++steps == part_steps) {
+              steps = 0;
+#pragma unroll
+              for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) {
+                    tot[m][f][r] = __fadd_rn(tot[m][f][r], acc[m][f][r]);
+                    acc[m][f][r] = 0.0f;
+                  }
+            }
+          }
+        } else {
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            if (m + 1 < 4) {
+              tlo[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_lo);
+              thi[(m + 1) & 1] = *reinterpret_cast<const u32x4*>(tl + (m + 1) * 2048 + rd_hi);
+            }
+            multiply(tlo[m & 1], m, 0);
+            multiply(thi[m & 1], m, 1);
+          }
         }
         return;
       }
@@ -219,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
       }
     }
 
-    if constexpr (BF) {
+    if constexpr (SPLIT) {
 #pragma unroll
       for (int m = 0; m < 4; ++m)
 #pragma unroll

@@ -16,9 +16,10 @@ int launch_w8a8_wide(int mode, const GemmParams& p, unsigned blocks, hipStream_t
 // routed row groups of at most 256 rows (mode 0 gate/up, 1 down), units of 128 activation or 256 output columns, those of
 // the *big_groups groups of more than 64 rows first; queue: sixteen words, zero
 int launch_w8a8_cohort(int mode, const GemmParams& p, const uint32_t* big_groups, uint32_t* queue, unsigned blocks, hipStream_t stream);
-// 128 x 128 tiles for E4M3 / E8M0 block-32 weights and activations (a_scales and w*_scales hold scale bytes)
-// and for BF16 weights and activations (a_codes holds BF16 rows, K counts elements; no scales)
-int launch_bf16_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream);
+// 128 x 128 tiles for BF16 weights and activations (a_codes holds BF16 rows, K counts elements; no scales): in one chain, or split, with K a
+// multiple of 256, in the eight partial sums of dense_splitk.cuh
+int launch_bf16_tile(int mode, bool split, const GemmParams& p, unsigned blocks, hipStream_t stream);
+// and for E4M3 / E8M0 block-32 weights and activations (a_scales and w*_scales hold scale bytes)
 int launch_mx_dense_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream);
 // E2M1 / E8M0 row groups of at most 64 tokens (mode 0 gate/up, 1 down), units of 128 activation or 256 output columns
 int launch_mx_tile(int mode, const MxParams& p, unsigned blocks, hipStream_t stream);

@@ -128,6 +128,34 @@ def test_prefill_bf16_shared_expert_tile_kernel_matches_the_float64_sums(rows, h
     assert_close_bf16(bits(op.shared_out), bits((act.double() @ w[2].double().t()).float().to(torch.bfloat16)), "shared expert", max_ulp=1)
 
 
+@pytest.mark.parametrize("rows,hidden,inter", [
+    (129, 256, 256),      # partial sums of one step: two end in every stage
+    (130, 768, 1280),     # of three and five steps: every other one ends inside a stage
+    (200, 1536, 512),     # of six and two
+    (257, 1024, 2048),    # dealt in chunks of 128 columns: one and two chunks a partial sum
+    (140, 7168, 256),     # seven chunks, then one step
+    (300, 1088, 192),     # not a multiple of 256: one chain
+    (4100, 512, 512),     # more tiles than CUs for the grouped kernel: one chain
+])
+def test_prefill_bf16_shared_expert_tile_kernel_equals_the_kernels_it_stands_in_for_bitwise(rows, hidden, inter, monkeypatch):
+    """The order of the FP32 sums is that of the split or the grouped kernel, whichever the shape takes."""
+    table = ops.ExpertTable.allocate(capi.FMT_FP8_CHANNEL, 1, hidden, 128)
+    sh = ops.ExpertTable.allocate(capi.FMT_BF16, 1, hidden, inter)
+    for i, s in enumerate([(inter, hidden), (inter, hidden), (hidden, inter)]):
+        sh.expert_views(0)[2 * i].copy_(synth.normal(s, 0.02, 195 + i).to(torch.bfloat16))
+    x = synth.normal((rows, hidden), 1.0, 198).to(torch.bfloat16).cuda()
+    ids, wt = torch.full((rows, 1), -1, dtype=torch.int32).cuda(), torch.ones((rows, 1)).cuda()
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_BF16_TILE", switch)
+        op = ops.PrefillOps(table, rows, 1, shared=sh.shared_struct(0), act_mode=capi.ACT_BF16)
+        op.contribute(x, ids, wt)
+        torch.cuda.synchronize()
+        out.append((op.scratch_views()["sh_act"].clone().view(torch.int16), op.shared_out.view(torch.int16)))
+    assert torch.equal(out[0][0], out[1][0])
+    assert torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("hidden,inter,counts", [
     (384, 256, [1, 16, 17, 0, 32, 33, 64, 65]),       # every number of live fragments; output columns past the last tile
     (1152, 128, [128, 129, 0, 256, 257, 3]),          # both sides of a 256-row group; nine K blocks, then one
