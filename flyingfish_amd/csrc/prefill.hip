@@ -595,15 +595,35 @@ int launch_mx_dense(const MxParams& p, int mf, unsigned blocks, hipStream_t stre
   return ff_launch_status();
 }
 
-// A dense BF16 expert (the shared expert next to experts of another format) over many rows on the same tiles (FFMOE_BF16_TILE: 1 always,
-// 0 never; same bits). The blocks that split the contraction (dense_splitk.cuh) pass the whole token panel through every block, and the grouped
-// kernel has a wave per SIMD. us gate/up + down, those / tiles: hidden 7168 / intermediate 2048, 128 rows 86 + 36 / 80 + 25, 192 126 + 52 /
-// 80 + 27, 768 494 + 180 / 80 + 33, 1021 122 + 78 / 85 + 36; 7168 / 768, 128 rows 45 + 35 / 80 + 13, 192 85 + 51 / 81 + 14; 2048 / 768, 128
-// rows 18 + 19 / 29 + 13, 192 33 + 19 / 29 + 13.
-bool use_bf16_tiles(int rows) {
+// A dense BF16 expert (the shared expert next to experts of another format) over many rows on the same tiles, per product (mode 0 gate/up,
+// n = its width; 2 down; FFMOE_BF16_TILE: 1 always, 0 never; same bits). A tile walks the whole contraction whatever else there is: 11.3 us
+// (down 6.2) and 9.8 ns per column of it, 1.4 times that for each round of two tiles per CU.
+// Split (dense_splitk.cuh): a round of one block per CU takes 6.3 us and 8.7 per 2048 columns begun (down, two fragments: 5.5 and 10.5), a
+// block whose 64 rows are not all there less. us, those / tiles, gate/up at hidden 7168: one round (512 wide, 256 rows) 46 / 83, with a
+// short second one (768, 160) 63 / 81, two (512, 320) 87 / 83, five (2048, 320) 209 / 79; down, hidden 2048, 129 rows: width 1024 19 / 16,
+// 2048 19 / 24; hidden 7168, 1536 wide, 768 rows 178 / 29.
+// Otherwise the 64-row kernel with one wave per block, for long contractions of gate/up as long as that gives a block per CU (hidden 7168:
+// 1408 wide, 129 rows 72 / 77, 384 rows 80 / 79; 384 wide, 1024 rows 71 / 75, 1500 rows 78 / 77; hidden 4096: 192 wide, 256 rows 42 / 44;
+// 3072: 320 wide, 448 rows 38.6 / 36.5; down at hidden 2048, 1408 wide, 129 rows 16.0 / 16.7, 320 18.3 / 17.0).
+// Up to 128 rows those kernels are ahead or the difference is small (7168 / 2048, 128 rows 86 + 36 / 80 + 25; 7168 / 768 45 + 35 / 80 + 13).
+bool use_bf16_tiles(int mode, int rows, int n, int k, bool splitk) {
   if (const char* f = getenv("FFMOE_BF16_TILE")) return atoi(f) != 0;
-  const char* se = getenv("FFMOE_SHARED_SPLITK");  // 0 asks for the grouped kernels
-  return rows > 128 && !(se && atoi(se) == 0);
+  if (rows <= 128) return false;
+  const int cus = num_cus_p(), rest = rows % 64;
+  const double partial = 0.45 + 0.55 * rest / 64;  // of a block's time, over rest rows
+  if (!splitk) {
+    return !(mode == 0 && k > 3072 && (long long)((rows + 63) / 64) * ((n + 31) / 32) <= cus);
+  }
+  const long long tiles = tile_units(mode, rows, n), columns = n / (mode == 0 ? 8 : 32), full = columns * (rows / 64);
+  const double tile = ((mode == 0 ? 11.3 : 6.2) + 0.0098 * k) * (tiles <= cus ? 1.0 : 1.4 * double((tiles + 2 * cus - 1) / (2 * cus)));
+  double rounds = double((full + cus - 1) / cus);
+  if (rest) {
+    const long long idle = (long long)rounds * cus - full;  // CUs that the last round of full blocks leaves to the others
+    if (columns > 2 * idle) rounds += partial * double((columns - idle + cus - 1) / cus);
+    else if (columns > idle) rounds = std::max(rounds, rounds - 1.0 + 2.0 * partial);
+  }
+  const int chunks = (k + 2047) / 2048;
+  return tile < 3.0 + rounds * (mode == 0 ? 6.3 + 8.7 * chunks : 5.5 + 10.5 * chunks);
 }
 
 struct PrefillLayout {
@@ -693,22 +713,21 @@ int shared_expert_w16(const ffmoe_shared_expert* shared, const void* x, int R, i
   const bool splitk = shared->format == FFMOE_FMT_BF16 && !(se && atoi(se) == 0) && H % 256 == 0 && SI % 256 == 0 &&
                       sgroups * uint32_t((SI + 127) / 128) < (unsigned)num_cus_p();
   // Many rows of either: 128 x 128 tiles, which sum in the order of the kernel that they stand in for
-  if (shared->format == FFMOE_FMT_BF16 && use_bf16_tiles(R)) {
+  const bool bf16 = shared->format == FFMOE_FMT_BF16;
+  auto tiles = [&](int mode, const void* a, uint64_t w0, uint64_t w1, void* out, int n, int k) {
     GemmParams g{};
     g.rows_total = R; g.top_k = 1; g.swiglu = swiglu; g.limit = limit;
-    auto run = [&](int mode) {
-      g.total_units = tile_units(mode, R, g.N);
-      return launch_bf16_tile(mode, splitk, g, std::min<unsigned>((g.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
-    };
-    if (stage_mask & 1) {
-      g.a_codes = (const uint8_t*)x; g.w0_codes = shared->slot[0]; g.w1_codes = shared->slot[2]; g.out = (uint16_t*)act; g.K = H; g.N = SI;
-      FF_TRY(run(0));
-    }
-    if (stage_mask & 2) {
-      g.a_codes = (const uint8_t*)act; g.w0_codes = shared->slot[4]; g.w1_codes = 0; g.out = (uint16_t*)shared_out; g.K = SI; g.N = H;
-      FF_TRY(run(2));
-    }
-    return 0;
+    g.a_codes = (const uint8_t*)a; g.w0_codes = w0; g.w1_codes = w1; g.out = (uint16_t*)out; g.K = k; g.N = n;
+    g.total_units = tile_units(mode, R, n);
+    return launch_bf16_tile(mode, splitk, g, std::min<unsigned>((g.total_units + 7u) & ~7u, unsigned(num_cus_p()) * 2u & ~7u), stream);
+  };
+  if ((stage_mask & 1) && bf16 && use_bf16_tiles(0, R, SI, H, splitk)) {
+    FF_TRY(tiles(0, x, shared->slot[0], shared->slot[2], act, SI, H));
+    stage_mask &= ~1;
+  }
+  if ((stage_mask & 2) && bf16 && use_bf16_tiles(2, R, H, SI, splitk)) {
+    if (stage_mask & 1) FF_TRY(shared_expert_w16(shared, x, R, H, swiglu, limit, act, shared_out, 1, stream_));
+    return tiles(2, act, shared->slot[4], 0, shared_out, H, SI);
   }
   if (splitk) {
     // 8 activation columns (gate + up rows in one fragment) or 16 output columns per block; tiles of half that size, for

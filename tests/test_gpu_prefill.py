@@ -138,7 +138,8 @@ def test_prefill_bf16_shared_expert_tile_kernel_matches_the_float64_sums(rows, h
     (4100, 512, 512),     # more tiles than CUs for the grouped kernel: one chain
 ])
 def test_prefill_bf16_shared_expert_tile_kernel_equals_the_kernels_it_stands_in_for_bitwise(rows, hidden, inter, monkeypatch):
-    """The order of the FP32 sums is that of the split or the grouped kernel, whichever the shape takes."""
+    """The order of the FP32 sums is that of the split or the grouped kernel, whichever the shape takes, also where the two products of the
+    default dispatch run on different kernels (7168 / 256)."""
     table = ops.ExpertTable.allocate(capi.FMT_FP8_CHANNEL, 1, hidden, 128)
     sh = ops.ExpertTable.allocate(capi.FMT_BF16, 1, hidden, inter)
     for i, s in enumerate([(inter, hidden), (inter, hidden), (hidden, inter)]):
@@ -146,14 +147,15 @@ def test_prefill_bf16_shared_expert_tile_kernel_equals_the_kernels_it_stands_in_
     x = synth.normal((rows, hidden), 1.0, 198).to(torch.bfloat16).cuda()
     ids, wt = torch.full((rows, 1), -1, dtype=torch.int32).cuda(), torch.ones((rows, 1)).cuda()
     out = []
-    for switch in ("0", "1"):
-        monkeypatch.setenv("FFMOE_BF16_TILE", switch)
+    for switch in ("0", "1", None):
+        monkeypatch.setenv("FFMOE_BF16_TILE", switch) if switch else monkeypatch.delenv("FFMOE_BF16_TILE")
         op = ops.PrefillOps(table, rows, 1, shared=sh.shared_struct(0), act_mode=capi.ACT_BF16)
         op.contribute(x, ids, wt)
         torch.cuda.synchronize()
         out.append((op.scratch_views()["sh_act"].clone().view(torch.int16), op.shared_out.view(torch.int16)))
-    assert torch.equal(out[0][0], out[1][0])
-    assert torch.equal(out[0][1], out[1][1])
+    for act, y in out[1:]:
+        assert torch.equal(out[0][0], act)
+        assert torch.equal(out[0][1], y)
 
 
 @pytest.mark.parametrize("hidden,inter,counts", [
