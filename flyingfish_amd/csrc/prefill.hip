@@ -537,10 +537,13 @@ bool use_tiles(int mode, int rows, int n, int k, bool mx = false) {
 // The 256 x 256 tile kernel (FFMOE_W8A8_WIDE: 1 wherever the tiles are used, 0 never; same bits) takes 1.83 us per K block and round of one
 // tile per CU, the 128 x 128 one 1.09 per round of two tiles per CU, and its start and end are longer: it wants rounds of the small tiles
 // to fall from at least 8 to 5. 2048 x 2048 -> 7168 (2 rounds to 1) 41.1 -> 32.3 us, 4096 x 2048 -> 7168 (4 to 2) 69.5 -> 62.2; 1024 x 7168 ->
-// 7168 (1 to 1) 59.8 against 85.1. Its token addresses are 32-bit offsets.
+// 7168 (1 to 1) 59.8 against 85.1. A gate/up tile's SwiGLU comes on top, which a short contraction does not outlast: 1024 small
+// tiles (2 to 1) over 128 columns 20.4 -> 21.5, 512 24.9 -> 26.1, 1024 34.0 -> 35.0, 2048 51.3 -> 49.0, 4096 82.9 -> 76.5; plain products gain
+// at any (8192 rows -> 4096 over 128 columns 24.3 -> 21.7). Its token addresses are 32-bit offsets.
 bool use_wide(int mode, const GemmParams& p) {
   if (uint64_t(p.rows_total) * uint64_t(p.K) >= (uint64_t(1) << 32)) return false;
   if (const char* f = getenv("FFMOE_W8A8_WIDE")) return atoi(f) != 0;
+  if (mode == 0 && p.K <= 1536) return false;
   const uint32_t cus = uint32_t(num_cus_p());
   const uint32_t small = (tile_units(mode, p.rows_total, p.N) + 2 * cus - 1) / (2 * cus), large = (wide_units(mode, p.rows_total, p.N) + cus - 1) / cus;
   return 5 * small >= 8 * large;
