@@ -754,22 +754,39 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_route_logits_bf16(co
   return ff_launch_status();
 }
 
+// k_route_logits_f32_rows: a block takes LG_MR * LG_TEAMS rows per pass and one block fits a CU: as many row chunks as keep the grid within
+// one round of blocks, eight (one per XCD) for a cohort
+static int logit_row_chunks(int rows, int etiles) {
+  return std::max(1, std::min(decode_cus() / etiles, (rows + LG_MR * LG_TEAMS - 1) / (LG_MR * LG_TEAMS)));
+}
+
+// Whether the matrix cores take less time than k_route_logits_f32_rows, by what either is made of: the chains' turns (vectors of one chain:
+// 2048 columns begun are one more), the vector kernel's passes of its blocks, the rounds of two matrix tiles (16 rows x 64 experts) per CU
+// or of one where that is all there is. 653 sizes from 8 experts at 512 to 1024 at 7168: within 15 % of the time for nearly all, no choice
+// more than 3 % behind the vector kernel. us back to back, vector / matrix: 64 experts at hidden 512, 2048 rows 14.2 / 20.1, 4096 26.2 / 20.1;
+// 256 at 2048, 768 rows 19.7 / 20.4, 1024 29 / 21; 64 at 7168, 2048 rows 42 / 56, 4096 78 / 57; 256 at 7168, 768 rows 55 / 56, 1024 78 / 57,
+// 1500 102 / 92, 4096 264 / 171 (inside a layer, at the lower clock that a launch finds there, 300 / 218).
+static bool logits_matrix_pays(int rows, int experts, int hidden) {
+  const int cus = decode_cus(), turns = (hidden + 2047) / 2048;
+  const int etiles = (experts + LG_ME - 1) / LG_ME, chunks = logit_row_chunks(rows, etiles);
+  const int passes = ((rows + chunks - 1) / chunks + LG_MR * LG_TEAMS - 1) / (LG_MR * LG_TEAMS);
+  const double vector = 2.5 + 0.00056 * hidden + double((etiles * chunks + cus - 1) / cus) * passes * (1.5 + 2.6 * turns);
+  const long long tiles = (long long)((rows + 15) / 16) * ((experts + 63) / 64), full = tiles / (2 * cus), rest = tiles % (2 * cus);
+  const double one = 8.4 + 11.85 * turns, two = 9.0 + 20.7 * turns;  // a round of one, two tiles per CU
+  const double matrix = 0.12 * (tiles <= cus ? one : two) + 0.88 * (double(full) * two + (rest > cus ? two : rest > 0 ? one : 0.0));
+  return vector > 1.03 * matrix;
+}
+
 extern "C" __attribute__((visibility("default"))) int ffmoe_route_logits_f32(const void* x, const void* router, float* logits, int rows, int experts, int hidden,
                                       void* stream) {
   FF_TRY(check_route_dims(rows, experts, hidden));
   FF_PTR16(x); FF_PTR16(router); FF_PTR4(logits);
   FF_NO_OVERLAP(logits, size_t(rows) * experts * 4, x, size_t(rows) * hidden * 2);
   FF_NO_OVERLAP(logits, size_t(rows) * experts * 4, router, size_t(experts) * hidden * 2);
-  // Very many rows: the matrix cores (FFMOE_ROUTE_LOGITS_MFMA: 1 wherever they can run, 0 never; same bits). A tile of 16 rows x 64 experts
-  // takes 4 us + 7.3 ns per column where a CU has one, 1.62 times that where it has two; the vector kernel 6 us + 3.4 us per 100 M fmas. us,
-  // vector / matrix: 64 experts at 7168, 2048 rows (one tile on half the CUs) 42 / 56, 4096 77 / 57; 128 at 2048, 1500 rows 21.0 / 21.0,
-  // 2048 29 / 21; 256 at 7168, 768 rows 56 / 57, 1024 75 / 57, 1500 97 / 92.
+  // Very many rows: the matrix cores (FFMOE_ROUTE_LOGITS_MFMA: 1 wherever they can run, 0 never; same bits)
   {
     const char* e = getenv("FFMOE_ROUTE_LOGITS_MFMA");
-    const long long tiles = (long long)((rows + 15) / 16) * ((experts + 63) / 64), cus = decode_cus();
-    const double matrix = (4.0 + 0.0073 * hidden) * (tiles <= cus ? 1.0 : 1.62 * double((tiles + 2 * cus - 1) / (2 * cus)));
-    const double vector = 6.0 + 3.4e-8 * double(rows) * double(experts) * double(hidden);
-    if (hidden % 32 == 0 && uint64_t(experts) * uint64_t(hidden) * 2 < (uint64_t(1) << 32) && (e ? atoi(e) != 0 : vector > 1.05 * matrix)) {
+    if (hidden % 32 == 0 && uint64_t(experts) * uint64_t(hidden) * 2 < (uint64_t(1) << 32) && (e ? atoi(e) != 0 : logits_matrix_pays(rows, experts, hidden))) {
       static const hipError_t ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_route_logits_f32_mfma), hipFuncAttributeMaxDynamicSharedMemorySize, LGM_LDS);
       if (ok == hipSuccess) {
         hipLaunchKernelGGL(k_route_logits_f32_mfma, dim3((rows + 15) / 16, (experts + 63) / 64), dim3(256), LGM_LDS, (hipStream_t)stream,
@@ -788,12 +805,7 @@ extern "C" __attribute__((visibility("default"))) int ffmoe_route_logits_f32(con
       if (lds_ok < 0)
         lds_ok = hipFuncSetAttribute(reinterpret_cast<const void*>(k_route_logits_f32_rows), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) == hipSuccess ? 1 : 0;
       if (lds_ok == 1) {
-        const int etiles = (experts + LG_ME - 1) / LG_ME;
-        // a block takes LG_MR * LG_TEAMS rows per pass and one block fits a CU: as many row chunks as keep the grid within
-        // one round of blocks, eight (one per XCD) for a cohort
-        const int per_pass = LG_MR * LG_TEAMS;
-        const int max_chunks = std::max(1, decode_cus() / etiles);
-        const int row_chunks = std::max(1, std::min(max_chunks, (rows + per_pass - 1) / per_pass));
+        const int etiles = (experts + LG_ME - 1) / LG_ME, row_chunks = logit_row_chunks(rows, etiles);
         hipLaunchKernelGGL(k_route_logits_f32_rows, dim3(unsigned(etiles) * unsigned(row_chunks)), dim3(256 * LG_TEAMS), lds, (hipStream_t)stream,
                            (const uint16_t*)x, (const uint16_t*)router, logits, rows, experts, hidden, row_chunks);
         return ff_launch_status();
