@@ -29,7 +29,11 @@ constexpr int WIDE_LAG = 3;  // matrix instructions between a product and its fm
 // their rows, MODE 1 weights its results and scatters them to their assignments).
 template <int MODE, bool GROUPED>
 __device__ __forceinline__ void wide_tile(const GemmParams& p, uint8_t* lds, int t, int start, int n, const uint64_t (&wc)[2], const uint64_t (&ws)[2]) {
-    const int tid = threadIdx.x, lane = tid & 63;
+    // What follows from the thread's index is worked out again for every unit: kept from unit to unit it spilled, and a launch with a scratch
+    // segment starts later (cohort kernel, 36 bytes per lane: a layer of 64 small groups at 4096 / 1536 253 us, 248 without)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const int wave = uni(tid >> 6);
     const int wr = wave >> 2, wt = wave & 3;  // weight half (128 rows), token quarter (64 tokens)
     const int K = p.K, N = p.N, KB = K >> 7;
@@ -305,7 +309,9 @@ template <int MODE, int MF>
 __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, int t, int start, int n, const uint64_t (&wc)[2], const uint64_t (&ws)[2]) {
   using Stage = StreamStage<MF>;
   constexpr int NS = stream_stages<MF>();
-  const int tid = threadIdx.x, lane = tid & 63;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // as in wide_tile
+  const int lane = tid & 63;
   const int wave = uni(tid >> 6);
   const int K = p.K, N = p.N, KB = K >> 7;
   const uint32_t lds0 = lds_address(lds);
