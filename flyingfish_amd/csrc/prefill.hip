@@ -73,18 +73,18 @@ __global__ __launch_bounds__(256) void k_prefill_count(const LiveTest t, uint32_
 // shared_rows > 0 appends the always-on expert as groups of expert id `experts` over rows 0 .. shared_rows - 1, their units
 // behind the routed ones (column tile outermost, so the row groups of a tile are neighbours and share its weights in L2):
 // the launches that run the routed experts then run the shared one as well.
-// Row groups of an expert with c rows: of tm rows, or (tm == 0) of 256 rows while more than 128 are left and of 64 rows for the rest. A
-// 256-row tile takes 3500 cycles per K block whatever its group holds, a 64-row group 2100 to 2600 (its share of the weight stream, or less where
-// it follows another of its expert): 4096 tokens 3.70 ms, with 64-row groups up to 192 rows 3.88.
-// The 256-row groups of all experts come first in the group and unit lists, the 64-row groups behind them; an expert's two counts share a
-// word (at most two small groups per expert), and so do their prefix sums.
+// Row groups of an expert with c rows: of tm rows, or (tm == 0) of 256 rows while more than 128 are left and one of the rest. A
+// 256-row tile takes 3500 cycles per K block whatever its group holds, a stream of up to 128 rows 2100 to 2800 (its share of the weight
+// stream).
+// The 256-row groups of all experts come first in the group and unit lists, the small groups behind them; an expert's two counts share a
+// word (at most one small group per expert), and so do their prefix sums.
 constexpr uint32_t SMALL_BITS = 12;
-static_assert(2 * FFMOE_MAX_EXPERTS < (1 << SMALL_BITS), "prefix sums of the small groups");
+static_assert(FFMOE_MAX_EXPERTS < (1 << SMALL_BITS), "prefix sums of the small groups");
 __device__ __forceinline__ uint32_t big_groups(uint32_t c) { return (c + 127u) / 256u; }
 __device__ __forceinline__ uint32_t group_count(uint32_t c, int tm) {
   if (tm > 0) return (c + tm - 1) / tm;
   const uint32_t big = big_groups(c);
-  return (big << SMALL_BITS) | (big * 256u >= c ? 0u : (c - big * 256u + 63u) / 64u);
+  return (big << SMALL_BITS) | (big * 256u >= c ? 0u : 1u);
 }
 // first row (of the expert's) and rows of group q among `total` groups, its expert and that expert's first row
 __device__ __forceinline__ GemmGroup group_of(const uint32_t* s_rows, const uint32_t* s_groups, int experts, int tm, uint32_t q) {
@@ -95,7 +95,7 @@ __device__ __forceinline__ GemmGroup group_of(const uint32_t* s_rows, const uint
   int lo = 0, hi = experts;  // last e with its first group <= key
   while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (field(s_groups[mid]) <= key) lo = mid; else hi = mid; }
   const uint32_t i = key - field(s_groups[lo]), c = s_rows[lo + 1] - s_rows[lo];
-  const uint32_t size = tm > 0 ? uint32_t(tm) : big ? 256u : 64u;
+  const uint32_t size = tm > 0 ? uint32_t(tm) : big ? 256u : 128u;
   const uint32_t first = (tm > 0 || big ? 0u : big_groups(c) * 256u) + i * size;
   GemmGroup gd;
   gd.expert = lo; gd.start = int(s_rows[lo] + first); gd.n = int(min(size, c - first)); gd.pad = 0;
@@ -568,14 +568,20 @@ int launch_tiles(int mode, const MxParams& q, hipStream_t stream) {
 
 // A W8A8 prompt chunk's routed experts on the cohort kernel (wide_gemm.cuh; FFMOE_W8A8_COHORT: 1 wherever it can run, 0 never; same bits).
 // Its units are large and a CU runs one at a time: it wants contractions that outlast a unit's start and end (about ten K blocks of time)
-// and enough units per CU. us per layer, 64-row kernel / this one, Zipf-like routing:
-//   rows                              65            128           256           512           1024          4096
-//   top-8 of 256, 7168 / 2048    1022 /  935   1425 / 1266   1649 / 1475   2014 / 1875   2347 / 2184   4027 / 3634
-//   top-6 of 64, 4096 / 1536      311 /  283    336 /  315    354 /  345    413 /  376    504 /  482   1100 /  985
-//   top-8 of 128, 2048 / 1408     181 /  176    200 /  199    253 /  237    320 /  295    398 /  344
-//   top-6 of 64, 3072 / 1024      188 /  187    203 /  206    242 /  228    264 /  246    341 /  303     (2.0 - 2.8 gate/up units per CU)
-//   top-4 of 64, 4096 / 768       188 /  192    200 /  205    223 /  238    242 /  267    306 /  289     (1.6 - 1.9)
-//   top-8 of 256, 2048 / 768      136 /  157    150 /  172    200 /  197    232 /  233    309 /  300     (16 and 6 K blocks)
+// and enough units per CU. us per call, 64-row kernel / this one, Zipf-like and even routing:
+//   rows                                  65            128           256           512           1024          2048          4096
+//   top-8 of 256, 7168 / 2048   Zipf 1095 /  993   1406 / 1270   1754 / 1587   1990 / 1828   2228 / 2018   2568 / 2309   3494 / 2830
+//                               even 1592 / 1451   1870 / 1721   1915 / 1756   1971 / 1823   2060 / 1952   2493 / 2228   3333 / 2978
+//   top-6 of 64, 4096 / 1536    Zipf  259 /  234    283 /  252    292 /  275    344 /  291    370 /  364    590 /  503    973 /  775
+//                               even  263 /  255    260 /  252    275 /  266    319 /  287    363 /  336    583 /  471    975 /  783
+//   top-8 of 128, 2048 / 1408   Zipf  212 /  198    237 /  228    279 /  245    293 /  262    344 /  309    459 /  415    747 /  599
+//   top-6 of 64, 3072 / 1024    Zipf  144 /  143    155 /  160    189 /  180    214 /  190    272 /  224    356 /  324    570 /  466
+//                               even  142 /  157    148 /  159    159 /  167    217 /  183    220 /  218    359 /  300    572 /  477
+//   top-4 of 64, 4096 / 768     Zipf  128 /  137    148 /  161    167 /  188    177 /  209    251 /  225    267 /  278    434 /  405
+//                               even  139 /  152    141 /  153    152 /  160    166 /  175    249 /  203    261 /  289    435 /  373
+// (3072 / 1024: 2.0 - 2.8 gate/up units per CU; 4096 / 768: 1.6 - 1.9; both go over at 1024 and 1500 rows.) The estimate takes every choice
+// for a live one: where seven of eight are not (experts that live elsewhere), those two narrow layers are 3 to 6 % behind at 1024 rows
+// and more.
 // The group sizes and orders that the environment asks for are the 64-row kernel's.
 bool use_cohort(int rows, int top_k, int experts, int hidden, int inter) {
   const uint64_t A = uint64_t(rows) * uint64_t(top_k), limit = uint64_t(1) << 32;
@@ -902,9 +908,9 @@ int prefill_impl(const ffmoe_expert_table* table, const ffmoe_prefill* args, int
   const bool nv_tile = a16 && table->format == FFMOE_FMT_NVFP4 && nvfp4_lines_enabled() && nvfp4_tiles(R, K, E, I) && H % 256 == 0 && I % 256 == 0;
   const int mf = nv ? 4 : pick_mf(double(A) / E, (mx || a16) ? 4 : 8, (!mx && !a16) || mx || nv_tile);
   // W8A8 and W*A16 cohorts in 64-row groups: eight waves per block share a token tile (FFMOE_PREFILL_WIDE=0: four, two blocks per CU)
-  // W8A8 of a prompt chunk: groups of up to 256 and 64 rows on the cohort kernel (wide_gemm.cuh)
+  // W8A8 of a prompt chunk: groups of up to 256 and 128 rows on the cohort kernel (wide_gemm.cuh)
   const bool cohort = !mx && !a16 && !nv && use_cohort(R, K, E, H, I);
-  const int tm = cohort ? 0 : 16 * mf;  // 0: k_prefill_plan's groups of 256 and 64
+  const int tm = cohort ? 0 : 16 * mf;  // 0: k_prefill_plan's groups of 256 and 128
   bool wide = mf == 4 && !mx && !nv_tile && !cohort;
   if (const char* f = getenv("FFMOE_PREFILL_WIDE")) wide = (wide && atoi(f) != 0) || nv;
   const int tiles0 = wide ? (I + 255) / 256 : (I + 127) / 128, tiles1 = wide ? (H + 511) / 512 : (H + 255) / 256;

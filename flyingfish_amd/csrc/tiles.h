@@ -14,7 +14,7 @@ int launch_w8a8_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t
 inline uint32_t wide_units(int mode, int rows, int n) { return uint32_t((rows + 255) / 256) * uint32_t(mode == 0 ? (n + 127) / 128 : (n + 255) / 256); }
 int launch_w8a8_wide(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream);
 // routed row groups of at most 256 rows (mode 0 gate/up, 1 down), units of 128 activation or 256 output columns, those of
-// the *big_groups groups of more than 64 rows first; queue: sixteen words, zero
+// the *big_groups groups of more than 128 rows first; queue: sixteen words, zero
 int launch_w8a8_cohort(int mode, const GemmParams& p, const uint32_t* big_groups, uint32_t* queue, unsigned blocks, hipStream_t stream);
 // 128 x 128 tiles for BF16 weights and activations (a_codes holds BF16 rows, K counts elements; no scales): in one chain, or split, with K a
 // multiple of 256, in the eight partial sums of dense_splitk.cuh

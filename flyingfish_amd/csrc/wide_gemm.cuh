@@ -294,16 +294,20 @@ __global__ __launch_bounds__(512, 2) void k_w8a8_wide(const GemmParams p) {
 }
 
 // ---- cohorts: token groups of a routed layer ---------------------------------------------------------------------------
-// Popular experts come in groups of up to 256 tokens, which run the tile above; the rest of an expert's tokens in groups of up to 64, which
-// stream the expert's weights past their live 16-token fragments (k_w8a8_cohort). 4096 tokens, top-8 of 256 experts at hidden 7168 /
+// Popular experts come in groups of up to 256 tokens, which run the tile above; the rest of an expert's tokens, up to 128, are one group, which
+// streams the expert's weights past its live 16-token fragments (k_w8a8_cohort). 4096 tokens, top-8 of 256 experts at hidden 7168 /
 // intermediate 2048, Zipf-like: gate/up 2197 -> 1800 us, down 1280 -> 1080 us against 64-row groups throughout; 65 tokens, all stream: a
 // layer 1022 -> 935 us. What bounds it: a tile is at 3500 of 2048 cycles per K block, a stream's share of memory gives it a K block of 32 KB
 // every 2200 cycles; between units a block waits for claims, descriptors and first operands (6000 cycles) and drains (a gate/up tile's SwiGLU 20000).
+// Two groups of 64 for the rest fetch the weights twice, too far apart to share them: evenly routed chunks of 64 to 128 tokens per expert were 10 to
+// 25 % behind the 64-row kernel, whose two groups run side by side. us per call, that one / two groups / one, even: 1024 tokens, top-6 of 64
+// at 4096 / 1536 360 / 456 / 338; 2048, top-8 of 256 at 7168 / 2048 2485 / 2761 / 2229; Zipf-like, 4096 of the latter 3424 / 3003 / 2835. The
+// larger groups in one list with the tiles, so that they start first: 2973 there.
 // Stage of a group of up to 16 MF tokens: a K block of 256 weight rows (32 per wave) and of the tokens; a ring of STAGES of them.
 template <int MF> struct StreamStage { uint8_t w[256 * 128]; uint8_t t[MF * 16 * 128]; };
 template <int MF> constexpr int stream_stages() { return MF > 2 ? 3 : 4; }
-constexpr int COHORT_SX = 4 * int(sizeof(StreamStage<2>)), COHORT_LDS = COHORT_SX + 2 * 64 * 8 * 4 + 16;  // the scales of eight K blocks, twice; the claim
-static_assert(WIDE_LDS <= COHORT_SX && 3 * int(sizeof(StreamStage<4>)) <= COHORT_SX && 4 * int(sizeof(StreamStage<1>)) <= COHORT_SX && COHORT_LDS <= 160 * 1024, "one block per CU");
+constexpr int COHORT_SX = 4 * int(sizeof(StreamStage<2>)), STREAM_SX = 128 * 8 * 4, COHORT_LDS = COHORT_SX + 2 * STREAM_SX + 16;  // the scales of eight K blocks, twice; the claim
+static_assert(WIDE_LDS <= COHORT_SX && 3 * int(sizeof(StreamStage<8>)) <= COHORT_SX && 4 * int(sizeof(StreamStage<1>)) <= COHORT_SX && COHORT_LDS <= 160 * 1024, "one block per CU");
 
 template <int MODE, int MF>
 __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, int t, int start, int n, const uint64_t (&wc)[2], const uint64_t (&ws)[2]) {
@@ -328,12 +332,17 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, i
   const float* sw0 = reinterpret_cast<const float*>(ws[0]) + size_t(min(column(0), N - 16) >> 7) * KB;
   const float* sw1 = reinterpret_cast<const float*>(ws[1]) + size_t(min(column(0), N - 16) >> 7) * KB;
   float swl0 = load_global<float>(sw0 + min(lane, KB - 1)), swl1 = MODE == 0 ? load_global<float>(sw1 + min(lane, KB - 1)) : 0.0f;
-  const bool mover = wave < 2 * MF;  // the waves that fetch eight tokens each
-  uint32_t toff = 0;
-  if (mover) {
-    const int pos = start + min(wave * 8 + (lane >> 3), n - 1);
-    const int row = MODE == 0 ? load_global<int>(p.perm + pos) / p.top_k : pos;
-    toff = uint32_t(row) * uint32_t(K) + (piece ^ (64u * (wave & 1)));
+  constexpr int TR = MF > 4 ? 2 : 1;  // token requests of a wave, of eight tokens each
+  const bool mover = wave * TR < 2 * MF;  // the waves that make them
+  uint32_t toff[TR];
+#pragma unroll
+  for (int i = 0; i < TR; ++i) {
+    toff[i] = 0;
+    if (mover) {
+      const int q = wave * TR + i, pos = start + min(q * 8 + (lane >> 3), n - 1);
+      const int row = MODE == 0 ? load_global<int>(p.perm + pos) / p.top_k : pos;
+      toff[i] = uint32_t(row) * uint32_t(K) + (piece ^ (64u * (q & 1)));
+    }
   }
   swl0 = landed(swl0);
   if (MODE == 0) swl1 = landed(swl1);
@@ -343,8 +352,12 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, i
     for (int i = 0; i < 4; ++i)
       lds_load16_nt(at + uint32_t(wave) * 4096u + i * 1024u, wbase[i >> 1] + uint64_t(uint32_t(q) * 128u) + ((i & 1) ? 8u * uint64_t(K) : 0u), woff ^ (64u * (i & 1)));
     if (mover) {
-      if ((q & 7) == 0) lds_load4(lds0 + uint32_t(COHORT_SX) + uint32_t((q >> 3) & 1) * 2048u + uint32_t(wave) * 256u, p.a_scales + (toff >> 7) + min(q + (lane & 7), KB - 1));
-      lds_load16(at + uint32_t(offsetof(Stage, t)) + uint32_t(wave) * 1024u, uint64_t(uintptr_t(p.a_codes)) + uint64_t(uint32_t(q) * 128u), toff);
+#pragma unroll
+      for (int i = 0; i < TR; ++i) {
+        const uint32_t t8 = uint32_t(wave) * TR + i;
+        if ((q & 7) == 0) lds_load4(lds0 + uint32_t(COHORT_SX) + uint32_t((q >> 3) & 1) * uint32_t(STREAM_SX) + t8 * 256u, p.a_scales + (toff[i] >> 7) + min(q + (lane & 7), KB - 1));
+        lds_load16(at + uint32_t(offsetof(Stage, t)) + t8 * 1024u, uint64_t(uintptr_t(p.a_codes)) + uint64_t(uint32_t(q) * 128u), toff[i]);
+      }
     }
   };
   float acc[MF][2][4];
@@ -363,7 +376,7 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, i
   for (int kb = 0; kb < KB; ++kb) {
     // K block kb has landed: behind it the requests of NS - 2 later ones (and scales now and then: the wait is one request stricter then)
     if (kb + NS - 2 < KB) {
-      if (mover) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 5) : "memory");
+      if (mover) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * (4 + TR)) : "memory");
       else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 4) : "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -382,7 +395,7 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, i
       const u32x4 lo = *reinterpret_cast<const u32x4*>(base + rd_lo), hi = *reinterpret_cast<const u32x4*>(base + rd_hi);
       return v8i{int(lo[0]), int(lo[1]), int(lo[2]), int(lo[3]), int(hi[0]), int(hi[1]), int(hi[2]), int(hi[3])};
     };
-    const float* sl = reinterpret_cast<const float*>(lds + COHORT_SX + ((kb >> 3) & 1) * 2048) + r16 * 8 + (kb & 7);
+    const float* sl = reinterpret_cast<const float*>(lds + COHORT_SX + ((kb >> 3) & 1) * STREAM_SX) + r16 * 8 + (kb & 7);
     v8i wf[2];
 #pragma unroll
     for (int f = 0; f < 2; ++f) wf[f] = read(st + wave * 4096 + f * 2048);
@@ -445,7 +458,7 @@ __device__ __forceinline__ void stream_tile(const GemmParams& p, uint8_t* lds, i
 template <int MODE>
 __global__ __launch_bounds__(512, 2) void k_w8a8_cohort(const GemmParams p, const uint32_t* big_groups, uint32_t* queue) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  uint32_t* const s_claim = reinterpret_cast<uint32_t*>(lds + COHORT_SX + 4096);
+  uint32_t* const s_claim = reinterpret_cast<uint32_t*>(lds + COHORT_SX + 2 * STREAM_SX);
   const int tid = threadIdx.x;
   const uint32_t tiles = uint32_t(p.N + (MODE == 0 ? 127 : 255)) / (MODE == 0 ? 128u : 256u);
   const uint32_t split = load_uniform<uint32_t>(big_groups) * tiles, total = load_uniform<uint32_t>(p.unit_total);
@@ -478,7 +491,9 @@ __global__ __launch_bounds__(512, 2) void k_w8a8_cohort(const GemmParams p, cons
       const uint64_t* sl = p.slots + size_t(expert) * 6 + (MODE == 0 ? 0 : 4);
       const uint64_t wc[2] = {load_uniform<uint64_t>(sl), load_uniform<uint64_t>(sl + (MODE == 0 ? 2 : 0))};
       const uint64_t ws[2] = {load_uniform<uint64_t>(sl + 1), load_uniform<uint64_t>(sl + (MODE == 0 ? 3 : 1))};
-      if (n > 64) wide_tile<MODE, true>(p, lds, t, start, n, wc, ws);
+      if (n > 128) wide_tile<MODE, true>(p, lds, t, start, n, wc, ws);
+      else if (n > 96) stream_tile<MODE, 8>(p, lds, t, start, n, wc, ws);
+      else if (n > 64) stream_tile<MODE, 6>(p, lds, t, start, n, wc, ws);
       else if (n > 32) stream_tile<MODE, 4>(p, lds, t, start, n, wc, ws);
       else if (n > 16) stream_tile<MODE, 2>(p, lds, t, start, n, wc, ws);
       else stream_tile<MODE, 1>(p, lds, t, start, n, wc, ws);

@@ -163,6 +163,7 @@ def test_prefill_bf16_shared_expert_tile_kernel_equals_the_kernels_it_stands_in_
     (1152, 128, [128, 129, 0, 256, 257, 3]),          # both sides of a 256-row group; nine K blocks, then one
     (256, 384, [1000, 385, 2, 448]),                  # several 256-row groups, with and without a rest
     (8320, 128, [5, 130, 40]),                        # 65 K blocks
+    (640, 384, [80, 81, 95, 96, 97, 111, 127, 128, 330, 384]),  # both sizes of a group of more than 64, alone and behind 256 rows
     (128, 2048, [300] * 24 + [20] * 40),              # more units of both kinds than blocks start on
 ])
 def test_prefill_cohort_kernel_equals_the_group_kernel_bitwise(hidden, inter, counts, monkeypatch):
