@@ -124,7 +124,7 @@ __device__ __forceinline__ float det_expf(float x) {
   return y;
 }
 
-// The same for x <= 0, without branches; a NaN stays one.
+// The same for x <= 0, without branches. A NaN gives 0: the caller looks for it.
 __device__ __forceinline__ float det_expf_neg(float x) {
   const float magic = 12582912.0f;
   const float c = fmaxf(x, -105.0f);  // in range for the arithmetic; the result is replaced below
@@ -222,7 +222,7 @@ __device__ __forceinline__ float silu_two_branch(float g) {
   const bool pos = g >= 0.0f;
   const float e = det_expf_neg(pos ? -g : g);
   const float y = __fmul_rn(g, div_by_1_to_2(pos ? 1.0f : e, __fadd_rn(1.0f, e)));
-  return g == g ? y : __fadd_rn(g, g);  // the remainders negate a NaN
+  return g == g ? y : __fadd_rn(g, g);  // a NaN went through the exponential as 0
 }
 __device__ __forceinline__ uint16_t swiglu_bf16_two_branch(float g, float u, int mode, float limit) {
   if (mode >= 2) {

@@ -184,6 +184,23 @@ def test_route_logits_f32_matrix_core_path_bit_exact(rows, experts, hidden, monk
     assert np.array_equal(got, out())
 
 
+def test_route_logits_f32_matrix_core_path_keeps_subnormals(monkeypatch):
+    """Rows whose products, chains and logits are subnormal, and chains that start subnormal and end normal: a unit that flushed them would
+    give zeros."""
+    hidden, experts = 7168, 70
+    x, r = rand_bf16((20, hidden), 1.0, 71), rand_bf16((experts, hidden), 0.5, 72)
+    x[:10] *= 2.0 ** -70
+    r[:40] *= 2.0 ** -66
+    x[10], r[40:44] = 2.0 ** -64, 2.0 ** -64  # equal products of 2^-128: sums cross 2^-126 after the fourth
+    monkeypatch.setenv("FFMOE_ROUTE_LOGITS_MFMA", "1")
+    got = RouteOps.logits_f32(x.to(DEV), r.to(DEV)).cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), orc.route_logits_f32(bits(x), bits(r)).view(np.uint32))
+    small = np.abs(got[:10, :40])
+    assert np.all((small > 0) & (small < 2.0 ** -126)) and np.all(got[10, 40:44] == hidden * 2.0 ** -128)
+    monkeypatch.setenv("FFMOE_ROUTE_LOGITS_MFMA", "0")
+    assert np.array_equal(got.view(np.uint32), RouteOps.logits_f32(x.to(DEV), r.to(DEV)).cpu().numpy().view(np.uint32))
+
+
 @pytest.mark.parametrize("score", [capi.SCORE_SOFTMAX, capi.SCORE_SIGMOID])
 @pytest.mark.parametrize("rows,experts,top_k", [(4, 64, 4), (3, 256, 8), (2, 1000, 32), (5, 48, 6)])
 def test_route_topk_bit_exact(score, rows, experts, top_k):

@@ -105,6 +105,55 @@ def test_prefill_shared_expert_wide_tile_kernel_equals_the_tile_kernel_bitwise(r
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+def test_wide_tile_kernel_with_several_tiles_per_block_equals_the_tile_kernel_bitwise(monkeypatch):
+    """More tiles than CUs over nine K blocks, plain and gate/up: a block's second tile follows a full contraction and its epilogue."""
+    monkeypatch.setenv("FFMOE_W8A8_TILE", "1")
+    rows, hidden, inter = 4200, 1152, 2176
+    table, _ = make_table(capi.FMT_FP8_BLOCK128, 2, hidden, inter, 83)
+    shared = table.shared_struct(1)
+    table.experts = 1
+    x = synth.normal((rows, hidden), 1.0, 84).to(torch.bfloat16).cuda()
+    ids, wt = torch.full((rows, 1), -1, dtype=torch.int32).cuda(), torch.ones((rows, 1)).cuda()
+    wc, ws = _fp8_matrix(4400, hidden, 85)
+    out = []
+    for switch in ("0", "1"):
+        monkeypatch.setenv("FFMOE_W8A8_WIDE", switch)
+        op = ops.PrefillOps(table, rows, 1, shared=shared)
+        op.contribute(x, ids, wt)
+        y = ops.Fp8Ops.linear(wc.cuda(), ws.cuda(), x, capi.ACT_FP8_BLOCK128)
+        torch.cuda.synchronize()
+        out.append([v.view(torch.int16) for v in (op.scratch_views()["sh_act"].clone(), op.shared_out, y)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("cohort", ["0", "1"])
+def test_prefill_w8a8_swiglu_of_infinities_and_nan(cohort, monkeypatch):
+    """Gates of +inf, -inf, NaN and zero: the bits of the sigmoid's two branches, NaN where they give one."""
+    hidden = inter = 128
+    table, ref = make_table(capi.FMT_FP8_BLOCK128, 1, hidden, inter, 86)
+    v = table.expert_views(0)
+    codes = torch.zeros((inter, hidden), dtype=torch.uint8)
+    codes[0:32], codes[32:64], codes[64:96] = 0x7e, 0xfe, 0x7f
+    v[0].copy_(codes.view(v[0].dtype))
+    v[1].fill_(3e38)
+    x = torch.ones((3, hidden), dtype=torch.bfloat16)
+    monkeypatch.setenv("FFMOE_W8A8_COHORT", cohort)
+    op = ops.PrefillOps(table, 3, 1)
+    op.contribute(x.cuda(), torch.zeros((3, 1), dtype=torch.int32).cuda(), torch.ones((3, 1)).cuda())
+    torch.cuda.synchronize()
+    act = bits(op.scratch_views()["act"].cpu().view(torch.bfloat16).reshape(3, inter))
+    gate = torch.zeros(inter)
+    gate[0:32], gate[32:64], gate[64:96] = float("inf"), -float("inf"), float("nan")
+    up = (x[:1].double() @ torch.from_numpy(ref[0][1].astype(np.int32) << 16).view(torch.float32).double().t())[0]
+    want = orc.silu_mul(bits(gate.to(torch.bfloat16)), bits(up.float().to(torch.bfloat16)), orc.TWICE, kind=orc.SILU_SIGMOID2)
+    nan = lambda b: (b & 0x7fff) > 0x7f80
+    assert nan(want)[32:96].all() and not nan(want)[0:32].any() and not nan(want)[96:].any()
+    for row in act:
+        assert np.array_equal(nan(row), nan(want))
+        assert np.array_equal(row[~nan(want)], want[~nan(want)])
+
+
 @pytest.mark.parametrize("rows,hidden,inter", [(1, 256, 128), (129, 192, 128), (130, 320, 192), (300, 1024, 256)])
 def test_prefill_bf16_shared_expert_tile_kernel_matches_the_float64_sums(rows, hidden, inter, monkeypatch):
     """Ragged rows and columns, one stage and numbers of stages that do not fill a fold; stage by stage against FP64 with the same BF16
@@ -165,9 +214,11 @@ def test_prefill_bf16_shared_expert_tile_kernel_equals_the_kernels_it_stands_in_
     (8320, 128, [5, 130, 40]),                        # 65 K blocks
     (640, 384, [80, 81, 95, 96, 97, 111, 127, 128, 330, 384]),  # both sizes of a group of more than 64, alone and behind 256 rows
     (128, 2048, [300] * 24 + [20] * 40),              # more units of both kinds than blocks start on
+    (1152, 1152, [300] * 30 + [100] * 10 + [20] * 10),  # in both launches, over nine K blocks: units of all kinds behind one another in a block
 ])
 def test_prefill_cohort_kernel_equals_the_group_kernel_bitwise(hidden, inter, counts, monkeypatch):
-    """The groups of 256 and 64 rows at their edges; a stage repeated without a plan finds its claim counters at zero again."""
+    """The groups of 256 and 128 rows at their edges; a stage repeated without a plan finds its claim counters at zero again (a claim that
+    finds them elsewhere leaves its unit's rows as they are: NaN)."""
     experts, rows = len(counts), sum(counts) + 3
     table, _ = make_table(capi.FMT_FP8_BLOCK128, experts, hidden, inter, 91)
     x = synth.normal((rows, hidden), 1.0, 92).to(torch.bfloat16).cuda()
@@ -181,6 +232,14 @@ def test_prefill_cohort_kernel_equals_the_group_kernel_bitwise(hidden, inter, co
         op.done.zero_()
         live = ids[:, 0] >= 0
         first = op.contribute(x, ids, w).clone()
+        torch.cuda.synchronize()
+        assert torch.equal(op.done != 0, live.reshape(op.done.shape))
+        op.done.zero_()
+        op.contributions.fill_(float("nan"))
+        views = op.scratch_views()
+        views["act"].fill_(float("nan"))
+        views["aq"].fill_(0x7f)
+        views["sa"].fill_(float("nan"))
         for stage in (1, 2, 3):
             op.contribute(x, ids, w, stage=stage)
         torch.cuda.synchronize()
