@@ -483,7 +483,7 @@ __global__ __launch_bounds__(512, 2) void k_w8a8_cohort(const GemmParams p, cons
     }
     if (j == 16u && !have) return;
     uint32_t claim = 0;
-    if (tid == 0 && j < 16u) claim = atomicAdd(queue + x, 1u);  // lands under this unit
+    if (tid == 0 && j < 16u) claim = atomicAdd(queue + x, 1u);  // has landed when the unit's first requests go out
     if (have) {
       const u32x2 un = load_uniform<u32x2>(p.units + u);
       const int* gd = reinterpret_cast<const int*>(p.groups + int(un.x));
