@@ -30,7 +30,7 @@ namespace ffmoe {
 // 7168 / intermediate 2048: 122 + 78 -> 85 + 36 us against the 64-row kernel.
 enum TileForm { TILE_W8A8, TILE_MX, TILE_BF16, TILE_BF16_SPLIT };
 template <int MODE, TileForm FORM>
-__global__ __launch_bounds__(256, 2) void k_w8a8_tile(const GemmParams p) {
+__global__ __launch_bounds__(256, 2) void k_dense_tile(const GemmParams p) {
   constexpr bool MX = FORM == TILE_MX, SPLIT = FORM == TILE_BF16_SPLIT, BF = FORM == TILE_BF16 || SPLIT;
   struct Stage { uint8_t w[128 * 128]; uint8_t t[128 * 128]; };
   __shared__ __attribute__((aligned(16))) Stage stage[2];

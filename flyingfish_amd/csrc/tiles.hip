@@ -9,19 +9,19 @@
 namespace ffmoe {
 
 int launch_w8a8_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
-  if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, TILE_W8A8>), dim3(blocks), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((k_w8a8_tile<2, TILE_W8A8>), dim3(blocks), dim3(256), 0, stream, p);
+  if (mode == 0) hipLaunchKernelGGL((k_dense_tile<0, TILE_W8A8>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((k_dense_tile<2, TILE_W8A8>), dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
 }
 int launch_mx_dense_tile(int mode, const GemmParams& p, unsigned blocks, hipStream_t stream) {
-  if (mode == 0) hipLaunchKernelGGL((k_w8a8_tile<0, TILE_MX>), dim3(blocks), dim3(256), 0, stream, p);
-  else hipLaunchKernelGGL((k_w8a8_tile<2, TILE_MX>), dim3(blocks), dim3(256), 0, stream, p);
+  if (mode == 0) hipLaunchKernelGGL((k_dense_tile<0, TILE_MX>), dim3(blocks), dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((k_dense_tile<2, TILE_MX>), dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
 }
 
 int launch_bf16_tile(int mode, bool split, const GemmParams& p, unsigned blocks, hipStream_t stream) {
-  const auto kernel = split ? (mode == 0 ? k_w8a8_tile<0, TILE_BF16_SPLIT> : k_w8a8_tile<2, TILE_BF16_SPLIT>)
-                            : (mode == 0 ? k_w8a8_tile<0, TILE_BF16> : k_w8a8_tile<2, TILE_BF16>);
+  const auto kernel = split ? (mode == 0 ? k_dense_tile<0, TILE_BF16_SPLIT> : k_dense_tile<2, TILE_BF16_SPLIT>)
+                            : (mode == 0 ? k_dense_tile<0, TILE_BF16> : k_dense_tile<2, TILE_BF16>);
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, p);
   return ff_launch_status();
 }

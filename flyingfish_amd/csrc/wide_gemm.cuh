@@ -1,5 +1,5 @@
 // Dense W8A8 GEMM over many rows: a 256 x 256 output tile per block of eight waves and CU, operands through LDS by direct loads.
-// Arithmetic of k_w8a8_tile (tile_gemm.cuh), instruction for instruction, so the same bits.
+// Arithmetic of k_dense_tile (tile_gemm.cuh), instruction for instruction, so the same bits.
 //
 // What bounds it: a K block of a tile is 256 matrix instructions = 2048 cycles per SIMD with four scale fmas behind each (an
 // instruction and its fmas issue in 35 cycles), next to 196 KB of operand reads and 64 KB of direct loads in the CU's LDS. A tile of
