@@ -27,7 +27,7 @@ HBM_PEAK_GBPS = 8000.0
 GATE_UP_TRAFFIC_BYTES = {(1, 256): 265451800}
 TRAFFIC_SOURCE = "profiles/decode_layer_fp8_c3_batch1.hbm_traffic.txt"
 # W8A8 gate/up launch of the default prefill cohort (4096 tokens, 256 experts, seed 20251): FETCH_SIZE x 1.99977 + WRITE_SIZE
-PREFILL_GATE_UP_TRAFFIC_BYTES = 9190000000 + 135000000
+PREFILL_GATE_UP_TRAFFIC_BYTES = 9113000000 + 134500000
 PREFILL_TRAFFIC_SOURCE = "profiles/prefill_fp8_c5_4096tok.kernel_stats.txt"
 
 
@@ -471,21 +471,21 @@ def prefill_main(args, torch, capi, ops, synth, prebuilt=None):
         "cohort_mfma_frac": flop_total / (ms * 1e-3) / 1e12 / peak,
         "weight_bytes_once": touched * per,
         "cohort_weight_gbps": touched * per / (ms * 1e-3) / 1e9,
-        "roofline": {"kernel": ("ffmoe::k_nvfp4_tile<0>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 0, P>" if a16 else "ffmoe::k_mx_tile<0>" if mx else "ffmoe::k_w8a8_grouped<MF, 0, P>") + " (gate/up grouped GEMM + SwiGLU)", "bound": "mfma",
+        "roofline": {"kernel": ("ffmoe::k_nvfp4_tile<0>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 0, P>" if a16 else "ffmoe::k_mx_tile<0>" if mx else "ffmoe::k_w8a8_grouped<MF, 0, P>" if w4a8 else "ffmoe::k_w8a8_cohort<0> or k_w8a8_grouped<MF, 0, P>, by size") + " (gate/up grouped GEMM + SwiGLU)", "bound": "mfma",
                      "achieved": flop0 / (k0_avg * 1e-3) / 1e12, "peak": peak, "unit": "TFLOP/s",
                      "frac": flop0 / (k0_avg * 1e-3) / 1e12 / peak,
                      "traffic": PREFILL_GATE_UP_TRAFFIC_BYTES if default_cohort else None,
                      "traffic_source": PREFILL_TRAFFIC_SOURCE if default_cohort else None,
                      "flop_per_launch": flop0, "avg_ms": k0_avg, "min_ms": k0[0],
                      "weight_bytes_once": touched * per * 2 // 3, "weight_gbps": touched * per * 2 / 3 / (k0_avg * 1e-3) / 1e9},
-        "down_kernel": {"kernel": "ffmoe::k_nvfp4_tile<1>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 1, P>" if a16 else "ffmoe::k_mx_tile<1>" if mx else "ffmoe::k_w8a8_grouped<MF, 1, P>", "avg_ms": k1_avg, "min_ms": k1[0],
+        "down_kernel": {"kernel": "ffmoe::k_nvfp4_tile<1>" if a16 and args.format == "nvfp4" else "ffmoe::k_w16_grouped<F, MF, 1, P>" if a16 else "ffmoe::k_mx_tile<1>" if mx else "ffmoe::k_w8a8_grouped<MF, 1, P>" if w4a8 else "ffmoe::k_w8a8_cohort<1> or k_w8a8_grouped<MF, 1, P>, by size", "avg_ms": k1_avg, "min_ms": k1[0],
                         "tflops": A * 2.0 * H * I / (k1_avg * 1e-3) / 1e12},
     }
-    out["router_logits"] = {"kernel": "ffmoe::k_route_logits_f32_rows (FP32 logits of all token rows, vector ALUs, the oracle's summation order)",
+    out["router_logits"] = {"kernel": "ffmoe::k_route_logits_f32_mfma or, for fewer rows, k_route_logits_f32_rows (FP32 logits of all token rows in the oracle's summation order)",
                             "ms": lg_ms, "flop": 2.0 * R * E * H, "tflops": 2.0 * R * E * H / (lg_ms * 1e-3) / 1e12,
                             "frac_of_fp32_vector_peak": 2.0 * R * E * H / (lg_ms * 1e-3) / 1e12 / 157.3,
                             "frac_of_unpacked_fp32_rate": 2.0 * R * E * H / (lg_ms * 1e-3) / 1e12 / 78.65, "parity": lg_parity,
-                            "note": "side pass, not part of `value`: the cohort starts from seeded logits (BASELINE config 5). The published 157.3 "
+                            "note": "side pass, not part of `value`: the cohort starts from seeded logits (BASELINE config 5). The matrix instructions of K = 1 reach twice the unpacked vector rate. The published 157.3 "
                                     "TFLOP/s counts two fmas per lane and instruction (packed FP32), which this build is compiled without; one "
                                     "v_fma_f32 per lane and instruction is half of it"}
     out["parity"] = parity if parity is not None else ("not gated in bench.py for this format (tests/test_gpu_e8m0.py, tests/test_gpu_fullsize.py)" if mx else None)
@@ -693,7 +693,7 @@ def linear_main(args, torch, capi, ops, synth):
            "ms_per_step": head["us"] * 1e-3, "higher_is_better": False, "scaling": "weak", "vs_baseline": None,
            "dtype": "fp8_e4m3 weights (f32 128x128 block scales), bf16 activations, f32 accumulate", "data": "synthetic",
            "config": {"workload": "standalone FP8 block-scaled skinny linear (BASELINE config 2), M = 16, K = 7168, N = 2048"},
-           "roofline": {"kernel": "ffmoe::k_linear_mfma<FmtFp8, TR> (more than 4 rows) / ffmoe::k_linear<FmtFp8, S, RG>", "bound": "hbm",
+           "roofline": {"kernel": "ffmoe::k_linear_fp8_split<TR> (more than 4 rows) / ffmoe::k_linear<FmtFp8, S, RG>", "bound": "hbm",
                         "achieved": head["gbps"], "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": head["hbm_frac"], "traffic": None},
            "cases": rows}
     return out

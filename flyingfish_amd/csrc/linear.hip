@@ -306,8 +306,8 @@ __global__ __launch_bounds__(512) void k_linear_mfma(const LinearParams p, int m
 // of them at a time, with a barrier and a latency in front of each: 13.5 us for 16 x 7168 -> 2048. A wave's share of the tokens is its
 // own, so nothing needs sharing: here each wave moves its K blocks of tokens and weights straight into a ring of its own in LDS
 // (D blocks, 160 KB per CU in flight at once) and waits by count; the only barrier is the one in front of the eight partial sums.
-// us per call, weights cold, against k_linear_mfma (7.5 us of either is a call's way through the host): 16 rows 7168 -> 2048 13.6 -> 7.8,
-// 7168 -> 7168 28.8 -> 13.0, 4096 -> 4096 12.4 -> 7.7; 64 rows (four launches there) 7168 -> 2048 54 -> 11.0, 7168 -> 7168 115 -> 44.5.
+// us by kernel, weights cold, against k_linear_mfma: 16 rows 7168 -> 2048 13.3 -> 7.7, 7168 -> 7168 28.6 -> 12.9, 4096 -> 4096 11.6 -> 6.1; 64 rows (four
+// launches there) 7168 -> 2048 53 -> 11.1, 7168 -> 7168 115 -> 45.0. At 16 rows of 7168 the tokens are four fifths of what a CU moves.
 // LDS: token row r 256 bytes, 16-byte piece c at c ^ r ^ (r & 4) << 1; weight row r 128 bytes, piece c at c ^ lds_key(r).
 template <int TR>
 __global__ __launch_bounds__(512) void k_linear_fp8_split(const LinearParams p) {
